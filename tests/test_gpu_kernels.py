@@ -159,6 +159,26 @@ def test_jacobi_random_symmetric(tk, n):
         assert np.max(np.abs(w.T @ w - np.eye(n))) < 1e-13 * n
 
 
+# sizes on both sides of every change of the kernel's layout: 16 / 24 / 32
+# wide matrices, then pairs of 16-wide blocks with the last one partly or
+# wholly empty
+@pytest.mark.parametrize("n", [3, 15, 16, 17, 24, 25, 32, 33, 48, 49, 65, 80, 81])
+def test_jacobi_layout_edges(tk, n):
+    rng = np.random.default_rng(100 + n)
+    G = rng.standard_normal((2, n, n)); G = G + G.transpose(0, 2, 1)
+    A = rng.standard_normal((2 * n, n)) * np.logspace(0, -9, n)
+    G = np.concatenate([G, (A.T @ A)[None], np.diag(np.arange(n) - n / 3.0)[None]])
+    lam, W, sw = jacobi(tk, G)
+    for g, l, w in zip(G, lam, W):
+        ref = np.linalg.eigvalsh(g)
+        ref = ref[np.argsort(-np.abs(ref), kind="stable")]
+        s = np.max(np.abs(ref))
+        assert np.max(np.abs(np.sort(l) - np.sort(ref))) < 1e-13 * s * n
+        assert np.all(np.abs(l[:-1]) >= np.abs(l[1:]))
+        assert np.max(np.abs(g @ w - w * l)) < 1e-13 * s * n
+        assert np.max(np.abs(w.T @ w - np.eye(n))) < 1e-13 * n
+
+
 def test_jacobi_graded_gram_relative_accuracy(tk):
     rng = np.random.default_rng(9)
     A = rng.standard_normal((200, 64)) * np.logspace(0, -12, 64)

@@ -991,246 +991,661 @@ __global__ __launch_bounds__(256) void k_lincomb(const LinDesc* __restrict__ des
 }
 
 // ------------------------------------------------------------- Jacobi eigen
-// One 1024-thread workgroup per symmetric n x n matrix (n <= LMAX).
-// Parallel cyclic Jacobi with the circle-method tournament ordering: each
-// round rotates the n/2 disjoint pairs (p_i, q_i) simultaneously,
-// G <- J^T G J, W <- W J.  A pair is rotated only while
+// One workgroup per symmetric n x n matrix (n <= LMAX): cyclic two-sided
+// Jacobi, G <- J^T G J, W <- W J.  A pair is rotated only while
 // |g_pq| > tol sqrt(|g_pp g_qq|) (relative criterion, which keeps the small
-// eigenvalues of graded Gram matrices relatively accurate).  A round is two
-// phases: (1) one thread per pair computes its rotation (the tournament
-// positions advance in registers); (2) every 2x2 block
-// B_ij = G[{p_i,q_i},{p_j,q_j}] becomes J_i^T B_ij J_j (diagonal blocks from
-// the closed form g_pp - t g_pq, g_qq + t g_pq, 0) and every row of W is
-// rotated.  A sweep starts with a parallel scan of all off-diagonal pairs and
-// the solve stops when none violates the criterion.  The input is
+// eigenvalues of graded Gram matrices relatively accurate).
+//
+// The solve is a chain of dependent rounds (n - 1 per sweep), so what counts
+// is the latency of one round, not its arithmetic.  A round of M / 2 disjoint
+// rotations on an M x M matrix (M <= 32) runs inside ONE wavefront, with no
+// workgroup barrier between the rotations and their use: lane x computes the
+// rotation of pair x, every lane rotates its one or two off-diagonal 2 x 2
+// pair blocks and fetches the other pair's rotation from its lane.  The
+// matrix sits in LDS in tournament order: positions t_0 .. t_{M/2-1},
+// b_0 .. b_{M/2-1}, pair i = (t_i, b_i), and a round writes its results straight
+// to the positions of the next round, so the LDS addresses of a lane never
+// change.  A second wave holds the rows of the accumulated Q in registers and
+// applies the rotations one round behind (one barrier per round, where the
+// first wave has only just consumed its loads).
+//   n <= 32: M = 16, 24 or 32, Q is W.
+//   n <= 96: block Jacobi over 16-wide blocks.  Each block round pairs the
+//   blocks up, every pair's 32 x 32 matrix takes one sweep of rounds in its
+//   own two waves (31 rounds in the first block round of a sweep, which
+//   also rotates inside the blocks, 16 in the others), then the pairs' Q are
+//   applied to the rest of G and, during the next block round, to W on MFMA.
+//   W stays in registers as strips of W^T: the MFMA result layout is the B
+//   operand layout of the next block round's product.
+// Block rounds (or, for n <= 32, sweeps) without a violating pair are
+// skipped, and the solve ends with a sweep without one.  The input is
 // symmetrised on load ((G + G^T)/2).  Output: eigenvalues by |lambda|
 // descending, eigenvectors as columns of W in the same order.
-constexpr int JT = 1024;
+//
+// Measured, one Gram matrix of random columns (us a launch), against the
+// former kernel (1024 threads, every pair block and W in LDS, two workgroup
+// barriers a round): n = 16 / 32 / 64 / 96: 100 / 245 / 754 / 2112 -> 32 / 86
+// / 263 / 662; nearly diagonal ones (the block iteration's): 50 / 102 / 274 /
+// 696 -> 15 / 43 / 102 / 214.  A round takes 0.28 us at M = 16, 0.35 at 32,
+// 0.40 / 0.54 with two / three block pairs side by side (Q in LDS as well:
+// 0.49 / 0.56, the LDS pipe was the limit; W's MFMA on the SIMDs of the
+// rotations: 0.49); a block round adds 2.8 us at n = 64, 5 us at 96, the
+// orthogonal W of final solves 1 / 4 / 14 us at n = 32 / 64 / 96 (|W^T W - 1|
+// 1e-14 -> 5e-16).
+constexpr int JWAVES = 2;          // per pair of blocks: rotations, Q
+constexpr int JB = 16;             // block width for n > 32
+constexpr int JM = 2 * JB;
+// solves to a tighter threshold than this (final ones, whose W is a factor of
+// the result) also get W orthogonal to roundoff
+constexpr double JPOLISH_BELOW = 1e-13;
 
-// Pair (p < q) that tournament slot `slot` (0 <= slot < np / 2) rotates in
-// round r of a sweep: slot 0 keeps position 0, every other position moves
-// one step round the circle 1..np-1 per round.
-__device__ __forceinline__ void jacobi_pair(int slot, int r, int np, int& p, int& q) {
-    const int m = np - 1;
-    int a = 0;
-    if (slot > 0) {
-        a = slot - 1 + r;
-        if (a >= m) a -= m;
-        a += 1;
-    }
-    int b = np - 2 - slot + r;
-    if (b >= m) b -= m;
-    b += 1;
-    p = min(a, b);
-    q = max(a, b);
+// Position of a round's position x in the next round (t_i = i, b_i = H + i).
+// Full tournament: t_0 stays, the others go round the circle t_1 .. t_{H-1},
+// b_{H-1} .. b_0 (all pairs in 2H - 1 rounds, which is the identity).  Cross
+// rounds: the t_i stay, the b_i go round (all t-b pairs in H rounds, the
+// identity again).
+__device__ __forceinline__ int jacobi_next(int x, int H, bool cross) {
+    if (cross) return x < H ? x : (x == H ? 2 * H - 1 : x - 1);
+    if (x < H) return x == 0 ? 0 : (x == H - 1 ? 2 * H - 1 : x + 1);
+    return x == H ? 1 : x - 1;
 }
 
 // A pair is rotated while g_pq^2 > tol^2 |g_pp g_qq| (the relative
 // criterion keeps the small eigenvalues of graded Gram matrices relatively
-// accurate); the sweep scan and the rounds use this same predicate.
+// accurate); the scans and the rounds use this same predicate.
 __device__ __forceinline__ int jacobi_violates(double gpp, double gqq, double gpq, double tol2) {
     return gpq != 0.0 && gpq * gpq > tol2 * fabs(gpp * gqq);
 }
 
-// Rotation zeroing g_pq: with a = g_qq - g_pp, b = 2 g_pq and
-// h = sqrt(a^2 + b^2), t = sign(a) b / (|a| + h) is the tangent of the
-// smaller angle, c = 1 / sqrt(1 + t^2), s = t c.  The square roots and the
-// reciprocal come from the hardware estimates (v_rsq_f64, v_rcp_f64)
-// refined by two Newton steps each, a short dependent chain instead of
-// IEEE division and square-root sequences; c^2 + s^2 = 1 to a few ulp.
+// 1 / sqrt(x) from the hardware estimate (v_rsq_f64, ~24 bits) and one
+// third-order step, a shorter dependent chain than two Newton steps:
+// with e = 1 - x y^2, y (1 + e / 2 + 3 e^2 / 8).
 __device__ __forceinline__ double rsqrt_refined(double x) {
-    double y = __builtin_amdgcn_rsq(x);
-#pragma unroll
-    for (int k = 0; k < 2; ++k) {
-        const double e = fma(-x * y, y, 1.0);       // 1 - x y^2
-        y = fma(0.5 * y, e, y);
-    }
-    return y;
+    const double y = __builtin_amdgcn_rsq(x);
+    const double e = fma(-x * y, y, 1.0);
+    return fma(y * e, fma(0.375, e, 0.5), y);
 }
 
-__device__ __forceinline__ double rcp_refined(double d) {
-    double y = __builtin_amdgcn_rcp(d);
-#pragma unroll
-    for (int k = 0; k < 2; ++k) {
-        const double e = fma(-d, y, 1.0);
-        y = fma(y, e, y);
-    }
-    return y;
-}
-
+// Rotation zeroing g_pq by the smaller angle: with a = g_qq - g_pp,
+// b = 2 g_pq and r = 1 / sqrt(a^2 + b^2), cos 2x = |a| r and
+// sin 2x = sign(a) b r, so c^2 = (1 + cos 2x) / 2, s = sin 2x / (2 c) and
+// t = s / c: two reciprocal square roots in a row and no division.
+// c^2 + s^2 = 1 to a few ulp.
 __device__ __forceinline__ void jacobi_rotation(double gpp, double gqq, double gpq, double& t,
                                                 double& c, double& s) {
     const double a = gqq - gpp, b = 2.0 * gpq;
-    const double h2 = fma(a, a, b * b);
-    const double h = h2 * rsqrt_refined(h2);
-    t = (a >= 0.0 ? b : -b) * rcp_refined(fabs(a) + h);
-    c = rsqrt_refined(fma(t, t, 1.0));
-    s = t * c;
+    const double hb = a >= 0.0 ? gpq : -gpq;
+    const double r = rsqrt_refined(fma(a, a, b * b));
+    const double x = fma(0.5 * fabs(a), r, 0.5);
+    const double y = rsqrt_refined(x);
+    const double hs = hb * r;
+    c = x * y;
+    s = hs * y;
+    t = s * y;
 }
 
-__global__ __launch_bounds__(JT) void k_jacobi(const JacobiDesc* __restrict__ descs, int nd,
-                                               double tol, int max_sweeps) {
-    extern __shared__ double lds[];
-    const JacobiDesc D = descs[blockIdx.x];
-    if (D.skip && *D.skip) return;
-    const int n = D.n;
-    const int np = n + (n & 1);
-    const int ld = np + 1;              // padded column stride (bank spread)
-    double* G = lds;                    // np x np, G[i + j*ld]
-    double* W = G + np * ld;
-    double4* rot = (double4*)(W + np * ld);      // (c, s, t, active) per pair
-    int* pos = (int*)(rot + LMAX / 2);           // output order (LMAX ints)
-    const int t = threadIdx.x;
-    const float inv_np = 1.0f / (float)np;
-    // G is symmetric and only its upper triangle (row <= column) is read
-    // or written after the load: gx(r, c) addresses entry (r, c) there
-    auto gx = [ld](int r, int c) { return r <= c ? r + c * ld : c + r * ld; };
-    for (int e = t; e < np * np; e += JT) {
-        const int j = (int)(((float)e + 0.5f) * inv_np), i = e - j * np;
-        G[i + j * ld] = (i < n && j < n)
-                            ? 0.5 * (D.G[i + (int64_t)j * D.ldg] + D.G[j + (int64_t)i * D.ldg])
-                            : 0.0;
-        W[i + j * ld] = (i == j) ? 1.0 : 0.0;
-    }
-    const int half = np / 2, m = np - 1;
-    const int ntri = half * (half + 1) / 2;      // pair blocks (i <= j), <= 2 * JT
-    const double tol2 = tol * tol;
-    // this thread's fixed tasks: pair blocks e = t, t + JT of the upper
-    // triangle, and (pair, row) entries e = t + u JT of W
-    int gi[2] = {-1, -1}, gj[2] = {-1, -1};
+// LDS of one block pair: the M x M matrix (upper triangle by position), Q by
+// columns (two for n > 32: the W strips read one while the rounds build the
+// other) and the rotations of two rounds.  The strides keep the Q rows'
+// rounds and the MFMA operand reads at two lanes per bank or fewer.
+template <int M, int NS>
+struct JacLds {
+    static constexpr int H = M / 2, SL = (H / 2 + 3) / 4;
+    static constexpr int LS = M + 1, LQ = M + 4;
+    static constexpr int SINK = M * LS;   // for results that go nowhere
+    static constexpr int Q = M * LS + 2, NQ = NS > 1 ? 2 : 1, CS = Q + NQ * M * LQ;
+    static constexpr int DOUBLES = CS + 4 * H;
+    static constexpr int NP = NS > 1 ? M * NS : 0, LG = NP + 2;   // the whole matrix, n > 32
+    static constexpr size_t ALL = (size_t)NP * LG + (size_t)NS * DOUBLES;
+    // waves: per block pair one for the rotations and one for Q; for n > 32
+    // one more per block pair, for two strips of W
+    static constexpr int WAVES = NS * (NS > 1 ? JWAVES + 1 : JWAVES);
+};
+
+// behind them: the waves' violation flags (two block rounds), the output order
+constexpr size_t JTAIL_BYTES = (2 * 3 * JWAVES + LMAX) * sizeof(int);
+
+size_t jacobi_lds_bytes(int n) {
+    const size_t d = n <= 16       ? JacLds<16, 1>::ALL
+                     : n <= 24     ? JacLds<24, 1>::ALL
+                     : n <= JM     ? JacLds<JM, 1>::ALL
+                     : n <= 2 * JM ? JacLds<JM, 2>::ALL
+                                   : JacLds<JM, 3>::ALL;
+    return d * sizeof(double) + JTAIL_BYTES;
+}
+
+int jacobi_threads(int n) {
+    return 64 * (n <= JM ? JacLds<JM, 1>::WAVES : n <= 2 * JM ? JacLds<JM, 2>::WAVES : JacLds<JM, 3>::WAVES);
+}
+
+// compiler and LDS order between this wave's own steps (the LDS unit runs a
+// wave's accesses in order)
+__device__ __forceinline__ void wave_order() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+__device__ __forceinline__ double lane_read(int byte_lane, double x) {
+    const int lo = __builtin_amdgcn_ds_bpermute(byte_lane, __double2loint(x));
+    const int hi = __builtin_amdgcn_ds_bpermute(byte_lane, __double2hiint(x));
+    return __hiloint2double(hi, lo);
+}
+
+// LDS places of a lane's entries in a round, and of its results for the next
+// round (full tournament, cross rounds).  Lane (g, x) of the wave's four rows
+// of 16 computes the rotation of pair x (each row again) and rotates the pair
+// blocks (x, x + g + 1 + 4 u mod H): its own rotation comes first, while the
+// other pair's is fetched from its lane.
+template <int M, int NS>
+struct JacPlaces {
+    using L = JacLds<M, NS>;
+    int from[L::SL], rd[L::SL][4], wr[2][L::SL][4], drd[3], dwr[2][3];
+    __device__ __forceinline__ explicit JacPlaces(int lane) {
+        constexpr int H = L::H;
+        auto at = [](int x, int y) { return min(x, y) + max(x, y) * L::LS; };
+        const int x0 = lane & 15, x = x0 < H ? x0 : x0 - H;   // spare lanes repeat others
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
-        const int e = t + u * JT;
-        if (e < ntri) {
-            int j = (int)((sqrtf(8.0f * (float)e + 1.0f) - 1.0f) * 0.5f);
-            while (j * (j + 1) / 2 > e) --j;
-            while ((j + 1) * (j + 2) / 2 <= e) ++j;
-            gi[u] = e - j * (j + 1) / 2;
-            gj[u] = j;
-        }
-    }
-    constexpr int WT = (LMAX / 2) * LMAX / JT + 1;   // W tasks per thread, max
-    int wslot[WT], wrow[WT];
-    {
-        int j = t / np, r = t - (t / np) * np;
-        const int wdj = JT / np, wdr = JT - (JT / np) * np;
+        for (int u = 0; u < L::SL; ++u) {
+            const int dist = min((lane >> 4) + 1 + 4 * u, H / 2);
+            const int y = x + dist < H ? x + dist : x + dist - H;
+            // the blocks of distance H / 2 are met from both ends: one end's
+            // results go nowhere
+            const bool twin = dist == H / 2 && x >= H / 2;
+            from[u] = 4 * y;
 #pragma unroll
-        for (int u = 0; u < WT; ++u) {
-            wslot[u] = j < half ? j : -1;
-            wrow[u] = r;
-            r += wdr;
-            j += wdj;
-            if (r >= np) { r -= np; ++j; }
+            for (int q = 0; q < 4; ++q) {
+                const int p = x + (q >> 1) * H, r = y + (q & 1) * H;
+                rd[u][q] = at(p, r);
+#pragma unroll
+                for (int c = 0; c < 2; ++c)
+                    wr[c][u][q] = twin ? L::SINK : at(jacobi_next(p, H, c), jacobi_next(r, H, c));
+            }
+        }
+        drd[0] = at(x, x); drd[1] = at(x + H, x + H); drd[2] = at(x, x + H);
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            const int p = jacobi_next(x, H, c), q = jacobi_next(x + H, H, c);
+            dwr[c][0] = at(p, p); dwr[c][1] = at(q, q); dwr[c][2] = at(p, q);
         }
     }
-    // any off-diagonal pair p < q that still violates the criterion
-    auto violated = [&]() {
-        int viol = 0;
-        for (int e = t; e < np * np; e += JT) {
-            const int q = (int)(((float)e + 0.5f) * inv_np), p = e - q * np;
-            if (p < q)
-                viol |= jacobi_violates(G[p + p * ld], G[q + q * ld], G[p + q * ld], tol2);
-        }
-        return __syncthreads_or(viol);
+};
+
+// One sweep of R rounds on the matrix in S by one wave, R + 1 barriers.
+template <int M, int NS>
+__device__ __forceinline__ void jacobi_rounds(const JacPlaces<M, NS>& P, double* S, double2* cs, int lane,
+                                              int R, bool cross, double tol2) {
+    using L = JacLds<M, NS>;
+    constexpr int H = L::H, SL = L::SL;
+    int wr[SL][4], dwr[3];
+#pragma unroll
+    for (int u = 0; u < SL; ++u)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) wr[u][q] = cross ? P.wr[1][u][q] : P.wr[0][u][q];
+#pragma unroll
+    for (int q = 0; q < 3; ++q) dwr[q] = cross ? P.dwr[1][q] : P.dwr[0][q];
+    double b[SL][4], d[3];
+    auto load = [&] {
+#pragma unroll
+        for (int k = 0; k < 3; ++k) d[k] = S[P.drd[k]];
+#pragma unroll
+        for (int u = 0; u < SL; ++u)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) b[u][q] = S[P.rd[u][q]];
     };
-    int sweeps = 0;
-    bool converged = false;
-    for (int sw = 0; sw < max_sweeps; ++sw) {
-        if (!violated()) {
-            converged = true;
-            break;
+    load();
+    for (int r = 0; r < R; ++r) {
+        // the diagonal's arrival means that every LDS access issued before
+        // it is done, the last round's rotations among them
+        asm volatile("s_barrier" ::"v"(d[0]), "v"(d[1]), "v"(d[2]) : "memory");
+        // once a round is run, pairs a hundred times below the threshold are
+        // rotated too: it costs nothing, and close eigenvalues' vectors feel
+        // what is left over their gap
+        const bool on = jacobi_violates(d[0], d[1], d[2], 1e-4 * tol2);
+        double c, s, t;
+        jacobi_rotation(d[0], d[1], d[2], t, c, s);
+        c = on ? c : 1.0;
+        s = on ? s : 0.0;
+        t = on ? t : 0.0;
+        double co[SL], so[SL];
+#pragma unroll
+        for (int u = 0; u < SL; ++u) {
+            co[u] = lane_read(P.from[u], c);
+            so[u] = lane_read(P.from[u], s);
         }
-        ++sweeps;
-        for (int rnd = 0; rnd < m; ++rnd) {
-            // The pairs of a round are fixed by the tournament schedule, so
-            // this thread's G block and W entries are loaded before the
-            // rotations are known (nothing writes G or W until the barrier
-            // after them).
-            int bp[2] = {0, 0}, bq[2] = {0, 0}, cp[2] = {0, 0}, cq[2] = {0, 0};
-            double b00[2], b01[2], b10[2], b11[2];
+        if (lane < H) {
+            cs[(r & 1) * H + lane] = make_double2(c, s);
+            S[dwr[0]] = d[0] - t * d[2];
+            S[dwr[1]] = d[1] + t * d[2];
+            S[dwr[2]] = on ? 0.0 : d[2];
+        }
 #pragma unroll
-            for (int u = 0; u < 2; ++u) {
-                if (gi[u] < 0) continue;
-                jacobi_pair(gi[u], rnd, np, bp[u], bq[u]);
-                jacobi_pair(gj[u], rnd, np, cp[u], cq[u]);
-                b00[u] = G[gx(bp[u], cp[u])];
-                b01[u] = G[gx(bp[u], cq[u])];
-                b10[u] = G[gx(bq[u], cp[u])];
-                b11[u] = G[gx(bq[u], cq[u])];
-            }
-            int wa[WT], wb[WT];
-            double wp[WT], wq[WT];
+        for (int u = 0; u < SL; ++u) {
+            const double y0 = c * b[u][0] - s * b[u][2], y1 = c * b[u][1] - s * b[u][3];
+            const double y2 = s * b[u][0] + c * b[u][2], y3 = s * b[u][1] + c * b[u][3];
+            b[u][0] = y0; b[u][1] = y1; b[u][2] = y2; b[u][3] = y3;
+        }
 #pragma unroll
-            for (int u = 0; u < WT; ++u) {
-                if (wslot[u] < 0) continue;
-                int p, q;
-                jacobi_pair(wslot[u], rnd, np, p, q);
-                wa[u] = wrow[u] + p * ld;
-                wb[u] = wrow[u] + q * ld;
-                wp[u] = W[wa[u]];
-                wq[u] = W[wb[u]];
-            }
-            if (t < half) {
-                int p, q;
-                jacobi_pair(t, rnd, np, p, q);
-                const double gpp = G[p + p * ld], gqq = G[q + q * ld], gpq = G[p + q * ld];
-                const int on = jacobi_violates(gpp, gqq, gpq, tol2);
-                double c = 1.0, sn = 0.0, tt = 0.0;
-                if (on) jacobi_rotation(gpp, gqq, gpq, tt, c, sn);
-                rot[t] = make_double4(c, sn, tt, on ? 1.0 : 0.0);
-            }
-            // every task checks its pairs' flags below, so a plain barrier
-            // suffices (a workgroup OR-reduction costs two)
-            __syncthreads();
-            // G <- J^T G J on the upper pair blocks; the lower ones are their
-            // transposes, kept only through gx
+        for (int u = 0; u < SL; ++u) {
+            const double y0 = co[u] * b[u][0] - so[u] * b[u][1], y1 = so[u] * b[u][0] + co[u] * b[u][1];
+            const double y2 = co[u] * b[u][2] - so[u] * b[u][3], y3 = so[u] * b[u][2] + co[u] * b[u][3];
+            S[wr[u][0]] = y0;
+            S[wr[u][1]] = y1;
+            S[wr[u][2]] = y2;
+            S[wr[u][3]] = y3;
+        }
+        wave_order();
+        load();
+    }
+    __syncthreads();
+}
+
+// Rows of the accumulated Q in one wave's registers, columns in tournament
+// order: lane (h, row) holds pairs HP h .. HP h + HP - 1 of row `row` (lanes
+// past M hold rows that are never read).
+template <int M>
+struct JacRows {
+    static constexpr int H = M / 2, HP = H / 2;
+    double t[HP], b[HP];
+    __device__ __forceinline__ void identity(int lane) {
+        const int row = lane & 31, p0 = HP * (lane >> 5);
 #pragma unroll
-            for (int u = 0; u < 2; ++u) {
-                const int i = gi[u], j = gj[u];
-                if (i < 0) continue;
-                const double4 ri = rot[i], rj = rot[j];
-                if (ri.w == 0.0 && rj.w == 0.0) continue;
-                const int pi = bp[u], qi = bq[u], pj = cp[u], qj = cq[u];
-                if (i == j) {
-                    const double tt = ri.z, gpq = b01[u];
-                    G[pi + pi * ld] = b00[u] - tt * gpq;
-                    G[qi + qi * ld] = b11[u] + tt * gpq;
-                    G[pi + qi * ld] = 0.0;   // pi < qi
-                    continue;
-                }
-                const double ci = ri.x, si = ri.y, cj = rj.x, sj = rj.y;
-                const double x00 = ci * b00[u] - si * b10[u], x01 = ci * b01[u] - si * b11[u];
-                const double x10 = si * b00[u] + ci * b10[u], x11 = si * b01[u] + ci * b11[u];
-                const double y00 = cj * x00 - sj * x01, y01 = sj * x00 + cj * x01;   // (.) J_j
-                const double y10 = cj * x10 - sj * x11, y11 = sj * x10 + cj * x11;
-                G[gx(pi, pj)] = y00;
-                G[gx(pi, qj)] = y01;
-                G[gx(qi, pj)] = y10;
-                G[gx(qi, qj)] = y11;
-            }
-            // W <- W J: this thread's (pair, row) tasks touch distinct columns
-#pragma unroll
-            for (int u = 0; u < WT; ++u) {
-                if (wslot[u] < 0) continue;
-                const double4 rj = rot[wslot[u]];
-                if (rj.w == 0.0) continue;
-                W[wa[u]] = rj.x * wp[u] - rj.y * wq[u];
-                W[wb[u]] = rj.y * wp[u] + rj.x * wq[u];
-            }
-            __syncthreads();
+        for (int i = 0; i < HP; ++i) {
+            t[i] = row == p0 + i ? 1.0 : 0.0;
+            b[i] = row == p0 + i + H ? 1.0 : 0.0;
         }
     }
-    // sweep cap reached: converged only if the last sweep left nothing to rotate
-    if (!converged && violated() && t == 0 && D.fail) *D.fail = 1.0;
+    // R rounds, one behind the rotations' wave, R + 1 barriers; the shifts
+    // are jacobi_next on the pairs, between the halves by a lane swap
+    template <bool CROSS>
+    __device__ __forceinline__ void rounds(const double2* cs, int lane, int R) {
+        const bool hi = lane >= 32;
+        asm volatile("s_barrier" ::: "memory");
+        for (int r = 0; r < R; ++r) {
+            // (the rotations of the round before have been read)
+            asm volatile("s_barrier" ::: "memory");
+            const double2* rot = cs + (r & 1) * H + HP * (lane >> 5);
+            double2 k[HP];
+#pragma unroll
+            for (int i = 0; i < HP; ++i) k[i] = rot[i];
+            double x[HP], y[HP];
+#pragma unroll
+            for (int i = 0; i < HP; ++i) {
+                x[i] = k[i].x * t[i] - k[i].y * b[i];
+                y[i] = k[i].y * t[i] + k[i].x * b[i];
+            }
+            const double v = CROSS || hi ? y[0] : x[HP - 1];
+            const auto lo2 = __builtin_amdgcn_permlane32_swap(__double2loint(v), __double2loint(v), false, false);
+            const auto hi2 = __builtin_amdgcn_permlane32_swap(__double2hiint(v), __double2hiint(v), false, false);
+            // .x: the lower half's value, .y: the upper half's, in every lane
+            const double got = hi ? __hiloint2double(hi2[0], lo2[0]) : __hiloint2double(hi2[1], lo2[1]);
+#pragma unroll
+            for (int i = 0; i + 1 < HP; ++i) b[i] = y[i + 1];
+            if (CROSS) {
+                b[HP - 1] = got;
+#pragma unroll
+                for (int i = 0; i < HP; ++i) t[i] = x[i];
+            } else {
+                b[HP - 1] = hi ? x[HP - 1] : got;
+                t[0] = hi ? got : x[0];
+                t[1] = hi ? x[0] : y[0];
+#pragma unroll
+                for (int i = 2; i < HP; ++i) t[i] = x[i - 1];
+            }
+        }
+    }
+    __device__ __forceinline__ void store(double* Q, int ld, int lane) const {
+        const int row = lane & 31, p0 = HP * (lane >> 5);
+        if (row >= M) return;
+#pragma unroll
+        for (int i = 0; i < HP; ++i) {
+            Q[row + (p0 + i) * ld] = t[i];
+            Q[row + (p0 + i + H) * ld] = b[i];
+        }
+    }
+};
+
+// A operand of one k-step of a product with Q^T: rows 16 o .. of Q^T (columns
+// of Q), k = 16 k0 + 4 kk ..
+__device__ __forceinline__ double jac_qt(const double* Q, int LQ, int lane, int o, int k0, int kk) {
+    return Q[16 * k0 + 4 * kk + (lane >> 4) + (16 * o + (lane & 15)) * LQ];
+}
+
+// position of slot x of the block tournament in the next block round
+constexpr int jac_slot_next(int x, int NS) {
+    return x < NS ? (x == 0 ? 0 : (x == NS - 1 ? 2 * NS - 1 : x + 1)) : (x == NS ? 1 : x - 1);
+}
+
+template <int M, int NS>
+__device__ void jacobi_body(const JacobiDesc& D, double* lds, double tol, int max_sweeps, bool polish) {
+    using L = JacLds<M, NS>;
+    constexpr int H = L::H, NB = NS > 1 ? 2 * NS : 1, NP = L::NP, LG = L::LG;
+    constexpr int NT = 64 * L::WAVES, ST = 64 * JWAVES, PW = NS * JWAVES;
+    const int n = D.n, t = threadIdx.x, lane = t & 63;
+    const int w = __builtin_amdgcn_readfirstlane(t >> 6);
+    if (w >= L::WAVES) return;   // a larger problem of the group set the block size
+    // The waves' work: per block pair `sub` one wave for the rotations (ROT)
+    // and one for Q, for n > 32 also one per block pair with two strips of W.
+    // Waves go round the four SIMDs, and FP64 MFMA keeps a SIMD's FP64 unit
+    // from its other waves: the rotations' waves get SIMDs of their own
+    // (n <= 64), or share one with the least there is (n <= 96).
+    enum { ROT, QROWS, STRIPS };
+    int role, sub;
+    if constexpr (NS == 1) {
+        role = w, sub = 0;
+    } else if constexpr (NS == 2) {
+        role = w < 2 ? QROWS : w < 4 ? ROT : STRIPS, sub = w & 1;
+    } else {
+        // SIMD 0: strips 0 and 1, Q 0; 1: rotations 0, strips 2; 2, 3: rotations, Q
+        role = w == 0 || w == 4 || w == 5 ? STRIPS : w < 4 ? ROT : QROWS;
+        sub = w == 0 ? 0 : w == 4 ? 1 : w == 5 ? 2 : w < 4 ? w - 1 : w == 8 ? 0 : w - 5;
+    }
+    const int slot = JWAVES * sub + role, ts = lane + 64 * role;   // (not the strips)
+    double* G = lds;
+    double* S0 = lds + NP * LG;
+    double* S = S0 + sub * L::DOUBLES;
+    double2* cs = (double2*)(S + L::CS);
+    int* flags = (int*)(S0 + NS * L::DOUBLES);   // [2][PW]
+    int* pos = flags + 2 * 3 * JWAVES;
+    // every lane loads (clamped, in bounds), so the loads are not predicated
+    // and stay in flight together
+    auto entry = [&](int x, int y) {
+        const int xc = min(x, n - 1), yc = min(y, n - 1);
+        const double v = 0.5 * (D.G[xc + (int64_t)yc * D.ldg] + D.G[yc + (int64_t)xc * D.ldg]);
+        return x < n && y < n ? v : 0.0;
+    };
+    if constexpr (NS == 1) {
+#pragma unroll 4
+        for (int e = t; e < M * M; e += NT) {
+            const int y = e / M, x = e - y * M;
+            const double v = entry(x, y);
+            if (x <= y) S[x + y * L::LS] = v;
+        }
+    } else {
+#pragma unroll 4
+        for (int e = t; e < NP * NP; e += NT) {
+            const int y = e / NP, x = e - y * NP;
+            G[x + y * LG] = entry(x, y);
+        }
+    }
+    __syncthreads();
+    constexpr int ROUNDS = NS > 1 ? NB - 1 : 1;   // block rounds of a sweep
+    const double tol2 = tol * tol;
+    int sweeps = 0;
+    // The sweeps, as every wave of the workgroup goes through them: `scan`
+    // writes this wave's flag for a block round, `act` gets `on` (the block
+    // pairs with a violating pair, one bit each), whether they are to be
+    // rotated, and whether within the blocks too.
+    auto drive = [&](auto&& scan, auto&& act) {
+        int par = 0;
+        for (int sw = 0;; ++sw) {
+            bool any = false, stop = false;
+#pragma unroll 1
+            for (int rnd = 0; rnd < ROUNDS; ++rnd) {
+                int* fl = flags + par * PW;
+                par ^= 1;
+                scan(fl, rnd);
+                __syncthreads();
+                int on = 0, f = 0;
+#pragma unroll
+                for (int s = 0; s < NS; ++s) {
+                    const int v = fl[JWAVES * s] | fl[JWAVES * s + 1];
+                    f |= v;
+                    on |= v ? 1 << s : 0;
+                }
+                f = __builtin_amdgcn_readfirstlane(f);
+                on = __builtin_amdgcn_readfirstlane(on);
+                if (f) {
+                    any = true;
+                    stop = sw == max_sweeps;
+                }
+                act(on, f && !stop, !(f & 2));
+            }
+            if (stop && t == 0 && D.fail) *D.fail = 1.0;   // sweep cap, a rotation still due
+            if (stop || !any) break;
+            ++sweeps;
+        }
+    };
+    auto rounds_of = [](bool cross) { return cross ? H : M - 1; };
+    int qbuf = 0;
+    // the blocks in the slots of the block tournament: tops 0 .. NS - 1, then
+    // bottoms
+    int ids[NB];
+#pragma unroll
+    for (int b = 0; b < NB; ++b) ids[b] = b;
+    int I = 0, J = 0;   // first rows of this block pair's blocks (J: less H)
+    // violating pairs of this block pair (within the blocks only in the first
+    // block round); its matrix into S
+    auto scan_pair = [&](int* fl, int rnd) {
+        if constexpr (NS > 1) {
+#pragma unroll
+            for (int s = 0; s < NS; ++s)
+                if (s == sub) {
+                    I = JB * ids[s];
+                    J = JB * ids[NS + s] - H;
+                }
+        }
+        int v = 0;
+        // entries (x <= y): the cross square, then both blocks' triangles in
+        // one square (upper: first block, lower: second), then the second's
+        // diagonal
+        constexpr int HH = H * H;
+#pragma unroll
+        for (int k = 0; k < (2 * HH + H + ST - 1) / ST; ++k) {
+            const int e = min(ts + k * ST, 2 * HH + H - 1);
+            const int sq = e / HH, r = e - sq * HH, c = r / H, a = r - c * H;   // column, row in the square
+            int x, y;
+            if (sq == 0) x = a, y = c + H;
+            else if (sq == 1) x = a <= c ? a : c + H, y = a <= c ? c : a + H;
+            else x = y = r + H;
+            const double* A = NS > 1 ? G : S;
+            constexpr int LA = NS > 1 ? LG : L::LS;
+            const int gx = (x < H ? I : J) + x, gy = (y < H ? I : J) + y;
+            const double gxy = A[gx + gy * LA], gxx = A[gx + gx * LA], gyy = A[gy + gy * LA];
+            if (NS > 1) S[x + y * L::LS] = gxy;
+            if (x != y && jacobi_violates(gxx, gyy, gxy, tol2)) v |= sq ? 2 : 1;
+        }
+        if (NS > 1 && rnd > 0) v &= 1;
+        v = (__any(v & 1) ? 1 : 0) | (__any(v & 2) ? 2 : 0);
+        if (lane == 0) fl[slot] = v;
+    };
+    // after the rounds: the block pairs' Q applied to the rest of G
+    auto apply = [&](int on) {
+        __syncthreads();
+        if constexpr (NS > 1) {
+            // the 32 x 32 off-diagonal matrix of each two block pairs a < b,
+            // G_ab <- Q_a^T G_ab Q_b: H = Q_a^T G_ab (into the Q buffer that
+            // the W strips are done with), then Q_b^T H^T, both triangles
+            // written.  A unit of either product is one 16 x 16 tile.
+            constexpr int UNITS = 2 * NS * (NS - 1);
+            auto unit = [&](int u, int* ra, int* rb) {   // first rows of a's and b's blocks; whether to do
+                const int a = u < 8 ? 0 : 1, b = u < 4 ? 1 : 2;
+#pragma unroll
+                for (int s = 0; s < NS; ++s) {
+                    if (s == a) { ra[0] = JB * ids[s]; ra[1] = JB * ids[NS + s]; }
+                    if (s == b) { rb[0] = JB * ids[s]; rb[1] = JB * ids[NS + s]; }
+                }
+                return (on >> a & 1) || (on >> b & 1);
+            };
+            auto qof = [&](int s, int buf) { return S0 + s * L::DOUBLES + L::Q + buf * M * L::LQ; };
+            for (int u = w; u < UNITS; u += L::WAVES) {
+                int ra[2], rb[2];
+                if (!unit(u, ra, rb)) continue;
+                const int o = u & 1, c = u >> 1 & 1;   // tile: rows of a, columns of b
+                const double* Qa = qof(u < 8 ? 0 : 1, qbuf);
+                const double* col = G + (lane >> 4) + ((c ? rb[1] : rb[0]) + (lane & 15)) * LG;
+                dbl4 h = dbl4{0, 0, 0, 0}, h2 = dbl4{0, 0, 0, 0};
+#pragma unroll
+                for (int kk = 0; kk < 4; ++kk) {
+                    h = __builtin_amdgcn_mfma_f64_16x16x4f64(jac_qt(Qa, L::LQ, lane, o, 0, kk),
+                                                             col[ra[0] + 4 * kk], h, 0, 0, 0);
+                    h2 = __builtin_amdgcn_mfma_f64_16x16x4f64(jac_qt(Qa, L::LQ, lane, o, 1, kk),
+                                                              col[ra[1] + 4 * kk], h2, 0, 0, 0);
+                }
+                h = h + h2;
+                double* dst = qof(u >> 2, qbuf ^ 1) + 16 * o + (lane >> 4) + (16 * c + (lane & 15)) * L::LQ;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) dst[4 * r] = h[r];
+            }
+            // the block pairs' own matrices, both triangles
+#pragma unroll
+            for (int s = 0; s < NS; ++s) {
+                if (!(on >> s & 1)) continue;
+                const int i0 = JB * ids[s], j0 = JB * ids[NS + s] - H;
+                const double* Ss = S0 + s * L::DOUBLES;
+#pragma unroll
+                for (int k = 0; k < (M * M + NT - 1) / NT; ++k) {
+                    const int e = min(t + k * NT, M * M - 1), y = e / M, x = e - y * M;
+                    G[(x < H ? i0 : j0) + x + ((y < H ? i0 : j0) + y) * LG] = Ss[min(x, y) + max(x, y) * L::LS];
+                }
+            }
+            __syncthreads();
+            for (int u = w; u < UNITS; u += L::WAVES) {
+                int ra[2], rb[2];
+                if (!unit(u, ra, rb)) continue;
+                const int o = u & 1, c = u >> 1 & 1;   // tile: columns of b, rows of a
+                const double* Qb = qof(u < 4 ? 1 : 2, qbuf);
+                const double* hs = qof(u >> 2, qbuf ^ 1) + 16 * c + (lane & 15) + (lane >> 4) * L::LQ;
+                dbl4 h = dbl4{0, 0, 0, 0}, h2 = dbl4{0, 0, 0, 0};
+#pragma unroll
+                for (int kk = 0; kk < 4; ++kk) {
+                    h = __builtin_amdgcn_mfma_f64_16x16x4f64(jac_qt(Qb, L::LQ, lane, o, 0, kk),
+                                                             hs[4 * kk * L::LQ], h, 0, 0, 0);
+                    h2 = __builtin_amdgcn_mfma_f64_16x16x4f64(jac_qt(Qb, L::LQ, lane, o, 1, kk),
+                                                              hs[(16 + 4 * kk) * L::LQ], h2, 0, 0, 0);
+                }
+                h = h + h2;
+                const int row = (c ? ra[1] : ra[0]) + (lane & 15), cb = (o ? rb[1] : rb[0]) + (lane >> 4);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    G[row + (cb + 4 * r) * LG] = h[r];
+                    G[cb + 4 * r + row * LG] = h[r];
+                }
+            }
+            __syncthreads();
+            qbuf ^= 1;
+        }
+    };
+    auto next_slots = [&] {
+        if constexpr (NS > 1) {
+            int nid[NB];
+#pragma unroll
+            for (int b = 0; b < NB; ++b) nid[jac_slot_next(b, NS)] = ids[b];
+#pragma unroll
+            for (int b = 0; b < NB; ++b) ids[b] = nid[b];
+        }
+    };
+    auto idle = [](int R) {
+        for (int r = 0; r <= R; ++r) asm volatile("s_barrier" ::: "memory");
+    };
+    // strips 2 sub, 2 sub + 1 of W^T (16 columns each), by slot
+    const int st0 = 2 * sub;
+    dbl4 wt[2][NB];
+    // (each role's loop is its own code, so that its registers are its own)
+    if (NS > 1 && role == STRIPS) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int b = 0; b < NB; ++b)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    wt[h][b][r] = (b == st0 + h && 4 * r + (lane >> 4) == (lane & 15)) ? 1.0 : 0.0;
+        int owed = 0;   // block pairs whose Q (in the other buffer) W still lacks
+        drive([](int*, int) {}, [&](int on, bool go, bool cross) {
+            // W^T <- Q^T W^T with the last rotated block round's Q, a few MFMAs
+            // per barrier of this one's rounds.  A result is laid out as the
+            // next product's B operand, so the strips never leave the registers.
+            const int R = rounds_of(cross);
+            int done = 0;
+#pragma unroll
+            for (int s = 0; s < NS; ++s) {
+                if (!(owed >> s & 1)) continue;
+                const double* Qs = S0 + s * L::DOUBLES + L::Q + (qbuf ^ 1) * M * L::LQ;
+                const int top = NS > 1 ? jac_slot_next(s, NS) : 0, bot = NS > 1 ? jac_slot_next(NS + s, NS) : 0;
+                dbl4 x[2][2];
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+#pragma unroll
+                    for (int o = 0; o < 2; ++o) x[h][o] = dbl4{0, 0, 0, 0};
+#pragma unroll
+                for (int k = 0; k < 2; ++k)
+#pragma unroll
+                    for (int kk = 0; kk < 4; ++kk) {
+                        if ((kk & 1) == 0 && go && done <= R) {
+                            asm volatile("s_barrier" ::: "memory");
+                            ++done;
+                        }
+#pragma unroll
+                        for (int o = 0; o < 2; ++o) {
+                            const double a = jac_qt(Qs, L::LQ, lane, o, k, kk);
+#pragma unroll
+                            for (int h = 0; h < 2; ++h)
+                                x[h][o] = __builtin_amdgcn_mfma_f64_16x16x4f64(
+                                    a, wt[h][k == 0 ? top : bot][kk], x[h][o], 0, 0, 0);
+                        }
+                    }
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    wt[h][top] = x[h][0];
+                    wt[h][bot] = x[h][1];
+                }
+            }
+            owed = 0;
+            if (go) {
+                for (; done <= R; ++done) asm volatile("s_barrier" ::: "memory");
+                apply(on);
+                owed = on;
+            }
+            next_slots();
+            dbl4 nx[2][NB];
+#pragma unroll
+            for (int b = 0; b < NB; ++b)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) nx[h][NS > 1 ? jac_slot_next(b, NS) : b] = wt[h][b];
+#pragma unroll
+            for (int b = 0; b < NB; ++b)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) wt[h][b] = nx[h][b];
+        });
+    } else if (role == ROT) {
+        const JacPlaces<M, NS> places(lane);
+        drive(scan_pair, [&](int on, bool go, bool cross) {
+            if (go) {
+                if (on >> sub & 1) jacobi_rounds<M, NS>(places, S, cs, lane, rounds_of(cross), cross, tol2);
+                else idle(rounds_of(cross));
+                apply(on);
+            }
+            next_slots();
+        });
+    } else {
+        JacRows<M> rows;
+        rows.identity(lane);
+        drive(scan_pair, [&](int on, bool go, bool cross) {
+            if (go) {
+                if (!(on >> sub & 1)) idle(rounds_of(cross));
+                else if (cross) rows.template rounds<true>(cs, lane, H);
+                else rows.template rounds<false>(cs, lane, M - 1);
+                if (NS > 1) {
+                    rows.store(S + L::Q + qbuf * M * L::LQ, L::LQ, lane);   // Q = 1 without a rotation
+                    rows.identity(lane);
+                }
+                apply(on);
+            }
+            next_slots();
+        });
+        if (NS == 1) rows.store(S + L::Q, L::LQ, lane);
+    }
+    // (the last sweep rotated nothing, so W lacks no Q; NB - 1 moves are the
+    // identity, so slot b holds block b)
     // order by |lambda| descending (stable by index), or keep the diagonal
     // positions, and write out
+    const double* dg = NS > 1 ? G : S0;
+    constexpr int LD1 = (NS > 1 ? LG : L::LS) + 1;
     if (t < n) {
-        const double li = G[t + t * ld], ai = fabs(li);
+        const double li = dg[t * LD1], ai = fabs(li);
         int k = t;
         if (!D.natural) {
             k = 0;
             for (int j = 0; j < n; ++j) {
-                const double aj = fabs(G[j + j * ld]);
+                const double aj = fabs(dg[j * LD1]);
                 k += (aj > ai) || (aj == ai && j < t);
             }
         }
@@ -1238,12 +1653,108 @@ __global__ __launch_bounds__(JT) void k_jacobi(const JacobiDesc* __restrict__ de
         D.lam[k] = li;
     }
     __syncthreads();
-    const float inv_n = 1.0f / (float)n;
-    for (int e = t; e < n * n; e += JT) {
-        const int i = (int)(((float)e + 0.5f) * inv_n), r = e - i * n;
-        D.W[r + (int64_t)pos[i] * D.ldw] = W[r + i * ld];
+    if (polish) {
+        // One Newton step towards the nearest orthogonal matrix,
+        // X <- (3/2 - X X^T / 2) X for X = W^T: a few hundred rotations leave
+        // W^T W off by ~1e-14, which singular vectors of close values feel as
+        // 1e-14 over their gap; the step leaves ~1e-15.  X takes G's place
+        // (n > 32), 3/2 - X X^T / 2 the block pairs' (n > 32) or S's.
+        constexpr int NX = NS > 1 ? NP : M, T = (NX + 15) / 16, LC = NS > 1 ? LG : L::LS;
+        static_assert(NX * LC <= (NS > 1 ? NS * L::DOUBLES : M * L::LS), "place for X X^T");
+        double* X = NS > 1 ? G : S + L::Q;
+        double* C = S0;
+        if (NS > 1 && role == STRIPS) {
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int b = 0; b < NB; ++b)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+                        X[JB * b + 4 * q + (lane >> 4) + (JB * (st0 + h) + (lane & 15)) * LG] = wt[h][b][q];
+        }
+        __syncthreads();
+        // entry (i, r) of X, 0 past its edge
+        auto x = [&](int i, int r) {
+            const int ic = NX % 16 ? min(i, NX - 1) : i, rc = NX % 16 ? min(r, NX - 1) : r;
+            const double v = NS > 1 ? X[ic + rc * LG] : X[rc + ic * L::LQ];
+            return NX % 16 && (i != ic || r != rc) ? 0.0 : v;
+        };
+        const int l0 = lane & 15, l1 = lane >> 4;
+        for (int u = w; u < T * (T + 1) / 2; u += L::WAVES) {
+            int J = 0;
+            while ((J + 1) * (J + 2) / 2 <= u) ++J;
+            const int I = u - J * (J + 1) / 2;
+            dbl4 c = dbl4{0, 0, 0, 0}, c2 = dbl4{0, 0, 0, 0};
+#pragma unroll 4
+            for (int kk = 0; kk < NX; kk += 8) {
+                c = __builtin_amdgcn_mfma_f64_16x16x4f64(x(16 * I + l0, kk + l1), x(16 * J + l0, kk + l1), c,
+                                                         0, 0, 0);
+                c2 = __builtin_amdgcn_mfma_f64_16x16x4f64(x(16 * I + l0, kk + 4 + l1),
+                                                          x(16 * J + l0, kk + 4 + l1), c2, 0, 0, 0);
+            }
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int i = 16 * I + 4 * q + l1, j = 16 * J + l0;
+                const double v = (i == j ? 1.5 : 0.0) - 0.5 * (c[q] + c2[q]);
+                if (NX % 16 == 0 || (i < NX && j < NX)) {
+                    C[i + j * LC] = v;
+                    C[j + i * LC] = v;
+                }
+            }
+        }
+        __syncthreads();
+        for (int u = w; u < T * T; u += L::WAVES) {
+            const int I = u / T, R = u - I * T;   // eigenvectors 16 I .., rows 16 R ..
+            const int ic = NX % 16 ? min(16 * I + l0, NX - 1) : 16 * I + l0;
+            dbl4 c = dbl4{0, 0, 0, 0}, c2 = dbl4{0, 0, 0, 0};
+#pragma unroll 4
+            for (int kk = 0; kk < NX; kk += 8) {
+                c = __builtin_amdgcn_mfma_f64_16x16x4f64(C[ic + (kk + l1) * LC], x(kk + l1, 16 * R + l0), c,
+                                                         0, 0, 0);
+                c2 = __builtin_amdgcn_mfma_f64_16x16x4f64(C[ic + (kk + 4 + l1) * LC],
+                                                          x(kk + 4 + l1, 16 * R + l0), c2, 0, 0, 0);
+            }
+            const int r = 16 * R + l0;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int i = 16 * I + 4 * q + l1;
+                if (i < n && r < n) D.W[r + (int64_t)pos[i] * D.ldw] = c[q] + c2[q];
+            }
+        }
+    } else if constexpr (NS == 1) {
+        for (int e = t; e < n * M; e += NT) {
+            const int i = e / M, r = e - i * M;
+            if (r < n) D.W[r + (int64_t)pos[i] * D.ldw] = S[L::Q + r + i * L::LQ];
+        }
+    } else if (role == STRIPS) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int r = JB * (st0 + h) + (lane & 15);
+#pragma unroll
+            for (int b = 0; b < NB; ++b)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const int i = JB * b + 4 * q + (lane >> 4);
+                    if (i < n && r < n) D.W[r + (int64_t)pos[i] * D.ldw] = wt[h][b][q];
+                }
+        }
     }
     if (t == 0 && D.sweeps) *D.sweeps = sweeps;
+}
+
+constexpr int JAC_TMAX = 64 * JacLds<JM, 3>::WAVES;
+
+__global__ __launch_bounds__(JAC_TMAX) void k_jacobi(const JacobiDesc* __restrict__ descs,
+                                                     int nd, double tol, int max_sweeps, bool polish) {
+    extern __shared__ double lds[];
+    const JacobiDesc D = descs[blockIdx.x];
+    if (D.skip && *D.skip) return;
+    // by the problem's own size, never by the rest of its group
+    if (D.n <= 16) jacobi_body<16, 1>(D, lds, tol, max_sweeps, polish);
+    else if (D.n <= 24) jacobi_body<24, 1>(D, lds, tol, max_sweeps, polish);
+    else if (D.n <= JM) jacobi_body<JM, 1>(D, lds, tol, max_sweeps, polish);
+    else if (D.n <= 2 * JM) jacobi_body<JM, 2>(D, lds, tol, max_sweeps, polish);
+    else jacobi_body<JM, 3>(D, lds, tol, max_sweeps, polish);
 }
 
 // ------------------------------------------------ pivoted Cholesky QR
@@ -2611,12 +3122,6 @@ void launch_trace_normalize(hipStream_t st, const TraceDesc* d_descs, const Trac
     TNR_HIP(hipGetLastError());
 }
 
-size_t jacobi_lds_bytes(int n) {
-    const size_t np = n + (n & 1);
-    return 2 * np * (np + 1) * sizeof(double) + (LMAX / 2) * sizeof(double) * 4 +
-           LMAX * sizeof(int);
-}
-
 void launch_jacobi(hipStream_t st, const JacobiDesc* d_descs, int nd, int nmax, double tol,
                    int max_sweeps) {
     if (nd <= 0) return;
@@ -2626,8 +3131,8 @@ void launch_jacobi(hipStream_t st, const JacobiDesc* d_descs, int nd, int nmax, 
         (int)jacobi_lds_bytes(LMAX));
     TNR_HIP(attr);
     ProfScope ps(st, PK_JACOBI, 0.0, 0.0);
-    TNR_LAUNCH(ps, k_jacobi, dim3(nd), dim3(JT), jacobi_lds_bytes(nmax), st, d_descs, nd, tol,
-                       max_sweeps);
+    TNR_LAUNCH(ps, k_jacobi, dim3(nd), dim3(jacobi_threads(nmax)), jacobi_lds_bytes(nmax), st, d_descs, nd,
+               tol, max_sweeps, tol < JPOLISH_BELOW);
     TNR_HIP(hipGetLastError());
     if (ps.active && prof_level() >= 2) {
         // profiling only: the work a launch did depends on the sweeps each
