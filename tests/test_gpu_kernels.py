@@ -247,6 +247,30 @@ def test_svd_block_wider_than_rank(tk):
     assert np.max(np.abs(V.T @ V - np.eye(k))) < 1e-12
 
 
+# block widths 2k on both sides of the Cholesky QR's 16-column panels and of
+# its 64-column kernel, on matrices whose rank ends inside, at the edge of and
+# beyond a panel
+@pytest.mark.parametrize("k", [3, 8, 12, 17, 24, 32, 33, 41])
+@pytest.mark.parametrize("extra", [0, 1, 7, 200])
+def test_svd_cholesky_panel_edges(tk, k, extra):
+    rng = np.random.default_rng(1000 + 10 * k + extra)
+    m, n = 230, 197
+    r = min(k + extra, n)
+    Ua, _ = np.linalg.qr(rng.standard_normal((m, r)))
+    Va, _ = np.linalg.qr(rng.standard_normal((n, r)))
+    sa = np.exp(-0.2 * np.arange(r))
+    M = (Ua * sa) @ Va.T
+    U, s, V, it = svd(tk, M, k)
+    assert it > 0
+    Ur, sr, Vtr = np.linalg.svd(M, full_matrices=False)
+    assert np.max(np.abs(s - sr[:k])) < 1e-13 * sr[0]
+    Mk = (U * s) @ V.T
+    Mr = (Ur[:, :k] * sr[:k]) @ Vtr[:k]
+    assert np.max(np.abs(Mk - Mr)) < 1e-12 * sr[0]
+    assert np.max(np.abs(U.T @ U - np.eye(k))) < 1e-12
+    assert np.max(np.abs(V.T @ V - np.eye(k))) < 1e-12
+
+
 @pytest.mark.parametrize("n,k", [(64, 16), (512, 32), (400, 120)])
 def test_eigh_truncated(tk, n, k):
     rng = np.random.default_rng(n)

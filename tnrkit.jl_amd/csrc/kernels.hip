@@ -1764,414 +1764,266 @@ __global__ __launch_bounds__(JAC_TMAX) void k_jacobi(const JacobiDesc* __restric
 // then X = R^{-1} (r x r).  Output W = P X (W[perm[i], j] = X[i, j], zero
 // columns from r on), so that Y W = Q has orthonormal columns spanning
 // span(Y), ordered by decreasing pivot; lam[j] = R[j][j] (the norm of
-// column j of Y after projecting out the earlier pivots).  Ties in the
-// pivot search go to the lowest index, so the result is a function of G.
-// k_cholqr64 takes n <= 64 in one wavefront, k_cholqr96 the larger sizes in
-// four; both keep the working matrix in registers.
-constexpr int CQ64 = 64;   // Gram matrices up to this size go to k_cholqr64
+// column j of Y after projecting out the earlier pivots).
+//
+// The n pivot steps depend on each other, so their latency is what counts.
+// Steps go in panels of 16 (left-looking inside a panel): one wave, lane =
+// row, finds the pivot by a 32-bit max over the wave, takes the pivot's column
+// of A as the last panel left it, subtracts this panel's earlier columns (the
+// lane's own row of L from registers, the pivot's from LDS) and updates the
+// remaining diagonal, with no barrier.  After a panel all waves update A by
+// L L^T on MFMA.  Rows are never moved: pivoted ones drop out of the search
+// and get L = 0.  X comes from the 16 x 16 diagonal blocks' inverses (lane =
+// column) and, by distance from the diagonal, X_IJ = -X_II sum_K R_IK X_KJ on
+// MFMA, the sum's result layout being the next product's operand layout.
+// The pivot search compares d to 17 (n <= 64) or 16 bits and settles ties
+// by the lowest index: a pivot within 2e-5 of the largest serves as well, and
+// the result is a function of G.
+// Measured (average launch in whole runs) against the former kernels, which
+// updated all of A and solved for X column by column after every pivot, in one
+// wave (n <= 64) or four: 39.6 -> 16.4 us at n = 32, 77 -> 35 at 64, 154 -> 60
+// at 96.
+constexpr int CQ64 = 64;   // Gram matrices up to this size take the 64-row kernel
 
-// Pivoted Cholesky QR of Gram matrices with at most CQ64 = 64 columns in
-// one wavefront that keeps the working matrix in registers, lane i
-// holding row i, so a pivot step has one wave-local barrier and no LDS
-// round trip per element.  Pivoting does not move data: the pivot's row is
-// broadcast through LDS and rows already pivoted drop out of the search.
-// Step j with pivot p, r = sqrt(A_j[p][p]): R[j][i] = A_j[p][i] / r (kept
-// over the original column indices), A_{j+1}[i][k] = A_j[i][k] -
-// (A_j[i][p] / r^2) A_j[p][k].  X = R^{-1} (R in pivot order) is solved
-// column by column, lane c holding column c in registers, by right-looking
-// elimination: rows kk from the last up, each scaled by 1 / R[kk][kk] and
-// eliminated from the rows above it.  Ties in the pivot search go to the
-// lowest row index.
-constexpr int CQLD = CQ64 + 1;   // padded stride of the LDS matrices
+template <int N>
+struct CholLds {
+    static constexpr int LD = N + 2;   // A, R, X by columns
+    static constexpr int LT = N + 1;   // L by rows (in X's place)
+    static constexpr int ROWS = (N + 63) / 64, BITS = N > 64 ? 7 : 6;
+    static constexpr int WAVES = N > 64 ? 8 : 4;
+    static constexpr size_t BYTES =
+        2 * (size_t)N * LD * sizeof(double) + 2 * N * sizeof(double) + (2 * N + 2) * sizeof(int);
+};
 
-size_t cholqr64_lds_bytes() {
-    return 2 * (size_t)CQ64 * CQLD * sizeof(double)   // R rows / staging, pivot-ordered R
-           + 2 * (size_t)CQ64 * sizeof(double)       // pivot rows (two, by step parity)
-           + 2 * (size_t)CQ64 * sizeof(double)       // R[j][j], 1 / R[j][j]
-           + 2 * (size_t)CQ64 * sizeof(int);         // perm, inverse perm
-}
-
-// One step of a wave argmax over (v, i) through DPP lane exchange CTRL:
-// larger v wins, equal v goes to the lower index.
+// Largest of x over the wave: within each row of 16 lanes by lane swaps, then
+// across rows (the broadcasts of the row before and of lane 31), read from
+// lane 63.
 template <int CTRL>
-__device__ __forceinline__ void argmax_dpp(double& v, int& i) {
-    const int lo = __double2loint(v), hi = __double2hiint(v);
-    const int lo2 = __builtin_amdgcn_update_dpp(lo, lo, CTRL, 0xF, 0xF, false);
-    const int hi2 = __builtin_amdgcn_update_dpp(hi, hi, CTRL, 0xF, 0xF, false);
-    const int i2 = __builtin_amdgcn_update_dpp(i, i, CTRL, 0xF, 0xF, false);
-    const double v2 = __hiloint2double(hi2, lo2);
-    const bool take = (v2 > v) | ((v2 == v) & (i2 < i));
-    v = take ? v2 : v;
-    i = take ? i2 : i;
+__device__ __forceinline__ unsigned max_dpp(unsigned x) {
+    return max(x, (unsigned)__builtin_amdgcn_update_dpp((int)x, (int)x, CTRL, 0xF, 0xF, false));
 }
 
-// Argmax of (v, i) over the wave, the same result in every lane: within
-// each row of 16 lanes by lane swaps (xor 1, xor 2, mirror within 8, mirror
-// within 16), then over the four rows' results read from lanes 0, 16, 32, 48.
-__device__ __forceinline__ void argmax_wave64(double& v, int& i) {
-    argmax_dpp<0xB1>(v, i);    // quad_perm [1, 0, 3, 2]
-    argmax_dpp<0x4E>(v, i);    // quad_perm [2, 3, 0, 1]
-    argmax_dpp<0x141>(v, i);   // row_half_mirror
-    argmax_dpp<0x140>(v, i);   // row_mirror
-    const int lo = __double2loint(v), hi = __double2hiint(v);
-    double bv = __hiloint2double(__builtin_amdgcn_readlane(hi, 0), __builtin_amdgcn_readlane(lo, 0));
-    int bi = __builtin_amdgcn_readlane(i, 0);
-#pragma unroll
-    for (int r = 1; r < 4; ++r) {
-        const double cv = __hiloint2double(__builtin_amdgcn_readlane(hi, 16 * r),
-                                           __builtin_amdgcn_readlane(lo, 16 * r));
-        const int ci = __builtin_amdgcn_readlane(i, 16 * r);
-        const bool take = (cv > bv) | ((cv == bv) & (ci < bi));
-        bv = take ? cv : bv;
-        bi = take ? ci : bi;
-    }
-    v = bv;
-    i = bi;
+__device__ __forceinline__ unsigned wave_max_u32(unsigned x) {
+    x = max_dpp<0xB1>(x);    // quad_perm [1, 0, 3, 2]
+    x = max_dpp<0x4E>(x);    // quad_perm [2, 3, 0, 1]
+    x = max_dpp<0x141>(x);   // row_half_mirror
+    x = max_dpp<0x140>(x);   // row_mirror
+    x = max_dpp<0x142>(x);   // row_bcast 15
+    x = max_dpp<0x143>(x);   // row_bcast 31
+    return (unsigned)__builtin_amdgcn_readlane((int)x, 63);
 }
 
-// (one wave per SIMD: the registers hold the rows and a whole pivot row in
-// flight)
-__global__ __launch_bounds__(CQ64) __attribute__((amdgpu_waves_per_eu(1, 1))) void k_cholqr64(
-    const JacobiDesc* __restrict__ descs, int nd, double null_rel2) {
+__device__ __forceinline__ double readlane_f64(double x, int l) {
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(x), l),
+                            __builtin_amdgcn_readlane(__double2loint(x), l));
+}
+
+template <int N>
+__global__ __launch_bounds__(64 * CholLds<N>::WAVES) void k_cholqr(const JacobiDesc* __restrict__ descs,
+                                                                  int nd, double null_rel2) {
+    using L = CholLds<N>;
+    constexpr int LD = L::LD, LT = L::LT, ROWS = L::ROWS, NT = 64 * L::WAVES;
     extern __shared__ double lds[];
     const JacobiDesc D = descs[blockIdx.x];
-    if (D.n > CQ64 || (D.skip && *D.skip)) return;
-    const int n = D.n, lane = threadIdx.x;
-    double* Rr = lds;                        // R[j][k] by original column: Rr[j * CQLD + k]
-    double* Rp = Rr + CQ64 * CQLD;           // G staging; later R[i][kk] at Rp[kk * CQ64 + i]
-    double* prow = Rp + CQ64 * CQLD;         // [2][CQ64]
-    double* rdiag = prow + 2 * CQ64;         // R[j][j]
-    double* rinv = rdiag + CQ64;             // 1 / R[j][j]
-    int* perm = (int*)(rinv + CQ64);
-    int* iperm = perm + CQ64;
-    const bool live = lane < n;
-    // G through LDS (coalesced column loads, zero outside n x n), then
-    // symmetrised rows into registers
-    {
-        // every lane loads (clamped, in bounds) and masks the bits, so the
-        // loads are not predicated and stay in flight together
-        const int ii = min(lane, n - 1);
+    // (the other sizes of the group are the other kernel's)
+    if (D.n > N || (N > CQ64 && D.n <= CQ64) || (D.skip && *D.skip)) return;
+    const int n = D.n, t = threadIdx.x, lane = t & 63, l0 = lane & 15, l1 = lane >> 4;
+    const int w = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int T = (n + 15) / 16, m = 16 * T;
+    double* A = lds;              // A[i + k LD]; later R in pivot order
+    double* X = A + N * LD;       // L[i][j] at X[i LT + j]; later X[i + j LD]
+    double* rdiag = X + N * LD;   // R[j][j], 1 / R[j][j]
+    double* rinv = rdiag + N;
+    int* perm = (int*)(rinv + N);
+    int* iperm = perm + N;
+    int* rank_ = iperm + N;
+    // every lane loads (clamped, in bounds), so the loads are not predicated
+    // and stay in flight together
+#pragma unroll 8
+    for (int e = t; e < m * N; e += NT) {
+        const int c = e / N, r = e - c * N;
+        const int rc = min(r, n - 1), cc = min(c, n - 1);
+        const double v = 0.5 * (D.G[rc + (int64_t)cc * D.ldg] + D.G[cc + (int64_t)rc * D.ldg]);
+        A[r + c * LD] = r < n && c < n ? v : 0.0;
+    }
+    if (t < N) {
+        iperm[t] = -1;
+        rdiag[t] = 0.0;
+        rinv[t] = 1.0;
+    }
+    if (t == 0) *rank_ = n;
+    __syncthreads();
+    // diagonal, and rows still to be pivoted (panel wave)
+    double d[ROWS];
+    bool left[ROWS];
+    double nfloor = 0.0, dmax = 0.0;
+    if (w == 0) {
 #pragma unroll
-        for (int c0 = 0; c0 < CQ64; c0 += 16) {
-            long long g[16];
+        for (int q = 0; q < ROWS; ++q) {
+            const int i = lane + 64 * q;
+            left[q] = i < n;
+            d[q] = left[q] ? A[min(i, n - 1) * (LD + 1)] : 0.0;
+            dmax = fmax(dmax, d[q]);
+        }
 #pragma unroll
-            for (int u = 0; u < 16; ++u)
-                g[u] = __double_as_longlong(D.G[ii + (int64_t)min(c0 + u, n - 1) * D.ldg]);
+        for (int o = 32; o > 0; o >>= 1) dmax = fmax(dmax, __shfl_xor(dmax, o, 64));
+        nfloor = null_rel2 * dmax;
+    }
+    // keys are taken of d / 2^e(dmax), in single precision's range
+    int e2 = 0;
+    if (dmax > 0.0 && dmax < INFINITY) e2 = ilogb(dmax);
+    int j = 0;
+    bool more = true;
+    for (int pb = 0; pb < T; ++pb) {
+        if (w == 0 && more) {
+            double lr[ROWS][16];
 #pragma unroll
-            for (int u = 0; u < 16; ++u) {
-                const long long keep = (live && c0 + u < n) ? -1LL : 0LL;
-                Rp[lane + (c0 + u) * CQLD] = __longlong_as_double(g[u] & keep);
+            for (int jj = 0; jj < 16; ++jj) {
+                if (!more) {
+#pragma unroll
+                    for (int q = 0; q < ROWS; ++q) {
+                        lr[q][jj] = 0.0;
+                        if (lane + 64 * q < N) X[(lane + 64 * q) * LT + 16 * pb + jj] = 0.0;
+                    }
+                    continue;
+                }
+                unsigned key = 0;
+#pragma unroll
+                for (int q = 0; q < ROWS; ++q) {
+                    const float s = fmaxf((float)ldexp(d[q], -e2), 0.0f);
+                    constexpr unsigned LOW = (1u << L::BITS) - 1;
+                    const unsigned kq = (__float_as_uint(s) & ~LOW) | (LOW - (unsigned)(lane + 64 * q));
+                    key = left[q] && kq > key ? kq : key;
+                }
+                key = wave_max_u32(key);
+                constexpr unsigned LOW = (1u << L::BITS) - 1;
+                const int p = (int)(LOW - (key & LOW));
+                const double v = key == 0 ? 0.0
+                                          : (ROWS > 1 && p >= 64 ? readlane_f64(d[ROWS - 1], p - 64)
+                                                                 : readlane_f64(d[0], p & 63));
+                j = 16 * pb + jj;
+                if (j >= n || !(v > nfloor && dmax > 0.0)) {
+                    more = false;
+                    if (lane == 0 && j < n) *rank_ = j;
+#pragma unroll
+                    for (int q = 0; q < ROWS; ++q) {
+                        lr[q][jj] = 0.0;
+                        if (lane + 64 * q < N) X[(lane + 64 * q) * LT + 16 * pb + jj] = 0.0;
+                    }
+                    continue;
+                }
+                const double rs = rsqrt_refined(v);
+                double c[ROWS], lp[16];
+#pragma unroll
+                for (int q = 0; q < ROWS; ++q) c[q] = A[min(lane + 64 * q, N - 1) + p * LD];
+#pragma unroll
+                for (int k = 0; k < jj; ++k) lp[k] = X[p * LT + 16 * pb + k];
+#pragma unroll
+                for (int q = 0; q < ROWS; ++q) {
+                    double c2 = 0.0;
+#pragma unroll
+                    for (int k = 0; k < jj; ++k) {
+                        if (k & 1) c2 = fma(-lr[q][k], lp[k], c2);
+                        else c[q] = fma(-lr[q][k], lp[k], c[q]);
+                    }
+                    const int i = lane + 64 * q;
+                    double l = (c[q] + c2) * rs;
+                    l = i == p ? v * rs : l;
+                    l = left[q] ? l : 0.0;
+                    lr[q][jj] = l;
+                    d[q] = fma(-l, l, d[q]);
+                    left[q] = left[q] && i != p;
+                    if (i < N) X[i * LT + j] = l;
+                }
+                if (lane == 0) {
+                    perm[j] = p;
+                    iperm[p] = j;
+                    rdiag[j] = v * rs;
+                    rinv[j] = rs;
+                }
+                wave_order();
             }
-        }
-    }
-    __syncthreads();
-    double a[CQ64];
-#pragma unroll
-    for (int k = 0; k < CQ64; ++k) a[k] = 0.5 * (Rp[lane + k * CQLD] + Rp[k + lane * CQLD]);
-    double d = Rp[lane + lane * CQLD];   // = a[lane]
-    double dmax = d;
-    {
-        int ii = lane;
-        argmax_wave64(dmax, ii);
-    }
-    const double nfloor = null_rel2 * dmax;
-    bool done = !live;
-    int rank = n;
-    double v = live ? d : -1.0;
-    int p = live ? lane : n;
-    argmax_wave64(v, p);
-    for (int j = 0; j < n; ++j) {
-        if (!(v > nfloor && dmax > 0.0)) {
-            rank = j;
-            break;
-        }
-        double* pr = prow + (j & 1) * CQ64;
-        if (lane == p) {
-#pragma unroll
-            for (int k = 0; k < CQ64; k += 2) *(double2*)(pr + k) = make_double2(a[k], a[k + 1]);
-            done = true;
-        }
-        const double r = sqrt(v), ri = 1.0 / r;
-        __syncthreads();
-        const double aip = pr[lane];                  // A_j[p][i] = A_j[i][p]
-        Rr[j * CQLD + lane] = lane == p ? r : aip * ri;
-        if (lane == 0) {
-            perm[j] = p;
-            rdiag[j] = r;
-            rinv[j] = ri;
-        }
-        // rows already pivoted keep their values (zero multiplier); the next
-        // pivot search needs only d and overlaps the row updates
-        const double f = done ? 0.0 : (aip * ri) * ri;
-        d = d - f * aip;
-        v = done ? -1.0 : d;
-        p = done ? n : lane;
-        double2 row[CQ64 / 2];
-#pragma unroll
-        for (int k = 0; k < CQ64 / 2; ++k) row[k] = *(const double2*)(pr + 2 * k);
-        argmax_wave64(v, p);
-#pragma unroll
-        for (int k = 0; k < CQ64 / 2; ++k) {
-            a[2 * k] = a[2 * k] - f * row[k].x;
-            a[2 * k + 1] = a[2 * k + 1] - f * row[k].y;
-        }
-    }
-    __syncthreads();
-    // R in pivot order, column kk contiguous: Rp[kk * CQ64 + i] = R[i][kk]
-    iperm[lane] = -1;
-    for (int kk = 0; kk < rank; ++kk) Rp[kk * CQ64 + lane] = Rr[lane * CQLD + perm[kk]];
-    __syncthreads();
-    if (lane < rank) iperm[perm[lane]] = lane;
-    // X = R^{-1}: lane c holds column c; rows kk from the last up, each
-    // scaled by 1 / R[kk][kk] and eliminated from the rows above it
-    double* x = a;
-#pragma unroll
-    for (int i = 0; i < CQ64; ++i) x[i] = (i == lane && lane < rank) ? 1.0 : 0.0;
-#pragma unroll
-    for (int kk = CQ64 - 1; kk >= 0; --kk) {
-        if (kk < rank) {
-            x[kk] *= rinv[kk];
-            const double* col = Rp + kk * CQ64;
-#pragma unroll
-            for (int i = 0; i + 1 < kk; i += 2) {
-                const double2 rr = *(const double2*)(col + i);
-                x[i] = x[i] - rr.x * x[kk];
-                x[i + 1] = x[i + 1] - rr.y * x[kk];
-            }
-            if (kk & 1) x[kk - 1] = x[kk - 1] - col[kk - 1] * x[kk];
-        }
-    }
-    // stage X by columns (X[i][c] at Rr[i + c * CQLD]), then W[perm[i]][c] =
-    // X[i][c] for i <= c < rank and zero elsewhere, one coalesced column at a time
-#pragma unroll
-    for (int i = 0; i < CQ64; ++i) Rr[i + lane * CQLD] = x[i];
-    __syncthreads();
-    const int ip = iperm[lane];
-    if (live)
-        for (int c = 0; c < n; ++c)
-            D.W[lane + (int64_t)c * D.ldw] =
-                (ip >= 0 && ip <= c && c < rank) ? Rr[ip + c * CQLD] : 0.0;
-    if (live) D.lam[lane] = lane < rank ? rdiag[lane] : 0.0;
-    if (lane == 0 && D.sweeps) *D.sweeps = 0;
-}
-
-// Pivoted Cholesky QR of Gram matrices with CQ64 < n <= LMAX columns: the
-// arithmetic of k_cholqr64 over four wavefronts.  Thread (w, lane) holds
-// row i = lane + 64 (w & 1) of the working matrix, columns CQH (w >> 1) to
-// CQH (w >> 1) + CQH - 1, in registers.  At each pivot step the best
-// remaining row of each row-wave (w & 1) publishes itself in LDS (buffers
-// alternate by step parity), so a step takes one workgroup barrier, after
-// which every thread picks the larger of the two candidates (ties to the
-// lower index) and reads its row.  X = R^{-1} is solved with thread (w,
-// lane) holding column c = lane + 64 (w & 1), rows CQH (w >> 1) to
-// CQH (w >> 1) + CQH - 1: the elimination runs from the last row up, so the
-// waves holding rows CQH.. finish them first and hand them through LDS to
-// the waves holding rows 0..CQH-1; every element takes the same updates in
-// the same order as in a one-thread right-looking elimination.
-constexpr int CQH = LMAX / 2;     // columns (factorisation) / rows (inverse) per thread
-constexpr int CQLDM = LMAX + 1;   // padded stride of the LDS matrices
-constexpr int CQ96T = 256;
-static_assert(LMAX * LMAX % (4 * CQ96T) == 0 && CQH % 2 == 0 && LMAX <= 2 * 64,
-              "k_cholqr96 tiling");
-
-size_t cholqr96_lds_bytes() {
-    return 2 * (size_t)LMAX * CQLDM * sizeof(double)   // G staging / pivot-ordered R; R rows / X
-           + 4 * (size_t)LMAX * sizeof(double)         // candidate rows [step parity][row-wave]
-           + 4 * sizeof(double)                        // candidate values
-           + 2 * (size_t)LMAX * sizeof(double)         // R[j][j], 1 / R[j][j]
-           + 4 * sizeof(int)                           // candidate rows' indices
-           + 2 * (size_t)LMAX * sizeof(int);           // perm, inverse perm
-}
-
-__global__ __launch_bounds__(CQ96T) __attribute__((amdgpu_waves_per_eu(1, 1))) void k_cholqr96(
-    const JacobiDesc* __restrict__ descs, int nd, double null_rel2) {
-    extern __shared__ double lds[];
-    const JacobiDesc D = descs[blockIdx.x];
-    if (D.n <= CQ64 || D.n > LMAX || (D.skip && *D.skip)) return;
-    const int n = D.n, t = threadIdx.x, lane = t & 63;
-    const int w = __builtin_amdgcn_readfirstlane(t >> 6), rw = w & 1, h = w >> 1;
-    const int i = lane + 64 * rw;    // row (factorisation), column (inverse)
-    const int ii = min(i, n - 1);    // in-bounds stand-in for rows past n
-    const bool live = i < n;
-    double* Gs = lds;                          // G staging; later R[r][kk] at Gs[kk * LMAX + r]
-    double* Rr = Gs + LMAX * CQLDM;            // R[j][k] by original column k; later X
-    double* cand = Rr + LMAX * CQLDM;          // [2][2][LMAX]
-    double* candv = cand + 4 * LMAX;           // [2][2]
-    double* rdiag = candv + 4;
-    double* rinv = rdiag + LMAX;
-    int* candp = (int*)(rinv + LMAX);          // [2][2]
-    int* perm = candp + 4;
-    int* iperm = perm + LMAX;
-    // G into LDS, zero outside n x n (clamped loads, masked bits, so the
-    // loads are not predicated and stay in flight together)
-    for (int e0 = 0; e0 < LMAX * LMAX; e0 += 4 * CQ96T) {
-        long long g[4];
-        int at[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int e = e0 + u * CQ96T + t, c = e / LMAX, r = e - c * LMAX;
-            g[u] = __double_as_longlong(D.G[min(r, n - 1) + (int64_t)min(c, n - 1) * D.ldg]);
-            g[u] &= (r < n && c < n) ? -1LL : 0LL;
-            at[u] = r + c * CQLDM;
-        }
-#pragma unroll
-        for (int u = 0; u < 4; ++u) Gs[at[u]] = __longlong_as_double(g[u]);
-    }
-    if (t < LMAX) iperm[t] = -1;
-    __syncthreads();
-    double a[CQH];
-#pragma unroll
-    for (int k = 0; k < CQH; ++k) {
-        const int c = h * CQH + k;
-        a[k] = 0.5 * (Gs[ii + c * CQLDM] + Gs[c + ii * CQLDM]);
-    }
-    double d = live ? Gs[ii + ii * CQLDM] : 0.0;
-    {
-        // largest diagonal over both row-waves, through the parity-1 value
-        // slots (first rewritten at step 1, after the step-0 barrier)
-        double dm = d;
-        int di = i;
-        argmax_wave64(dm, di);
-        if (h == 0 && lane == 0) candv[2 + rw] = dm;
-    }
-    __syncthreads();
-    const double dmax = candv[3] > candv[2] ? candv[3] : candv[2];
-    const double nfloor = null_rel2 * dmax;
-    bool done = !live;
-    int rank = n;
-    double v = live ? d : -1.0;
-    int p = live ? i : n;
-    argmax_wave64(v, p);
-    for (int j = 0; j < n; ++j) {
-        const int b = j & 1;
-        double* cb = cand + b * 2 * LMAX;
-        if (p < n && i == p) {
-            double* dst = cb + rw * LMAX + h * CQH;
-#pragma unroll
-            for (int k = 0; k < CQH; k += 2) *(double2*)(dst + k) = make_double2(a[k], a[k + 1]);
-        }
-        if (h == 0 && lane == 0) {
-            candv[2 * b + rw] = v;
-            candp[2 * b + rw] = p;
         }
         __syncthreads();
-        // buffers of parity b are next written at step j + 2, after the
-        // step j + 1 barrier, which every thread reaches only once it has
-        // read them here
-        const double v0 = candv[2 * b], v1 = candv[2 * b + 1];
-        const int p0 = candp[2 * b], p1 = candp[2 * b + 1];
-        const bool s1 = (v1 > v0) | ((v1 == v0) & (p1 < p0));
-        const double vb = s1 ? v1 : v0;
-        const int pb = s1 ? p1 : p0;
-        if (!(vb > nfloor && dmax > 0.0)) {
-            rank = j;
-            break;
-        }
-        const double* pr = cb + (s1 ? LMAX : 0);
-        const double r = sqrt(vb), ri = 1.0 / r;
-        const double aip = pr[ii];   // A_j[p][i] = A_j[i][p]
-        if (h == 0 && live) Rr[j * CQLDM + i] = i == pb ? r : aip * ri;
-        if (t == 0) {
-            perm[j] = pb;
-            rdiag[j] = r;
-            rinv[j] = ri;
-        }
-        if (i == pb) done = true;
-        const double f = done ? 0.0 : (aip * ri) * ri;
-        d = d - f * aip;
-        v = done ? -1.0 : d;
-        p = done ? n : i;
-        double2 row[CQH / 2];
+        if (*rank_ < min(n, 16 * (pb + 1))) break;   // (the same for every thread)
+        if (pb + 1 < T) {
+            for (int u = w; u < T * (T + 1) / 2; u += L::WAVES) {
+                int J = 0;
+                while ((J + 1) * (J + 2) / 2 <= u) ++J;
+                const int I = u - J * (J + 1) / 2;
+                dbl4 c;
+                double* at = A + 16 * I + l1 + (16 * J + l0) * LD;
 #pragma unroll
-        for (int k = 0; k < CQH / 2; ++k) row[k] = *(const double2*)(pr + h * CQH + 2 * k);
-        argmax_wave64(v, p);
+                for (int q = 0; q < 4; ++q) c[q] = at[4 * q];
 #pragma unroll
-        for (int k = 0; k < CQH / 2; ++k) {
-            a[2 * k] = a[2 * k] - f * row[k].x;
-            a[2 * k + 1] = a[2 * k + 1] - f * row[k].y;
-        }
-    }
-    __syncthreads();
-    // R in pivot order, column kk contiguous: Rp[kk * LMAX + r] = R[r][kk]
-    double* Rp = Gs;
-    for (int e = t; e < rank * LMAX; e += CQ96T) {
-        const int kk = e / LMAX, r = e - kk * LMAX;
-        Rp[e] = r < rank ? Rr[r * CQLDM + perm[kk]] : 0.0;
-    }
-    if (t < rank) iperm[perm[t]] = t;
-    __syncthreads();
-    // X = R^{-1}, X[r][c] staged at X[r + c * CQLDM]
-    double* X = Rr;
-    const int c = i, cc = min(c, LMAX - 1);
-    double x[CQH];
+                for (int kk = 0; kk < 4; ++kk)
+                    c = __builtin_amdgcn_mfma_f64_16x16x4f64(-X[(16 * I + l0) * LT + 16 * pb + 4 * kk + l1],
+                                                             X[(16 * J + l0) * LT + 16 * pb + 4 * kk + l1], c,
+                                                             0, 0, 0);
+                double* ta = A + 16 * J + l0 + (16 * I + l1) * LD;
 #pragma unroll
-    for (int k = 0; k < CQH; ++k) x[k] = (h * CQH + k == c && c < rank) ? 1.0 : 0.0;
-    if (h == 1) {
-        // rows CQH.. : rows kk from the last up, scaled and eliminated from
-        // the rows above them within this half
-#pragma unroll
-        for (int kk = LMAX - 1; kk >= CQH; --kk) {
-            if (kk < rank) {
-                const int q = kk - CQH;
-                x[q] *= rinv[kk];
-                const double* col = Rp + kk * LMAX + CQH;
-#pragma unroll
-                for (int m = 0; m + 1 < q; m += 2) {
-                    const double2 rr = *(const double2*)(col + m);
-                    x[m] = x[m] - rr.x * x[q];
-                    x[m + 1] = x[m + 1] - rr.y * x[q];
-                }
-                if (q & 1) x[q - 1] = x[q - 1] - col[q - 1] * x[q];
-            }
-        }
-        if (c < n)
-#pragma unroll
-            for (int k = 0; k < CQH; ++k) X[CQH + k + c * CQLDM] = x[k];
-    }
-    __syncthreads();
-    if (h == 0) {
-        // rows below CQH: first the eliminations of rows CQH.. (final now),
-        // in the same descending order, then their own
-#pragma unroll
-        for (int kk = LMAX - 1; kk >= CQH; --kk) {
-            if (kk < rank) {
-                const double xk = X[kk + cc * CQLDM];
-                const double* col = Rp + kk * LMAX;
-#pragma unroll
-                for (int m = 0; m < CQH; m += 2) {
-                    const double2 rr = *(const double2*)(col + m);
-                    x[m] = x[m] - rr.x * xk;
-                    x[m + 1] = x[m + 1] - rr.y * xk;
+                for (int q = 0; q < 4; ++q) {
+                    at[4 * q] = c[q];
+                    if (I != J) ta[4 * q * LD] = c[q];
                 }
             }
+            __syncthreads();
         }
-#pragma unroll
-        for (int kk = CQH - 1; kk >= 0; --kk) {
-            if (kk < rank) {
-                x[kk] *= rinv[kk];
-                const double* col = Rp + kk * LMAX;
-#pragma unroll
-                for (int m = 0; m + 1 < kk; m += 2) {
-                    const double2 rr = *(const double2*)(col + m);
-                    x[m] = x[m] - rr.x * x[kk];
-                    x[m + 1] = x[m + 1] - rr.y * x[kk];
-                }
-                if (kk & 1) x[kk - 1] = x[kk - 1] - col[kk - 1] * x[kk];
-            }
-        }
-        if (c < n)
-#pragma unroll
-            for (int k = 0; k < CQH; ++k) X[k + c * CQLDM] = x[k];
+    }
+    const int rank = *rank_;
+    // R in pivot order: R[i + k LD] = R[i][k] for i <= k < rank, else 1 / 0
+    // (in A's place)
+    for (int e = t; e < m * m; e += NT) {
+        const int c = e / m, r = e - c * m;
+        A[r + c * LD] = c < rank && r <= c ? X[perm[c] * LT + r] : (r == c ? 1.0 : 0.0);
     }
     __syncthreads();
-    // W[perm[r]][cj] = X[r][cj] for r <= cj < rank, zero elsewhere; one
-    // coalesced column per wave at a time
-    for (int cj = w; cj < n; cj += CQ96T / 64)
-        for (int r = lane; r < n; r += 64) {
-            const int ip = iperm[r];
-            D.W[r + (int64_t)cj * D.ldw] =
-                (ip >= 0 && ip <= cj && cj < rank) ? X[ip + cj * CQLDM] : 0.0;
+    // diagonal blocks of X = R^{-1}, four a wave: lane = (block, column)
+    for (int b0 = 4 * w; b0 < T; b0 += 4 * L::WAVES) {
+        const int B = min(b0 + l1, T - 1);
+        double x[16];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) x[i] = i == l0 ? 1.0 : 0.0;
+#pragma unroll
+        for (int kk = 15; kk >= 0; --kk) {
+            x[kk] *= rinv[16 * B + kk];
+            const double* col = A + 16 * B + (16 * B + kk) * LD;
+#pragma unroll
+            for (int i = 0; i < kk; ++i) x[i] = fma(-col[i], x[kk], x[i]);
         }
+        // (spare lanes repeat the last block)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) X[16 * B + i + (16 * B + l0) * LD] = x[i];
+    }
+    __syncthreads();
+    for (int dist = 1; dist < T; ++dist) {
+        for (int I = w; I + dist < T; I += L::WAVES) {
+            const int J = I + dist;
+            dbl4 s = dbl4{0, 0, 0, 0};
+            for (int K = I + 1; K <= J; ++K)
+#pragma unroll
+                for (int kk = 0; kk < 4; ++kk)
+                    s = __builtin_amdgcn_mfma_f64_16x16x4f64(A[16 * I + l0 + (16 * K + 4 * kk + l1) * LD],
+                                                             X[16 * K + 4 * kk + l1 + (16 * J + l0) * LD], s,
+                                                             0, 0, 0);
+            dbl4 x = dbl4{0, 0, 0, 0};
+#pragma unroll
+            for (int kk = 0; kk < 4; ++kk)
+                x = __builtin_amdgcn_mfma_f64_16x16x4f64(-X[16 * I + l0 + (16 * I + 4 * kk + l1) * LD], s[kk],
+                                                         x, 0, 0, 0);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) X[16 * I + l1 + 4 * q + (16 * J + l0) * LD] = x[q];
+        }
+        __syncthreads();
+    }
+    // W[perm[r]][c] = X[r][c] for r <= c < rank, zero elsewhere
+#pragma unroll 4
+    for (int e = t; e < n * N; e += NT) {
+        const int c = e / N, r = e - c * N;
+        const int ip = iperm[r];
+        if (r < n)
+            D.W[r + (int64_t)c * D.ldw] = ip >= 0 && ip <= c && c < rank ? X[ip + c * LD] : 0.0;
+    }
     if (t < n) D.lam[t] = t < rank ? rdiag[t] : 0.0;
     if (t == 0 && D.sweeps) *D.sweeps = 0;
 }
@@ -3160,32 +3012,25 @@ void launch_jacobi(hipStream_t st, const JacobiDesc* d_descs, int nd, int nmax, 
 }
 
 
-// Problems of at most CQ64 columns run on k_cholqr64, larger ones on
-// k_cholqr96 (each kernel skips the other's), so the kernel a problem gets
+// Problems of at most CQ64 columns run on k_cholqr<64>, larger ones on
+// k_cholqr<LMAX> (each kernel skips the other's), so the kernel a problem gets
 // depends on its own size only, never on the rest of its launch group.
+template <int N>
+static void launch_cholqr_n(hipStream_t st, const JacobiDesc* d_descs, int nd, double null_rel2) {
+    static const hipError_t attr = hipFuncSetAttribute(
+        (const void*)k_cholqr<N>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)CholLds<N>::BYTES);
+    TNR_HIP(attr);
+    ProfScope ps(st, PK_JACOBI, 0.0, 0.0);
+    TNR_LAUNCH(ps, k_cholqr<N>, dim3(nd), dim3(64 * CholLds<N>::WAVES), CholLds<N>::BYTES, st, d_descs, nd,
+               null_rel2);
+    TNR_HIP(hipGetLastError());
+}
+
 void launch_cholqr(hipStream_t st, const JacobiDesc* d_descs, int nd, int nmin, int nmax,
                    double null_rel2) {
     if (nd <= 0) return;
-    static const hipError_t attr = hipFuncSetAttribute(
-        (const void*)k_cholqr96, hipFuncAttributeMaxDynamicSharedMemorySize,
-        (int)cholqr96_lds_bytes());
-    TNR_HIP(attr);
-    static const hipError_t attr64 = hipFuncSetAttribute(
-        (const void*)k_cholqr64, hipFuncAttributeMaxDynamicSharedMemorySize,
-        (int)cholqr64_lds_bytes());
-    TNR_HIP(attr64);
-    if (nmin <= CQ64) {
-        ProfScope ps(st, PK_JACOBI, 0.0, 0.0);
-        TNR_LAUNCH(ps, k_cholqr64, dim3(nd), dim3(CQ64), cholqr64_lds_bytes(), st, d_descs, nd,
-                   null_rel2);
-        TNR_HIP(hipGetLastError());
-    }
-    if (nmax > CQ64) {
-        ProfScope ps(st, PK_JACOBI, 0.0, 0.0);
-        TNR_LAUNCH(ps, k_cholqr96, dim3(nd), dim3(CQ96T), cholqr96_lds_bytes(), st, d_descs, nd,
-                   null_rel2);
-        TNR_HIP(hipGetLastError());
-    }
+    if (nmin <= CQ64) launch_cholqr_n<CQ64>(st, d_descs, nd, null_rel2);
+    if (nmax > CQ64) launch_cholqr_n<LMAX>(st, d_descs, nd, null_rel2);
 }
 
 void launch_lincomb(hipStream_t st, const LinDesc* d_descs, int nd, int64_t total) {
