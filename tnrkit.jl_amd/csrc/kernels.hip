@@ -1776,21 +1776,22 @@ __global__ __launch_bounds__(JAC_TMAX) void k_jacobi(const JacobiDesc* __restric
 // and get L = 0.  X comes from the 16 x 16 diagonal blocks' inverses (lane =
 // column) and, by distance from the diagonal, X_IJ = -X_II sum_K R_IK X_KJ on
 // MFMA, the sum's result layout being the next product's operand layout.
-// The pivot search compares d to 17 (n <= 64) or 16 bits and settles ties
-// by the lowest index: a pivot within 2e-5 of the largest serves as well, and
-// the result is a function of G.
+// The pivot search compares the leading 14 (n <= 64) or 13 bits of d's mantissa
+// and settles ties by the lowest index: a pivot within 1e-4 of the largest
+// serves as well, and the result is a function of G.  G is taken as the
+// product of one GEMM, whose two triangles agree bit for bit.
 // Measured (average launch in whole runs) against the former kernels, which
 // updated all of A and solved for X column by column after every pivot, in one
-// wave (n <= 64) or four: 39.6 -> 16.4 us at n = 32, 77 -> 35 at 64, 154 -> 60
-// at 96.
+// wave (n <= 64) or four: 39.6 -> 11.6 us at n = 32, 77 -> 22 at 64, 154 -> 46
+// at 96.  A pivot step takes 0.23 us (0.38 with the control flow in vector
+// registers and keys converted to single precision).
 constexpr int CQ64 = 64;   // Gram matrices up to this size take the 64-row kernel
 
 template <int N>
 struct CholLds {
-    static constexpr int LD = N + 2;   // A, R, X by columns
-    static constexpr int LT = N + 1;   // L by rows (in X's place)
+    static constexpr int LD = N + 2;   // A, R, X by columns; L by rows (in X's place)
     static constexpr int ROWS = (N + 63) / 64, BITS = N > 64 ? 7 : 6;
-    static constexpr int WAVES = N > 64 ? 8 : 4;
+    static constexpr int WAVES = 8;
     static constexpr size_t BYTES =
         2 * (size_t)N * LD * sizeof(double) + 2 * N * sizeof(double) + (2 * N + 2) * sizeof(int);
 };
@@ -1799,30 +1800,25 @@ struct CholLds {
 // across rows (the broadcasts of the row before and of lane 31), read from
 // lane 63.
 template <int CTRL>
-__device__ __forceinline__ unsigned max_dpp(unsigned x) {
-    return max(x, (unsigned)__builtin_amdgcn_update_dpp((int)x, (int)x, CTRL, 0xF, 0xF, false));
+__device__ __forceinline__ int max_dpp(int x) {
+    return max(x, __builtin_amdgcn_update_dpp(INT32_MIN, x, CTRL, 0xF, 0xF, false));
 }
 
-__device__ __forceinline__ unsigned wave_max_u32(unsigned x) {
+__device__ __forceinline__ int wave_max_i32(int x) {
     x = max_dpp<0xB1>(x);    // quad_perm [1, 0, 3, 2]
     x = max_dpp<0x4E>(x);    // quad_perm [2, 3, 0, 1]
     x = max_dpp<0x141>(x);   // row_half_mirror
     x = max_dpp<0x140>(x);   // row_mirror
     x = max_dpp<0x142>(x);   // row_bcast 15
     x = max_dpp<0x143>(x);   // row_bcast 31
-    return (unsigned)__builtin_amdgcn_readlane((int)x, 63);
-}
-
-__device__ __forceinline__ double readlane_f64(double x, int l) {
-    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(x), l),
-                            __builtin_amdgcn_readlane(__double2loint(x), l));
+    return __builtin_amdgcn_readlane(x, 63);
 }
 
 template <int N>
 __global__ __launch_bounds__(64 * CholLds<N>::WAVES) void k_cholqr(const JacobiDesc* __restrict__ descs,
                                                                   int nd, double null_rel2) {
     using L = CholLds<N>;
-    constexpr int LD = L::LD, LT = L::LT, ROWS = L::ROWS, NT = 64 * L::WAVES;
+    constexpr int LD = L::LD, ROWS = L::ROWS, NT = 64 * L::WAVES;
     extern __shared__ double lds[];
     const JacobiDesc D = descs[blockIdx.x];
     // (the other sizes of the group are the other kernel's)
@@ -1831,9 +1827,9 @@ __global__ __launch_bounds__(64 * CholLds<N>::WAVES) void k_cholqr(const JacobiD
     const int w = __builtin_amdgcn_readfirstlane(t >> 6);
     const int T = (n + 15) / 16, m = 16 * T;
     double* A = lds;              // A[i + k LD]; later R in pivot order
-    double* X = A + N * LD;       // L[i][j] at X[i LT + j]; later X[i + j LD]
-    double* rdiag = X + N * LD;   // R[j][j], 1 / R[j][j]
-    double* rinv = rdiag + N;
+    double* X = A + N * LD;       // L[i][j] at X[i LD + j]; later X[i + j LD]
+    double* piv = X + N * LD;     // pivot values, then R[j][j]
+    double* rinv = piv + N;       // 1 / R[j][j]
     int* perm = (int*)(rinv + N);
     int* iperm = perm + N;
     int* rank_ = iperm + N;
@@ -1842,140 +1838,132 @@ __global__ __launch_bounds__(64 * CholLds<N>::WAVES) void k_cholqr(const JacobiD
 #pragma unroll 8
     for (int e = t; e < m * N; e += NT) {
         const int c = e / N, r = e - c * N;
-        const int rc = min(r, n - 1), cc = min(c, n - 1);
-        const double v = 0.5 * (D.G[rc + (int64_t)cc * D.ldg] + D.G[cc + (int64_t)rc * D.ldg]);
+        const double v = D.G[min(r, n - 1) + (int64_t)min(c, n - 1) * D.ldg];
         A[r + c * LD] = r < n && c < n ? v : 0.0;
     }
-    if (t < N) {
-        iperm[t] = -1;
-        rdiag[t] = 0.0;
-        rinv[t] = 1.0;
-    }
+    if (t < N) iperm[t] = -1;
     if (t == 0) *rank_ = n;
     __syncthreads();
-    // diagonal, and rows still to be pivoted (panel wave)
+    // what is left of the diagonal (panel wave); -1 in a pivoted row, whose
+    // entries of L, A and R-to-be past its own step are not used
     double d[ROWS];
-    bool left[ROWS];
-    double nfloor = 0.0, dmax = 0.0;
+    double nfloor = 0.0;
     if (w == 0) {
+        double dmax = 0.0;
 #pragma unroll
         for (int q = 0; q < ROWS; ++q) {
             const int i = lane + 64 * q;
-            left[q] = i < n;
-            d[q] = left[q] ? A[min(i, n - 1) * (LD + 1)] : 0.0;
+            d[q] = i < n ? A[min(i, n - 1) * (LD + 1)] : -1.0;
             dmax = fmax(dmax, d[q]);
         }
 #pragma unroll
         for (int o = 32; o > 0; o >>= 1) dmax = fmax(dmax, __shfl_xor(dmax, o, 64));
         nfloor = null_rel2 * dmax;
     }
-    // keys are taken of d / 2^e(dmax), in single precision's range
-    int e2 = 0;
-    if (dmax > 0.0 && dmax < INFINITY) e2 = ilogb(dmax);
-    int j = 0;
-    bool more = true;
     for (int pb = 0; pb < T; ++pb) {
-        if (w == 0 && more) {
+        if (w == 0) {
+            const int steps = min(16, n - 16 * pb);
             double lr[ROWS][16];
+            int pv = 0, vl = 0, vh = 0, stop = 16;   // lane jj: pivot row and value of step jj
 #pragma unroll
             for (int jj = 0; jj < 16; ++jj) {
-                if (!more) {
+                if (stop < 16) continue;
+                constexpr int LOW = (1 << L::BITS) - 1;
+                int key = INT32_MIN;
 #pragma unroll
-                    for (int q = 0; q < ROWS; ++q) {
-                        lr[q][jj] = 0.0;
-                        if (lane + 64 * q < N) X[(lane + 64 * q) * LT + 16 * pb + jj] = 0.0;
-                    }
+                for (int q = 0; q < ROWS; ++q)
+                    key = max(key, (__double2hiint(d[q]) & ~LOW) | (LOW - (lane + 64 * q)));
+                const int p = LOW - (wave_max_i32(key) & LOW);
+                int hi, lo;
+                if (ROWS > 1 && p >= 64) {
+                    hi = __builtin_amdgcn_readlane(__double2hiint(d[ROWS - 1]), p - 64);
+                    lo = __builtin_amdgcn_readlane(__double2loint(d[ROWS - 1]), p - 64);
+                } else {
+                    hi = __builtin_amdgcn_readlane(__double2hiint(d[0]), p & 63);
+                    lo = __builtin_amdgcn_readlane(__double2loint(d[0]), p & 63);
+                }
+                const double v = __hiloint2double(hi, lo);
+                // (a NaN goes on, into the results)
+                if (jj >= steps || __builtin_amdgcn_readfirstlane(v <= nfloor)) {
+                    stop = jj;
                     continue;
                 }
-                unsigned key = 0;
-#pragma unroll
-                for (int q = 0; q < ROWS; ++q) {
-                    const float s = fmaxf((float)ldexp(d[q], -e2), 0.0f);
-                    constexpr unsigned LOW = (1u << L::BITS) - 1;
-                    const unsigned kq = (__float_as_uint(s) & ~LOW) | (LOW - (unsigned)(lane + 64 * q));
-                    key = left[q] && kq > key ? kq : key;
-                }
-                key = wave_max_u32(key);
-                constexpr unsigned LOW = (1u << L::BITS) - 1;
-                const int p = (int)(LOW - (key & LOW));
-                const double v = key == 0 ? 0.0
-                                          : (ROWS > 1 && p >= 64 ? readlane_f64(d[ROWS - 1], p - 64)
-                                                                 : readlane_f64(d[0], p & 63));
-                j = 16 * pb + jj;
-                if (j >= n || !(v > nfloor && dmax > 0.0)) {
-                    more = false;
-                    if (lane == 0 && j < n) *rank_ = j;
-#pragma unroll
-                    for (int q = 0; q < ROWS; ++q) {
-                        lr[q][jj] = 0.0;
-                        if (lane + 64 * q < N) X[(lane + 64 * q) * LT + 16 * pb + jj] = 0.0;
-                    }
-                    continue;
-                }
-                const double rs = rsqrt_refined(v);
+                const double* ap = A + p * LD;
+                const double* xp = X + p * LD + 16 * pb;
                 double c[ROWS], lp[16];
 #pragma unroll
-                for (int q = 0; q < ROWS; ++q) c[q] = A[min(lane + 64 * q, N - 1) + p * LD];
+                for (int q = 0; q < ROWS; ++q) c[q] = ap[min(lane + 64 * q, N - 1)];
 #pragma unroll
-                for (int k = 0; k < jj; ++k) lp[k] = X[p * LT + 16 * pb + k];
+                for (int k = 0; k < jj; ++k) lp[k] = xp[k];
+                const double rs = rsqrt_refined(v);
+                pv = lane == jj ? p : pv;
+                vh = lane == jj ? hi : vh;
+                vl = lane == jj ? lo : vl;
 #pragma unroll
                 for (int q = 0; q < ROWS; ++q) {
+                    const int i = lane + 64 * q;
                     double c2 = 0.0;
 #pragma unroll
                     for (int k = 0; k < jj; ++k) {
                         if (k & 1) c2 = fma(-lr[q][k], lp[k], c2);
                         else c[q] = fma(-lr[q][k], lp[k], c[q]);
                     }
-                    const int i = lane + 64 * q;
-                    double l = (c[q] + c2) * rs;
-                    l = i == p ? v * rs : l;
-                    l = left[q] ? l : 0.0;
+                    const double l = (c[q] + c2) * rs;
                     lr[q][jj] = l;
-                    d[q] = fma(-l, l, d[q]);
-                    left[q] = left[q] && i != p;
-                    if (i < N) X[i * LT + j] = l;
-                }
-                if (lane == 0) {
-                    perm[j] = p;
-                    iperm[p] = j;
-                    rdiag[j] = v * rs;
-                    rinv[j] = rs;
+                    d[q] = i == p ? -1.0 : fma(-l, l, d[q]);
+                    if (i < N) X[i * LD + 16 * pb + jj] = l;
                 }
                 wave_order();
             }
+            if (lane < stop) {
+                perm[16 * pb + lane] = pv;
+                piv[16 * pb + lane] = __hiloint2double(vh, vl);
+            }
+            if (stop < steps && lane == 0) *rank_ = 16 * pb + stop;
+            // no step: no column
+#pragma unroll
+            for (int q = 0; q < ROWS; ++q)
+                for (int jj = stop; jj < 16; ++jj)
+                    if (lane + 64 * q < N) X[(lane + 64 * q) * LD + 16 * pb + jj] = 0.0;
         }
         __syncthreads();
-        if (*rank_ < min(n, 16 * (pb + 1))) break;   // (the same for every thread)
-        if (pb + 1 < T) {
-            for (int u = w; u < T * (T + 1) / 2; u += L::WAVES) {
-                int J = 0;
-                while ((J + 1) * (J + 2) / 2 <= u) ++J;
-                const int I = u - J * (J + 1) / 2;
-                dbl4 c;
-                double* at = A + 16 * I + l1 + (16 * J + l0) * LD;
+        if (*rank_ < min(n, 16 * (pb + 1)) || pb + 1 == T) break;   // (the same for every thread)
+        for (int u = w; u < T * (T + 1) / 2; u += L::WAVES) {
+            int J = 0;
+            while ((J + 1) * (J + 2) / 2 <= u) ++J;
+            const int I = u - J * (J + 1) / 2;
+            dbl4 c;
+            double* at = A + 16 * I + l1 + (16 * J + l0) * LD;
 #pragma unroll
-                for (int q = 0; q < 4; ++q) c[q] = at[4 * q];
+            for (int q = 0; q < 4; ++q) c[q] = at[4 * q];
 #pragma unroll
-                for (int kk = 0; kk < 4; ++kk)
-                    c = __builtin_amdgcn_mfma_f64_16x16x4f64(-X[(16 * I + l0) * LT + 16 * pb + 4 * kk + l1],
-                                                             X[(16 * J + l0) * LT + 16 * pb + 4 * kk + l1], c,
-                                                             0, 0, 0);
-                double* ta = A + 16 * J + l0 + (16 * I + l1) * LD;
+            for (int kk = 0; kk < 4; ++kk)
+                c = __builtin_amdgcn_mfma_f64_16x16x4f64(-X[(16 * I + l0) * LD + 16 * pb + 4 * kk + l1],
+                                                         X[(16 * J + l0) * LD + 16 * pb + 4 * kk + l1], c, 0,
+                                                         0, 0);
+            double* ta = A + 16 * J + l0 + (16 * I + l1) * LD;
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    at[4 * q] = c[q];
-                    if (I != J) ta[4 * q * LD] = c[q];
-                }
+            for (int q = 0; q < 4; ++q) {
+                at[4 * q] = c[q];
+                if (I != J) ta[4 * q * LD] = c[q];
             }
-            __syncthreads();
         }
+        __syncthreads();
     }
     const int rank = *rank_;
     // R in pivot order: R[i + k LD] = R[i][k] for i <= k < rank, else 1 / 0
     // (in A's place)
-    for (int e = t; e < m * m; e += NT) {
-        const int c = e / m, r = e - c * m;
-        A[r + c * LD] = c < rank && r <= c ? X[perm[c] * LT + r] : (r == c ? 1.0 : 0.0);
+#pragma unroll 4
+    for (int e = t; e < m * N; e += NT) {
+        const int c = e / N, r = e - c * N;
+        const double v = X[(c < rank ? perm[c] : 0) * LD + r];
+        A[r + c * LD] = c < rank && r <= c ? v : (r == c ? 1.0 : 0.0);
+    }
+    if (t < N) {
+        const double rs = t < rank ? rsqrt_refined(piv[t]) : 1.0;
+        rinv[t] = rs;
+        piv[t] = t < rank ? piv[t] * rs : 0.0;
+        if (t < rank) iperm[perm[t]] = t;
     }
     __syncthreads();
     // diagonal blocks of X = R^{-1}, four a wave: lane = (block, column)
@@ -2024,7 +2012,7 @@ __global__ __launch_bounds__(64 * CholLds<N>::WAVES) void k_cholqr(const JacobiD
         if (r < n)
             D.W[r + (int64_t)c * D.ldw] = ip >= 0 && ip <= c && c < rank ? X[ip + c * LD] : 0.0;
     }
-    if (t < n) D.lam[t] = t < rank ? rdiag[t] : 0.0;
+    if (t < n) D.lam[t] = piv[t];
     if (t == 0 && D.sweeps) *D.sweeps = 0;
 }
 
