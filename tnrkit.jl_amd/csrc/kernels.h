@@ -174,6 +174,14 @@ struct ConvDesc {
     int32_t whole_ok;             // a stall is refactorised whole: give up early
 };
 
+// stall_from > 0: from that iteration on, a problem with whole_ok set stops
+// (unconverged) once prod * r^(2 (max_iters - it)) >= target, i.e. even at twice
+// its current rate it could not reach the target in the iterations left
+struct ConvRule {
+    double null_rtol = 0.0, target = 0.0;
+    int32_t min_iters = 0, max_iters = 0, stall_from = 0;
+};
+
 // Deterministic uniform(-1,1) fill of a rows x cols column-major matrix.
 struct FillDesc {
     double* p;
@@ -223,18 +231,15 @@ void launch_trace_normalize(hipStream_t st, const TraceDesc* d_descs, const Trac
                             int nprob, int64_t max_size);
 size_t jacobi_lds_bytes(int n);
 // pivoted Cholesky QR of Gram matrices (JacobiDesc: G in, W = P R^{-1} out,
-// lam = R_jj); columns below null_rel2 * max diag are dropped
+// lam = R_jj); columns below null_rel2 * max diag are dropped.  With d_conv
+// the stopping rule follows, on each problem's R_jj.
 void launch_cholqr(hipStream_t st, const JacobiDesc* d_descs, int nd, int nmin, int nmax,
-                   double null_rel2);
+                   double null_rel2, const ConvDesc* d_conv = nullptr, const ConvRule& rule = ConvRule());
 void launch_jacobi(hipStream_t st, const JacobiDesc* d_descs, int nd, int nmax, double tol,
                    int max_sweeps);
 void launch_colnorm(hipStream_t st, const ColDesc* d_descs, int nd, int ncol_max, double rtol);
 void launch_symmetrize(hipStream_t st, const ColDesc* d_descs, int nd, int nmax);
-// stall_from > 0: from that iteration on, a problem with whole_ok set stops
-// (unconverged) once prod * r^(2 (max_iters - it)) >= target, i.e. even at twice
-// its current rate it could not reach the target in the iterations left
-void launch_conv(hipStream_t st, const ConvDesc* d_descs, int nd, double null_rtol, double target,
-                 int min_iters, int max_iters, int stall_from);
+void launch_conv(hipStream_t st, const ConvDesc* d_descs, int nd, const ConvRule& rule);
 // sigma[0] of each descriptor = squared Frobenius norm of its nrow x ncol
 // matrix Y (ld ldy), summed in a fixed order over FROB_PARTS column ranges;
 // partial: nd * FROB_PARTS doubles of scratch

@@ -1757,6 +1757,41 @@ __global__ __launch_bounds__(JAC_TMAX) void k_jacobi(const JacobiDesc* __restric
     else jacobi_body<JM, 3>(D, lds, tol, max_sweeps, polish);
 }
 
+// ------------------------------------------------ stopping rule
+// Stopping rule of the block iteration by one wave, after an iteration whose
+// l values (largest first) are in sv: the contraction of the top-k subspace,
+// (sv_l / sv_k)^2 (or ^1), is accumulated from iteration min_iters on, and the
+// problem is done below the target or at max_iters; one that will be
+// factorised whole anyway stops once even twice its current rate could not
+// reach the target in the iterations left.
+__device__ __forceinline__ void conv_step(const ConvDesc& D, const double* sv, const ConvRule& rule,
+                                          int lane) {
+    // the last of the k wanted values above the null threshold
+    int kk = 0;
+    const double top = sv[0];
+    for (int i0 = 0; i0 < D.kmax; i0 += 64) {
+        const int i = i0 + lane;
+        const unsigned long long b = __ballot(i < D.kmax && sv[min(i, D.kmax - 1)] > rule.null_rtol * top);
+        if (b) kk = i0 + 64 - __clzll((long long)b);
+    }
+    if (lane != 0) return;
+    const int it = *D.it + 1;
+    double r = 0.0;
+    if (kk > 0 && sv[kk - 1] > 0.0) {
+        r = sv[D.l - 1] / sv[kk - 1];
+        if (D.squared) r *= r;
+        r = fmin(r, 1.0);
+    }
+    double prod = *D.prod;
+    if (it >= rule.min_iters) prod *= r;
+    *D.it = it;
+    *D.prod = prod;
+    if ((it >= rule.min_iters && prod < rule.target) || it >= rule.max_iters) *D.done = 1;
+    else if (D.whole_ok && rule.stall_from > 0 && it >= rule.stall_from && it >= rule.min_iters &&
+             prod * pow(r, 2.0 * (rule.max_iters - it)) >= rule.target)
+        *D.done = 1;
+}
+
 // ------------------------------------------------ pivoted Cholesky QR
 // One workgroup per n x n Gram matrix G = Y^T Y (n <= LMAX):
 // diagonal-pivoted Cholesky G[p, p] = R^T R, stopped where the largest
@@ -1816,7 +1851,9 @@ __device__ __forceinline__ int wave_max_i32(int x) {
 
 template <int N>
 __global__ __launch_bounds__(64 * CholLds<N>::WAVES) void k_cholqr(const JacobiDesc* __restrict__ descs,
-                                                                  int nd, double null_rel2) {
+                                                                  int nd, double null_rel2,
+                                                                  const ConvDesc* __restrict__ conv,
+                                                                  ConvRule rule) {
     using L = CholLds<N>;
     constexpr int LD = L::LD, ROWS = L::ROWS, NT = 64 * L::WAVES;
     extern __shared__ double lds[];
@@ -2014,6 +2051,8 @@ __global__ __launch_bounds__(64 * CholLds<N>::WAVES) void k_cholqr(const JacobiD
     }
     if (t < n) D.lam[t] = piv[t];
     if (t == 0 && D.sweeps) *D.sweeps = 0;
+    // (a problem that is done needs no product with W any more)
+    if (conv && w == 0) conv_step(conv[blockIdx.x], piv, rule, lane);
 }
 
 // ------------------------------------------------- column norms / normalise
@@ -2531,34 +2570,12 @@ __global__ __launch_bounds__(EIGT) void k_eig_hqr_g(const EigDesc* __restrict__ 
     eig_hqr_body(D, D.work);
 }
 
-// stopping rule of the block iteration, one thread per problem
-__global__ void k_conv(const ConvDesc* __restrict__ descs, int nd, double null_rtol,
-                       double target, int min_iters, int max_iters, int stall_from) {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= nd) return;
-    const ConvDesc D = descs[p];
+// conv_step for values that another kernel wrote (the eigensolver's Ritz
+// values), one wave per problem.
+__global__ __launch_bounds__(64) void k_conv(const ConvDesc* __restrict__ descs, int nd, ConvRule rule) {
+    const ConvDesc D = descs[blockIdx.x];
     if (*D.done) return;
-    const int it = *D.it + 1;
-    const double* sv = D.sigma;
-    int kk = 0;
-    for (int i = 0; i < D.kmax; ++i)
-        if (sv[i] > null_rtol * sv[0]) kk = i + 1;
-    double r = 0.0;
-    if (kk > 0 && sv[kk - 1] > 0.0) {
-        r = sv[D.l - 1] / sv[kk - 1];
-        if (D.squared) r *= r;
-        r = fmin(r, 1.0);
-    }
-    double prod = *D.prod;
-    if (it >= min_iters) prod *= r;
-    *D.it = it;
-    *D.prod = prod;
-    if ((it >= min_iters && prod < target) || it >= max_iters) *D.done = 1;
-    // a stall that will be factorised whole anyway: stop iterating once even
-    // twice the current rate could not reach the target in the iterations left
-    else if (D.whole_ok && stall_from > 0 && it >= stall_from && it >= min_iters &&
-             prod * pow(r, 2.0 * (max_iters - it)) >= target)
-        *D.done = 1;
+    conv_step(D, D.sigma, rule, threadIdx.x);
 }
 
 // in-place (M + M^T)/2 of square blocks (project_hermitian)
@@ -3004,21 +3021,22 @@ void launch_jacobi(hipStream_t st, const JacobiDesc* d_descs, int nd, int nmax, 
 // k_cholqr<LMAX> (each kernel skips the other's), so the kernel a problem gets
 // depends on its own size only, never on the rest of its launch group.
 template <int N>
-static void launch_cholqr_n(hipStream_t st, const JacobiDesc* d_descs, int nd, double null_rel2) {
+static void launch_cholqr_n(hipStream_t st, const JacobiDesc* d_descs, int nd, double null_rel2,
+                            const ConvDesc* d_conv, const ConvRule& rule) {
     static const hipError_t attr = hipFuncSetAttribute(
         (const void*)k_cholqr<N>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)CholLds<N>::BYTES);
     TNR_HIP(attr);
     ProfScope ps(st, PK_JACOBI, 0.0, 0.0);
     TNR_LAUNCH(ps, k_cholqr<N>, dim3(nd), dim3(64 * CholLds<N>::WAVES), CholLds<N>::BYTES, st, d_descs, nd,
-               null_rel2);
+               null_rel2, d_conv, rule);
     TNR_HIP(hipGetLastError());
 }
 
 void launch_cholqr(hipStream_t st, const JacobiDesc* d_descs, int nd, int nmin, int nmax,
-                   double null_rel2) {
+                   double null_rel2, const ConvDesc* d_conv, const ConvRule& rule) {
     if (nd <= 0) return;
-    if (nmin <= CQ64) launch_cholqr_n<CQ64>(st, d_descs, nd, null_rel2);
-    if (nmax > CQ64) launch_cholqr_n<LMAX>(st, d_descs, nd, null_rel2);
+    if (nmin <= CQ64) launch_cholqr_n<CQ64>(st, d_descs, nd, null_rel2, d_conv, rule);
+    if (nmax > CQ64) launch_cholqr_n<LMAX>(st, d_descs, nd, null_rel2, d_conv, rule);
 }
 
 void launch_lincomb(hipStream_t st, const LinDesc* d_descs, int nd, int64_t total) {
@@ -3096,12 +3114,10 @@ void launch_symmetrize(hipStream_t st, const ColDesc* d_descs, int nd, int nmax)
     TNR_HIP(hipGetLastError());
 }
 
-void launch_conv(hipStream_t st, const ConvDesc* d_descs, int nd, double null_rtol, double target,
-                 int min_iters, int max_iters, int stall_from) {
+void launch_conv(hipStream_t st, const ConvDesc* d_descs, int nd, const ConvRule& rule) {
     if (nd <= 0) return;
     ProfScope ps(st, PK_MISC, 0.0, 0.0);
-    TNR_LAUNCH(ps, k_conv, dim3((nd + 63) / 64), dim3(64), 0, st, d_descs, nd, null_rtol, target,
-                       min_iters, max_iters, stall_from);
+    TNR_LAUNCH(ps, k_conv, dim3(nd), dim3(64), 0, st, d_descs, nd, rule);
     TNR_HIP(hipGetLastError());
 }
 

@@ -81,6 +81,10 @@ void set_solver_cfg(const char* spec) {
 
 namespace {
 
+ConvRule conv_rule(const SolverCfg& cfg) {
+    return ConvRule{cfg.null_rtol, cfg.conv_target, cfg.min_iters, cfg.max_iters, cfg.stall_from};
+}
+
 // One Gram/Jacobi Rayleigh-Ritz job: rotates the columns of Y (rows x l) to
 // the Ritz basis of span(Y), normalises them into U and writes the column
 // norms to sigma.  Wtot (optional) receives the total rotation.
@@ -142,7 +146,9 @@ RRPlan rr_plan(Ctx& ctx, const std::vector<RR>& jobs, int passes, bool chol = fa
             GemmJob g{Y, Y, j.G, j.l, j.l, j.rows, ld, ld, j.l, 1, 0};   // G = Y^T Y
             g.skip = j.skip;
             gj.push_back(g);
-            GemmJob r = pass == 0
+            // Cholesky QR: the rotated columns are the orthonormal basis itself
+            GemmJob r = chol ? GemmJob{j.Y, W1, j.U, j.rows, j.l, j.l, j.ldy, j.l, j.ldu, 0, 0}
+                        : pass == 0
                             ? GemmJob{j.Y, W1, j.Y2, j.rows, j.l, j.l, j.ldy, j.l, j.rows, 0, 0}
                             : GemmJob{j.Y2, j.W2, j.Y, j.rows, j.l, j.l, j.rows, j.l, j.ldy, 0, 0};
             r.skip = j.skip;
@@ -159,9 +165,11 @@ RRPlan rr_plan(Ctx& ctx, const std::vector<RR>& jobs, int passes, bool chol = fa
         P.rot[pass] = gemm_plan(ctx, rj);
     }
     // rotated columns: Y2 after one pass, Y after two
-    for (auto& j : jobs)
-        P.col.push_back(passes == 1 ? ColDesc{j.Y2, j.U, j.sigma, j.rows, j.l, j.rows, j.ldu, j.skip}
-                                    : ColDesc{j.Y, j.U, j.sigma, j.rows, j.l, j.ldy, j.ldu, j.skip});
+    if (!chol)
+        for (auto& j : jobs)
+            P.col.push_back(passes == 1
+                                ? ColDesc{j.Y2, j.U, j.sigma, j.rows, j.l, j.rows, j.ldu, j.skip}
+                                : ColDesc{j.Y, j.U, j.sigma, j.rows, j.l, j.ldy, j.ldu, j.skip});
     return P;
 }
 
@@ -185,14 +193,15 @@ void rr_bind(RRPlan& P, const DescArena& a) {
 
 // `first`: the block iteration's first step, whose Rayleigh-Ritz step only
 // has to align a random basis roughly (jacobi_tol_first)
-void rr_issue(Ctx& ctx, RRPlan& P, bool first = false) {
+// `conv` (Cholesky QR only): the stopping rule, one descriptor per job
+void rr_issue(Ctx& ctx, RRPlan& P, bool first = false, const ConvDesc* conv = nullptr) {
     const SolverCfg& cfg = solver_cfg();
     for (int pass = 0; pass < P.passes; ++pass) {
         gemm_issue(ctx, P.gram[pass]);
         const bool in_loop = P.passes == 1 && !P.tight;
         if (P.chol)
             launch_cholqr(ctx.stream, P.d_jac[pass], (int)P.jac[pass].size(), P.lmin, P.lmax,
-                          cfg.null_rtol * cfg.null_rtol);
+                          cfg.null_rtol * cfg.null_rtol, conv, conv_rule(cfg));
         else
             launch_jacobi(ctx.stream, P.d_jac[pass], (int)P.jac[pass].size(), P.lmax,
                           !in_loop ? cfg.jacobi_tol
@@ -200,7 +209,7 @@ void rr_issue(Ctx& ctx, RRPlan& P, bool first = false) {
                           in_loop ? cfg.jacobi_sweeps_iter : cfg.jacobi_sweeps);
         gemm_issue(ctx, P.rot[pass]);
     }
-    launch_colnorm(ctx.stream, P.d_col, (int)P.col.size(), P.lmax, cfg.null_rtol);
+    if (!P.chol) launch_colnorm(ctx.stream, P.d_col, (int)P.col.size(), P.lmax, cfg.null_rtol);
 }
 
 void rr_grouped(Ctx& ctx, const std::vector<RR>& jobs, int passes, bool tight = false) {
@@ -931,9 +940,8 @@ void svd_grouped(Ctx& ctx, const std::vector<SvdIn>& in, std::vector<SvdOut>& ou
             gemm_issue(ctx, pMV);
             rr_issue(ctx, pY, it == 0);
             gemm_issue(ctx, pMtU);
-            rr_issue(ctx, pZ, it == 0);
-            launch_conv(ctx.stream, d_conv, P, cfg.null_rtol, cfg.conv_target, cfg.min_iters,
-                        cfg.max_iters, cfg.stall_from);
+            rr_issue(ctx, pZ, it == 0, cfg.cholqr_z ? d_conv : nullptr);
+            if (!cfg.cholqr_z) launch_conv(ctx.stream, d_conv, P, conv_rule(cfg));
         });
         // the loop orthonormalises only to its looser Jacobi threshold: V is
         // rebuilt at full accuracy before the final extraction relies on
@@ -1096,8 +1104,7 @@ void eigh_grouped(Ctx& ctx, const std::vector<EighIn>& in, std::vector<EighOut>&
         iterate(ctx, cs, [&](int it) {
             gemm_issue(ctx, pMV);
             rr_issue(ctx, pY, it == 0);
-            launch_conv(ctx.stream, d_conv, P, cfg.null_rtol, cfg.conv_target, cfg.min_iters,
-                        cfg.max_iters, cfg.stall_from);
+            launch_conv(ctx.stream, d_conv, P, conv_rule(cfg));
         });
         // V at full orthonormality from the loop's last rotated Y = M V W
         // (the loop uses a looser Jacobi threshold; one pass at the final
