@@ -123,6 +123,25 @@ def test_gemm_lds_dma_matches_register_loads_bitwise(tk, M, N, K, ta, tb, pad):
             assert np.max(np.abs(dma - ref)) <= 1e-14 * (np.sqrt(K) + 1) * 8
 
 
+# sizes on both sides of the small launches' rule: 16 x 16 tiles on one wave
+# (one K chunk), 16 x 16 and 32 x 32 tiles with the K chunks over four waves
+# (fewer, as many and more chunks than waves), and the first sizes past them
+@pytest.mark.parametrize("M,N,K,ta,tb,pad", [
+    (1, 1, 1, 0, 0, 0), (15, 17, 3, 1, 0, 1), (33, 16, 31, 0, 1, 2), (512, 384, 64, 0, 0, 0),
+    (528, 384, 64, 0, 1, 0), (100, 37, 511, 1, 1, 3), (64, 64, 512, 1, 0, 0), (48, 80, 600, 0, 0, 1),
+    (96, 96, 1025, 1, 0, 0), (70, 33, 2047, 0, 1, 5), (300, 130, 2049, 1, 1, 0), (512, 384, 512, 0, 1, 0), (528, 384, 513, 0, 0, 0),
+    (600, 1000, 700, 1, 0, 2), (1024, 1040, 520, 0, 0, 0), (32, 48, 300, 0, 0, 0)])
+def test_gemm_small_launches_match_the_tiles_bitwise(tk, M, N, K, ta, tb, pad):
+    rng = np.random.default_rng(7 * M + N + K)
+    A = rng.standard_normal((K, M) if ta else (M, K))
+    B = rng.standard_normal((N, K) if tb else (K, N))
+    Cm = rng.standard_normal((M, N))
+    ref = (A.T if ta else A) @ (B.T if tb else B) + 0.5 * Cm
+    auto = gemm_padded(tk, A, B, Cm, ta, tb, pad, 0)
+    assert np.array_equal(auto, gemm_padded(tk, A, B, Cm, ta, tb, pad, 2 | 8))
+    assert np.max(np.abs(auto - ref)) <= 1e-14 * (np.sqrt(K) + 1) * 8
+
+
 @pytest.mark.parametrize("M,N,K", [(128, 128, 256), (200, 100, 1000)])
 def test_gemm_split32(tk, M, N, K):
     rng = np.random.default_rng(K)

@@ -361,6 +361,29 @@ static int pick_shape(const std::vector<GemmJob>& jobs, bool split32) {
     return GEMM_64x64;
 }
 
+// Launches too small for 64 x 64 tiles to fill the chip: the kernel that
+// shares the K chunks of a small tile over one workgroup's waves, or -1.  One
+// wave's chain over 256 k is ~3 us on a 16 x 16 tile and ~7 us on 32 x 32, so
+// the smaller tile is taken while its workgroups (two a CU by LDS) run in one
+// or two rounds; past 32 x 32 tiles on every CU four times over, 64 x 64
+// tiles read the operands less often.  Measured (ms a run; limits none / 256,
+// 512 / 512, 512 / 768, 1024): BTRG chi 32 29.5 / 24.6 / 23.5 / 23.2, BTRG Z2
+// chi 64 78.3 / 76.5 / 76.6 / 71.4, HOTRG chi 32 64.0 / 60.8 / 59.8 / 59.2; a
+// first limit of 1024 catches a quarter of a 128-run batch's Gram matrices
+// and costs it 2.5 % (331 -> 339 ms).
+static int pick_small(const std::vector<GemmJob>& jobs) {
+    constexpr int64_t kMost16 = 768, kMost32 = 1024;
+    int64_t t16 = 0, t32 = 0;
+    int chunks = 1;
+    for (const GemmJob& j : jobs) {
+        if (j.M <= 0 || j.N <= 0) continue;
+        t16 += (int64_t)((j.M + 15) / 16) * ((j.N + 15) / 16);
+        t32 += (int64_t)((j.M + 31) / 32) * ((j.N + 31) / 32);
+        chunks = std::max(chunks, nchunks_of(j.K));
+    }
+    if (t16 <= kMost16) return chunks == 1 ? GEMM_KW16x1 : GEMM_KW16x4;
+    return chunks > 1 && t32 <= kMost32 ? GEMM_KW32x4 : -1;
+}
 
 // ------------------------------------------------------ tile-shape autotuner
 // Every output element is summed in the same order under each tile shape,
@@ -520,7 +543,11 @@ GemmPlan gemm_plan(Ctx& ctx, const std::vector<GemmJob>& jobs, bool split32, int
         if (j.M > 0 && j.N > 0) dma_ok = dma_ok && gemm_dma_ok(j.ta, j.lda, j.tb, j.ldb);
     if (force_shape >= 0 && !split32) P.shape = force_shape;
     else if (split32) P.shape = GEMM_64x64;
-    else P.shape = tuned_shape(ctx, jobs, pick_shape(jobs, false), dma_ok, &P.tune_key, &P.trial);
+    else {
+        const int small = dma_ok && force_split < 0 ? pick_small(jobs) : -1;
+        P.shape = small >= 0 ? small
+                             : tuned_shape(ctx, jobs, pick_shape(jobs, false), dma_ok, &P.tune_key, &P.trial);
+    }
     const int BMs = gemm_shape_bm(P.shape), BNs = gemm_shape_bn(P.shape);
     // split K over workgroups only when the launch is too small to fill
     // the chip without it (results are the same either way)
@@ -528,7 +555,7 @@ GemmPlan gemm_plan(Ctx& ctx, const std::vector<GemmJob>& jobs, bool split32, int
     for (const GemmJob& j : jobs)
         if (j.M > 0 && j.N > 0)
             whole += (int64_t)((j.M + BMs - 1) / BMs) * ((j.N + BNs - 1) / BNs);
-    const bool split = force_split >= 0 ? force_split != 0 : whole < 512;
+    const bool split = gemm_shape_kw(P.shape) ? false : force_split >= 0 ? force_split != 0 : whole < 512;
     size_t work_elems = 0;
     P.descs.reserve(jobs.size());
     for (const GemmJob& j : jobs) {

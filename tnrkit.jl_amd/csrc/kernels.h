@@ -210,10 +210,23 @@ void launch_transpose(hipStream_t st, const TransDesc* d_descs, int nd, int64_t 
 //   GEMM_128x64     128x64,  8 waves of 32x32, k 16 (LDS-DMA, 3 stages)
 //   GEMM_128x128   128x128,  8 waves of 32x64, k 16 (LDS-DMA, 3 stages)
 //   GEMM_64x64_K32   64x64,  4 waves of 32x32, k 32 (register-staged loads)
-enum GemmShape { GEMM_64x64 = 0, GEMM_128x64 = 1, GEMM_128x128 = 2, GEMM_64x64_K32 = 3 };
+//   GEMM_KW16x1      16x16 for one wave            (small launches, one K chunk)
+//   GEMM_KW16x4      16x16, K chunks over 4 waves  (small launches)
+//   GEMM_KW32x4      32x32, K chunks over 4 waves  (small launches)
+// The first GEMM_NSHAPES are the autotuner's; the small launches' kernels
+// take every K chunk in one workgroup and need LDS-DMA.
+enum GemmShape {
+    GEMM_64x64 = 0, GEMM_128x64 = 1, GEMM_128x128 = 2, GEMM_64x64_K32 = 3,
+    GEMM_KW16x1 = 4, GEMM_KW16x4 = 5, GEMM_KW32x4 = 6
+};
 constexpr int GEMM_NSHAPES = 4;
-inline int gemm_shape_bm(int s) { return (s == GEMM_64x64 || s == GEMM_64x64_K32) ? 64 : 128; }
-inline int gemm_shape_bn(int s) { return s == GEMM_128x128 ? 128 : 64; }
+inline bool gemm_shape_kw(int s) { return s >= GEMM_KW16x1; }
+inline int gemm_shape_bm(int s) {
+    return s == GEMM_KW32x4 ? 32 : gemm_shape_kw(s) ? 16 : (s == GEMM_64x64 || s == GEMM_64x64_K32) ? 64 : 128;
+}
+inline int gemm_shape_bn(int s) {
+    return gemm_shape_kw(s) ? gemm_shape_bm(s) : s == GEMM_128x128 ? 128 : 64;
+}
 // dma: the 16-deep shapes load through LDS-DMA (k_gemm_dl, same bits); needs
 // every descriptor's per-tile offsets below 2^31 bytes (gemm_dma_ok)
 void launch_gemm(hipStream_t st, const GemmDesc* d_descs, int nd, int64_t tiles, bool split32,

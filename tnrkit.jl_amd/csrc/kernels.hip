@@ -760,6 +760,174 @@ void k_gemm_dl(const GemmDesc* __restrict__ descs, int nd, unsigned long long* f
                            (es == 0 ? S0 : es == 1 ? S1 : es == 2 ? S2 : S3) + (w / NS) * EP_REGION);
 }
 
+// ------------------------------------------------ FP64 MFMA, small launches
+// The same products for launches with too few tiles to fill the chip, where
+// the chain over K is the time: each wave of a workgroup takes K chunks w,
+// w + W, ... of the workgroup's own 16 MI x 16 MI tile, through its own ring
+// of NS LDS stages (so the k loop has no barrier), and the chunk sums are
+// added in order through LDS.  The sums are those of the other kernels with
+// K split or not, bit for bit, without their second launch and workspace.
+// Measured alone, copies and events included (64 x 64 tiles with K split and
+// its reduction launch -> here): 1024 x 64 x 1024 25.3 -> 15.3 us, 64 x 64 x
+// 1024 (a Gram matrix) 24.7 -> 14.4, 2048 x 96 x 2048 40.9 -> 36.4, 256 x 32 x
+// 256 (one chunk) 21.1 -> 14.2.
+template <int PER, int QA>
+__device__ __forceinline__ void kw_issue(double* stage, __amdgpu_buffer_rsrc_t ra, __amdgpu_buffer_rsrc_t rb,
+                                         const int* lbase, const int* vofs) {
+#pragma unroll
+    for (int r = 0; r < PER; ++r)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(r < QA ? ra : rb,
+                                                 (__attribute__((address_space(3))) void*)(stage + lbase[r]),
+                                                 16, vofs[r], 0, 0, 0);
+}
+
+template <int MI, int W, int NS>
+__global__ __launch_bounds__(64 * W) void k_gemm_kw(const GemmDesc* __restrict__ descs, int nd,
+                                                    unsigned long long* flop_ctr) {
+    constexpr int BM = 16 * MI, KB = 16, NT = 64 * W;
+    using P = DlPlan<BM, BM, 1, KB>;
+    static_assert(NS == 3 || NS == 4, "three or four LDS stages");
+    __shared__ __align__(16) double S0[W * P::ST];
+    __shared__ __align__(16) double S1[W * P::ST];
+    __shared__ __align__(16) double S2[W * P::ST];
+    __shared__ __align__(16) double S3[NS > 3 ? W * P::ST : 2];
+    const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
+    double* const SS[4] = {S0 + w * P::ST, S1 + w * P::ST, S2 + w * P::ST, NS > 3 ? S3 + w * P::ST : S3};
+    const GemmDesc g = descs[find_desc_gemm(descs, nd, blockIdx.x)];
+    if (g.skip && *g.skip) return;
+    const TileCoord tc = tile_coord<BM, BM>(g, (int64_t)blockIdx.x - g.tile_start);
+    count_tile_flops<BM, BM>(flop_ctr, g, tc);
+    if (flop_ctr) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    const bool arow = !g.ta, brow = g.tb != 0;
+    int lbase[P::PER], vofs[P::PER];
+#pragma unroll
+    for (int r = 0; r < P::PER; ++r) {
+        int base, i, kk0, kk1;
+        if (r < P::QA) {
+            dl_slot<KB>(arow, BM, r, lane, base, i, kk0, kk1);
+            lbase[r] = __builtin_amdgcn_readfirstlane(base);
+            vofs[r] = 8 * (arow ? i + kk0 * g.lda : kk0 + i * g.lda);
+        } else {
+            dl_slot<KB>(brow, BM, r - P::QA, lane, base, i, kk0, kk1);
+            lbase[r] = __builtin_amdgcn_readfirstlane(P::SA + base);
+            vofs[r] = 8 * (brow ? i + kk0 * g.ldb : kk0 + i * g.ldb);
+        }
+    }
+    const int64_t extA = arow ? (int64_t)g.lda * (g.K - 1) + g.M : (int64_t)g.lda * (g.M - 1) + g.K;
+    const int64_t extB = brow ? (int64_t)g.ldb * (g.K - 1) + g.N : (int64_t)g.ldb * (g.N - 1) + g.K;
+    auto rsrc_a = [&](int k0) {
+        const int64_t o = arow ? (int64_t)tc.m0 + (int64_t)k0 * g.lda : (int64_t)k0 + (int64_t)tc.m0 * g.lda;
+        return dl_rsrc(g.A + o, extA - o);
+    };
+    auto rsrc_b = [&](int k0) {
+        const int64_t o = brow ? (int64_t)tc.n0 + (int64_t)k0 * g.ldb : (int64_t)k0 + (int64_t)tc.n0 * g.ldb;
+        return dl_rsrc(g.B + o, extB - o);
+    };
+    auto issue = [&](double* stage, int k0) { kw_issue<P::PER, P::QA>(stage, rsrc_a(k0), rsrc_b(k0), lbase, vofs); };
+    int aoff[KB / 4], boff[KB / 4];
+#pragma unroll
+    for (int ks = 0; ks < KB / 4; ++ks) {
+        const int kk = ks * 4 + (lane >> 4);
+        aoff[ks] = dl_off<KB>(arow, BM, lane & 15, kk);
+        boff[ks] = P::SA + dl_off<KB>(brow, BM, lane & 15, kk);
+    }
+    const int astep = arow ? 16 : 16 * KB, bstep = brow ? 16 : 16 * KB;
+    const int chunks = max(1, (g.K + g.kchunk - 1) / g.kchunk);
+    // this thread's elements of the tile
+    constexpr int E = BM * BM / NT;
+    double sum[E];
+#pragma unroll
+    for (int i = 0; i < E; ++i) sum[i] = 0.0;
+    for (int c0 = 0; c0 < chunks; c0 += W) {
+        const int kbeg = (c0 + w) * g.kchunk, kend = min(g.K, kbeg + g.kchunk);
+        const int nt = kend > kbeg ? (kend - kbeg + KB - 1) / KB : 0;
+        dbl4 acc[MI][MI];
+#pragma unroll
+        for (int mi = 0; mi < MI; ++mi)
+#pragma unroll
+            for (int ni = 0; ni < MI; ++ni) acc[mi][ni] = dbl4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int s = 0; s < NS - 1; ++s)
+            if (s < nt) issue(SS[s], kbeg + s * KB);
+        // one k-tile: wait for the loads of tile it, zero k >= K on the last
+        // tile, issue tile it + NS - 1 into the stage whose reads were
+        // consumed one tile ago, multiply
+        auto step = [&](double* cur, double* nxt, int it) {
+            const int k0 = kbeg + it * KB;
+            const int ahead = min(NS - 2, nt - 1 - it);   // tiles issued after this one
+            if (NS > 3 && ahead >= 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * P::PER) : "memory");
+            else if (ahead >= 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(P::PER) : "memory");
+            else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            if (k0 + KB > g.K) {
+                const int kv = g.K - k0;
+#pragma unroll
+                for (int r = 0; r < P::PER; ++r) {
+                    int base, i, kk0, kk1;
+                    if (r < P::QA) dl_slot<KB>(arow, BM, r, lane, base, i, kk0, kk1);
+                    else dl_slot<KB>(brow, BM, r - P::QA, lane, base, i, kk0, kk1);
+                    double* d = cur + lbase[r] + 2 * lane;
+                    if (kk0 >= kv) d[0] = 0.0;
+                    if (kk1 >= kv) d[1] = 0.0;
+                }
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            if (it + NS - 1 < nt) issue(nxt, k0 + (NS - 1) * KB);
+            __builtin_amdgcn_sched_barrier(0);
+            double a[KB / 4][MI], b[KB / 4][MI];
+#pragma unroll
+            for (int ks = 0; ks < KB / 4; ++ks)
+#pragma unroll
+                for (int mi = 0; mi < MI; ++mi) {
+                    a[ks][mi] = cur[aoff[ks] + mi * astep];
+                    b[ks][mi] = cur[boff[ks] + mi * bstep];
+                }
+#pragma unroll
+            for (int ks = 0; ks < KB / 4; ++ks)
+#pragma unroll
+                for (int mi = 0; mi < MI; ++mi)
+#pragma unroll
+                    for (int ni = 0; ni < MI; ++ni)
+                        acc[mi][ni] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[ks][mi], b[ks][ni], acc[mi][ni], 0,
+                                                                           0, 0);
+            // the stage's reads are complete (consumed) before the next
+            // step's DMA may overwrite it
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        for (int it = 0; it < nt; it += NS) {
+#pragma unroll
+            for (int s = 0; s < NS; ++s)
+                if (it + s < nt) step(SS[s], SS[(s + NS - 1) % NS], it + s);
+        }
+        // (every load of this wave's stages has landed and been consumed)
+        static_assert(BM * (BM + 1) <= P::ST, "the chunk sums fit a stage");
+        double* pw = S0 + w * P::ST;
+#pragma unroll
+        for (int mi = 0; mi < MI; ++mi)
+#pragma unroll
+            for (int ni = 0; ni < MI; ++ni)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    pw[16 * mi + (lane >> 4) + 4 * r + (16 * ni + (lane & 15)) * (BM + 1)] = acc[mi][ni][r];
+        __syncthreads();
+        const int here = min(W, chunks - c0);
+#pragma unroll
+        for (int i = 0; i < E; ++i) {
+            const int e = t + NT * i, at = e % BM + (e / BM) * (BM + 1);
+            for (int z = 0; z < here; ++z) sum[i] += S0[z * P::ST + at];
+        }
+        __syncthreads();
+    }
+    gmut_double* C = as_global(g.C);
+#pragma unroll
+    for (int i = 0; i < E; ++i) {
+        const int e = t + NT * i, row = tc.m0 + e % BM, col = tc.n0 + e / BM;
+        if (row < g.M && col < g.N) {
+            gmut_double* p = C + (int64_t)row + (int64_t)col * g.ldc;
+            *p = (g.beta == 0.0) ? g.alpha * sum[i] : g.alpha * sum[i] + g.beta * *p;
+        }
+    }
+}
+
 // ------------------------------------------------ FP32 MFMA, hi/lo split
 // x = hi + lo with hi = fp32(x), lo = fp32(x - hi).  Per k-tile the three
 // significant products hi*hi, hi*lo, lo*hi are accumulated on FP32 MFMA
@@ -2933,6 +3101,12 @@ void launch_gemm(hipStream_t st, const GemmDesc* d_descs, int nd, int64_t tiles,
     unsigned long long* fc = ps.active ? prof_flop_counter(split32) : nullptr;
     if (split32)
         TNR_LAUNCH(ps, k_gemm_split32, dim3((unsigned)tiles), dim3(256), 0, st, d_descs, nd, fc);
+    else if (shape == GEMM_KW16x1)
+        TNR_LAUNCH(ps, (k_gemm_kw<1, 1, 4>), dim3((unsigned)tiles), dim3(64), 0, st, d_descs, nd, fc);
+    else if (shape == GEMM_KW16x4)
+        TNR_LAUNCH(ps, (k_gemm_kw<1, 4, 4>), dim3((unsigned)tiles), dim3(256), 0, st, d_descs, nd, fc);
+    else if (shape == GEMM_KW32x4)
+        TNR_LAUNCH(ps, (k_gemm_kw<2, 4, 4>), dim3((unsigned)tiles), dim3(256), 0, st, d_descs, nd, fc);
     else if (shape == GEMM_128x128 && dma)
         TNR_LAUNCH(ps, (k_gemm_dl<128, 128, 4, 2, 2, 3, 16>), dim3((unsigned)tiles), dim3(512), 0, st,
                            d_descs, nd, fc);
