@@ -307,6 +307,39 @@ def test_eigh_truncated(tk, n, k):
     assert np.max(np.abs(Pk - Pr)) < 1e-9
 
 
+# The block iteration's Cholesky QR has to keep every direction of a steep
+# spectrum: after the random start all columns are within 1e-8 of the leading
+# eigenvectors, below what their Gram matrix resolves.  Spectra: steep ones
+# (also so steep that the block's last values are roundoff), +- pairs, a gap of
+# nine decades inside and at the edge of the wanted values, low rank; block
+# widths on both sides of 64 and k + 2.  Roundoff of the products, n eps ~
+# 4e-14, and the rule's 1e-14 contraction of a start within 1e2 of the subspace
+# bound the residual by 1e-12 of the largest |lambda|.
+@pytest.mark.parametrize("k", [1, 8, 24, 33, 47])
+@pytest.mark.parametrize("spec", ["0.8", "0.5", "0.1", "pairs", "gap", "rank", "flat"])
+def test_eigh_cholesky_loop_keeps_every_direction(tk, spec, k):
+    n = 203
+    j = np.arange(n)
+    w = {"pairs": 0.6 ** (j // 2) * (-1.0) ** j, "gap": np.where(j < 10, 1.0, 1e-9) * 0.8 ** j,
+         "rank": np.where(j < 12, 0.5 ** j, 0.0),
+         "flat": np.where(j <= k, 1.0, 1e-3) * (1 + 0.1 * np.cos(j))}.get(spec)
+    if w is None:
+        w = float(spec) ** j
+    rng = np.random.default_rng(n + k)
+    Q, _ = np.linalg.qr(rng.standard_normal((n, n)))
+    M = (Q * w) @ Q.T
+    M = 0.5 * (M + M.T)
+    U = np.zeros((n, k), order="F"); lam = np.zeros(k); it = C.c_int()
+    st = tk.lib().tnr_kernel_eigh(n, p(np.asfortranarray(M)), k, p(U), p(lam), C.byref(it))
+    assert st == 0, tk.lib().tnr_last_error()
+    top = np.max(np.abs(w))
+    ref = np.sort(np.abs(w))[::-1][:k]
+    assert np.max(np.abs(np.abs(lam) - ref)) < 1e-13 * top
+    live = np.abs(lam) > 1e-13 * top
+    assert np.max(np.abs(M @ U - U * lam)[:, live]) < 1e-12 * top
+    assert np.max(np.abs(U.T @ U - np.eye(k))[np.ix_(live, live)]) < 1e-12
+
+
 # A spectrum that decays too slowly for the block iteration (the top-k
 # subspace contracts by sigma_l / sigma_k ~ 0.97 per iteration, so 80
 # iterations leave it far from converged): such blocks, up to 384 on their

@@ -244,10 +244,12 @@ void launch_trace_normalize(hipStream_t st, const TraceDesc* d_descs, const Trac
                             int nprob, int64_t max_size);
 size_t jacobi_lds_bytes(int n);
 // pivoted Cholesky QR of Gram matrices (JacobiDesc: G in, W = P R^{-1} out,
-// lam = R_jj); columns below null_rel2 * max diag are dropped.  With d_conv
+// lam = R_jj); columns below null_rel2 * max diag are dropped, or with span
+// (null_rel2 0) unresolved columns kept as they are.  With d_conv
 // the stopping rule follows, on each problem's R_jj.
 void launch_cholqr(hipStream_t st, const JacobiDesc* d_descs, int nd, int nmin, int nmax,
-                   double null_rel2, const ConvDesc* d_conv = nullptr, const ConvRule& rule = ConvRule());
+                   double null_rel2, bool span = false, const ConvDesc* d_conv = nullptr,
+                   const ConvRule& rule = ConvRule());
 void launch_jacobi(hipStream_t st, const JacobiDesc* d_descs, int nd, int nmax, double tol,
                    int max_sweeps);
 void launch_colnorm(hipStream_t st, const ColDesc* d_descs, int nd, int ncol_max, double rtol);

@@ -1933,7 +1933,7 @@ __global__ __launch_bounds__(JAC_TMAX) void k_jacobi(const JacobiDesc* __restric
 // factorised whole anyway stops once even twice its current rate could not
 // reach the target in the iterations left.
 __device__ __forceinline__ void conv_step(const ConvDesc& D, const double* sv, const ConvRule& rule,
-                                          int lane) {
+                                          int lane, bool noisy = false) {
     // the last of the k wanted values above the null threshold
     int kk = 0;
     const double top = sv[0];
@@ -1950,8 +1950,12 @@ __device__ __forceinline__ void conv_step(const ConvDesc& D, const double* sv, c
         if (D.squared) r *= r;
         r = fmin(r, 1.0);
     }
+    // (2 stands for 1 after a first step with columns below its resolution:
+    // the next pivots are too small, their ratio does not count)
     double prod = *D.prod;
-    if (it >= rule.min_iters) prod *= r;
+    if (prod > 1.0) prod = 1.0;
+    else if (it >= rule.min_iters) prod *= r;
+    if (it == 1 && noisy) prod = 2.0;
     *D.it = it;
     *D.prod = prod;
     if ((it >= rule.min_iters && prod < rule.target) || it >= rule.max_iters) *D.done = 1;
@@ -2017,7 +2021,17 @@ __device__ __forceinline__ int wave_max_i32(int x) {
     return __builtin_amdgcn_readlane(x, 63);
 }
 
-template <int N>
+//
+// SPAN: the basis must keep all n directions.  G resolves a column down to
+// 1e-7 of its own norm; what it has left below that (d <= SPAN_FLOOR G_pp) is
+// noise, and dropping or eliminating with such a column would lose its direction
+// for good (after a random start, every eigenvalue below 1e-8 of the
+// largest).  It stays as it is, less the resolved pivots and divided by that
+// floor: the next product's columns are graded and resolve it.  lam of such
+// a column is the floor, the stopping rule is told.
+constexpr double SPAN_FLOOR = 1e-14;
+
+template <int N, bool SPAN>
 __global__ __launch_bounds__(64 * CholLds<N>::WAVES) void k_cholqr(const JacobiDesc* __restrict__ descs,
                                                                   int nd, double null_rel2,
                                                                   const ConvDesc* __restrict__ conv,
@@ -2051,14 +2065,16 @@ __global__ __launch_bounds__(64 * CholLds<N>::WAVES) void k_cholqr(const JacobiD
     __syncthreads();
     // what is left of the diagonal (panel wave); -1 in a pivoted row, whose
     // entries of L, A and R-to-be past its own step are not used
-    double d[ROWS];
+    double d[ROWS], dfloor[ROWS];
     double nfloor = 0.0;
+    bool noisy = false;
     if (w == 0) {
         double dmax = 0.0;
 #pragma unroll
         for (int q = 0; q < ROWS; ++q) {
             const int i = lane + 64 * q;
             d[q] = i < n ? A[min(i, n - 1) * (LD + 1)] : -1.0;
+            dfloor[q] = i < n ? SPAN_FLOOR * d[q] : -1.0;
             dmax = fmax(dmax, d[q]);
         }
 #pragma unroll
@@ -2100,7 +2116,13 @@ __global__ __launch_bounds__(64 * CholLds<N>::WAVES) void k_cholqr(const JacobiD
                 for (int q = 0; q < ROWS; ++q) c[q] = ap[min(lane + 64 * q, N - 1)];
 #pragma unroll
                 for (int k = 0; k < jj; ++k) lp[k] = xp[k];
-                const double rs = rsqrt_refined(v);
+                double rs = rsqrt_refined(v);
+                if (SPAN) {   // (a column of noise: nothing is eliminated with it)
+                    const double f = lane_read(4 * (p & 63), ROWS > 1 && p >= 64 ? dfloor[ROWS - 1] : dfloor[0]);
+                    const bool noise = __builtin_amdgcn_readfirstlane(v <= f);
+                    noisy = noisy || noise;
+                    rs = noise ? 0.0 : rs;
+                }
                 pv = lane == jj ? p : pv;
                 vh = lane == jj ? hi : vh;
                 vl = lane == jj ? lo : vl;
@@ -2116,6 +2138,10 @@ __global__ __launch_bounds__(64 * CholLds<N>::WAVES) void k_cholqr(const JacobiD
                     const double l = (c[q] + c2) * rs;
                     lr[q][jj] = l;
                     d[q] = i == p ? -1.0 : fma(-l, l, d[q]);
+                    if (SPAN) {
+                        dfloor[q] = i == p ? -1.0 : dfloor[q];
+                        d[q] = d[q] < dfloor[q] ? dfloor[q] : d[q];
+                    }
                     if (i < N) X[i * LD + 16 * pb + jj] = l;
                 }
                 wave_order();
@@ -2220,7 +2246,7 @@ __global__ __launch_bounds__(64 * CholLds<N>::WAVES) void k_cholqr(const JacobiD
     if (t < n) D.lam[t] = piv[t];
     if (t == 0 && D.sweeps) *D.sweeps = 0;
     // (a problem that is done needs no product with W any more)
-    if (conv && w == 0) conv_step(conv[blockIdx.x], piv, rule, lane);
+    if (conv && w == 0) conv_step(conv[blockIdx.x], piv, rule, lane, noisy);
 }
 
 // ------------------------------------------------- column norms / normalise
@@ -3194,23 +3220,25 @@ void launch_jacobi(hipStream_t st, const JacobiDesc* d_descs, int nd, int nmax, 
 // Problems of at most CQ64 columns run on k_cholqr<64>, larger ones on
 // k_cholqr<LMAX> (each kernel skips the other's), so the kernel a problem gets
 // depends on its own size only, never on the rest of its launch group.
-template <int N>
+template <int N, bool SPAN>
 static void launch_cholqr_n(hipStream_t st, const JacobiDesc* d_descs, int nd, double null_rel2,
                             const ConvDesc* d_conv, const ConvRule& rule) {
     static const hipError_t attr = hipFuncSetAttribute(
-        (const void*)k_cholqr<N>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)CholLds<N>::BYTES);
+        (const void*)k_cholqr<N, SPAN>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)CholLds<N>::BYTES);
     TNR_HIP(attr);
     ProfScope ps(st, PK_JACOBI, 0.0, 0.0);
-    TNR_LAUNCH(ps, k_cholqr<N>, dim3(nd), dim3(64 * CholLds<N>::WAVES), CholLds<N>::BYTES, st, d_descs, nd,
-               null_rel2, d_conv, rule);
+    TNR_LAUNCH(ps, (k_cholqr<N, SPAN>), dim3(nd), dim3(64 * CholLds<N>::WAVES), CholLds<N>::BYTES, st, d_descs,
+               nd, null_rel2, d_conv, rule);
     TNR_HIP(hipGetLastError());
 }
 
 void launch_cholqr(hipStream_t st, const JacobiDesc* d_descs, int nd, int nmin, int nmax,
-                   double null_rel2, const ConvDesc* d_conv, const ConvRule& rule) {
+                   double null_rel2, bool span, const ConvDesc* d_conv, const ConvRule& rule) {
     if (nd <= 0) return;
-    if (nmin <= CQ64) launch_cholqr_n<CQ64>(st, d_descs, nd, null_rel2, d_conv, rule);
-    if (nmax > CQ64) launch_cholqr_n<LMAX>(st, d_descs, nd, null_rel2, d_conv, rule);
+    if (nmin <= CQ64) (span ? launch_cholqr_n<CQ64, true> : launch_cholqr_n<CQ64, false>)(
+        st, d_descs, nd, null_rel2, d_conv, rule);
+    if (nmax > CQ64) (span ? launch_cholqr_n<LMAX, true> : launch_cholqr_n<LMAX, false>)(
+        st, d_descs, nd, null_rel2, d_conv, rule);
 }
 
 void launch_lincomb(hipStream_t st, const LinDesc* d_descs, int nd, int64_t total) {

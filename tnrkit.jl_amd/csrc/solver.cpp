@@ -112,6 +112,7 @@ struct RR {
 struct RRPlan {
     int passes = 1, lmax = 0, lmin = 0;
     bool chol = false;          // one pass, pivoted Cholesky QR instead of Jacobi
+    bool span = false;          // Cholesky QR that keeps every direction (null_rel2 = 0)
     bool tight = false;
     GemmPlan gram[2], rot[2];
     std::vector<JacobiDesc> jac[2];
@@ -201,7 +202,7 @@ void rr_issue(Ctx& ctx, RRPlan& P, bool first = false, const ConvDesc* conv = nu
         const bool in_loop = P.passes == 1 && !P.tight;
         if (P.chol)
             launch_cholqr(ctx.stream, P.d_jac[pass], (int)P.jac[pass].size(), P.lmin, P.lmax,
-                          cfg.null_rtol * cfg.null_rtol, conv, conv_rule(cfg));
+                          P.span ? 0.0 : cfg.null_rtol * cfg.null_rtol, P.span, conv, conv_rule(cfg));
         else
             launch_jacobi(ctx.stream, P.d_jac[pass], (int)P.jac[pass].size(), P.lmax,
                           !in_loop ? cfg.jacobi_tol
@@ -212,9 +213,10 @@ void rr_issue(Ctx& ctx, RRPlan& P, bool first = false, const ConvDesc* conv = nu
     if (!P.chol) launch_colnorm(ctx.stream, P.d_col, (int)P.col.size(), P.lmax, cfg.null_rtol);
 }
 
-void rr_grouped(Ctx& ctx, const std::vector<RR>& jobs, int passes, bool tight = false) {
+void rr_grouped(Ctx& ctx, const std::vector<RR>& jobs, int passes, bool tight = false, bool chol = false) {
     if (jobs.empty()) return;
-    RRPlan P = rr_plan(ctx, jobs, passes, false, tight);
+    RRPlan P = rr_plan(ctx, jobs, passes, chol, tight);
+    P.span = chol;
     DescArena a;
     rr_stage(P, a);
     a.commit(ctx);
@@ -1045,7 +1047,7 @@ void eigh_grouped(Ctx& ctx, const std::vector<EighIn>& in, std::vector<EighOut>&
         std::vector<FillDesc> fills;
         std::vector<RR> rY, rV;
         std::vector<ColDesc> sym;
-        std::vector<GemmJob> jMV, jF, jH;
+        std::vector<GemmJob> jMV, jQ, jF, jH;
         std::vector<ConvDesc> conv;
         int nmax = 0;
         for (int i = 0; i < P; ++i) {
@@ -1074,15 +1076,14 @@ void eigh_grouped(Ctx& ctx, const std::vector<EighIn>& in, std::vector<EighOut>&
             conv.push_back(ConvDesc{cfg.cholqr_eigh ? x.lam.d() : sv, l, s.kmax, 0, cs.it(i),
                                     cs.prod(i), cs.done(i), s.n <= kWholeMax});
             // one tight pass on the loop's last rotated Y (in Y2), output into
-            // Y; after Cholesky QR steps Y2 is no Ritz basis: two passes on Y
+            // Y.  A Cholesky QR step that ends the loop leaves out its last
+            // rotation: Y2 = Y W first, then a second step on these columns
+            // (Jacobi would not do: equal diagonals, rotated by 45 degrees
+            // at every off-diagonal above roundoff, need not settle).
             if (cfg.cholqr_eigh)
-                rV.push_back(RR{x.Y.d(), s.n, l, s.n, x.Y2.d(), x.G.d(), x.W.d(), x.W2.d(),
-                                x.lam.d(), x.sw.as<int>(), nullptr, x.V.d(), s.n, sv, nullptr,
-                                failv.d() + iter[i]});
-            else
-                rV.push_back(RR{x.Y2.d(), s.n, l, s.n, x.Y.d(), x.G.d(), x.W.d(), x.W2.d(),
-                                x.lam.d(), x.sw.as<int>(), nullptr, x.V.d(), s.n, sv, nullptr,
-                                failv.d() + iter[i]});
+                jQ.push_back(GemmJob{x.Y.d(), x.W.d(), x.Y2.d(), s.n, l, l, s.n, l, s.n, 0, 0});
+            rV.push_back(RR{x.Y2.d(), s.n, l, s.n, x.Y.d(), x.G.d(), x.W.d(), x.W2.d(), x.lam.d(),
+                            x.sw.as<int>(), nullptr, x.V.d(), s.n, sv, nullptr, failv.d() + iter[i]});
             jF.push_back(GemmJob{s.M, x.V.d(), x.Y.d(), s.n, l, s.n, s.ld, s.n, s.n, 0, 0});
             jH.push_back(GemmJob{x.V.d(), x.Y.d(), x.G.d(), l, l, s.n, s.n, s.n, l, 1, 0});
             nmax = std::max(nmax, s.n);
@@ -1093,6 +1094,7 @@ void eigh_grouped(Ctx& ctx, const std::vector<EighIn>& in, std::vector<EighOut>&
         // (random start block used as is, see svd_grouped)
         GemmPlan pMV = gemm_plan(ctx, jMV);
         RRPlan pY = rr_plan(ctx, rY, 1, cfg.cholqr_eigh);
+        pY.span = cfg.cholqr_eigh;
         DescArena a;
         gemm_stage(pMV, a);
         rr_stage(pY, a);
@@ -1103,14 +1105,18 @@ void eigh_grouped(Ctx& ctx, const std::vector<EighIn>& in, std::vector<EighOut>&
         const ConvDesc* d_conv = a.at<ConvDesc>(o_conv);
         iterate(ctx, cs, [&](int it) {
             gemm_issue(ctx, pMV);
-            rr_issue(ctx, pY, it == 0);
-            launch_conv(ctx.stream, d_conv, P, conv_rule(cfg));
+            rr_issue(ctx, pY, it == 0, cfg.cholqr_eigh ? d_conv : nullptr);
+            if (!cfg.cholqr_eigh) launch_conv(ctx.stream, d_conv, P, conv_rule(cfg));
         });
         // V at full orthonormality from the loop's last rotated Y = M V W
         // (the loop uses a looser Jacobi threshold; one pass at the final
-        // threshold, as in svd_grouped), or from the last Y in two passes
-        if (cfg.cholqr_eigh) rr_grouped(ctx, rV, 2);
-        else rr_grouped(ctx, rV, 1, true);
+        // threshold, as in svd_grouped) or from the last Cholesky QR basis
+        if (cfg.cholqr_eigh) {
+            gemm_grouped(ctx, jQ);
+            rr_grouped(ctx, rV, 1, false, true);
+        } else {
+            rr_grouped(ctx, rV, 1, true);
+        }
         // Ritz pairs: H = V^T (M V), eigendecompose, U = V W
         gemm_grouped(ctx, jF);
         gemm_grouped(ctx, jH);

@@ -4,10 +4,11 @@
 // MFMA, parallel-order Jacobi in LDS, a second Gram/Jacobi pass on the
 // rotated columns (which are then nearly orthogonal, so the second pass is
 // relatively accurate), column norms.  Larger problems run block subspace
-// iteration (Y = M V, Z = M^T U) with the same two-pass Gram/Jacobi
-// Rayleigh-Ritz step after every product, until the top-k subspace has
-// converged to working precision; the Ritz triplets are then extracted from
-// Y = M V.  All problems of a call advance together in grouped launches.
+// iteration (Y = M V, Z = M^T U; Y = M V for eigenpairs) with a pivoted
+// Cholesky QR step after every product, until the top-k subspace has
+// converged to working precision; the Ritz triplets (pairs) are then extracted
+// by Gram/Jacobi steps.  All problems of a call advance together in grouped
+// launches.
 #pragma once
 
 #include <vector>
@@ -88,11 +89,15 @@ struct SolverCfg {
     // vectors one by one, so the Gram matrices of the final extraction are
     // nearly diagonal and cheap for Jacobi.  Measured on single BTRG
     // chi = 32 runs: 17 % less time with the Z side on Cholesky QR.  The
-    // eigensolver keeps Rayleigh-Ritz: with Cholesky QR its stopping rule on
-    // the pivots ended HOTRG chi = 48 solves early (1e-7 norm errors).
+    // eigensolver's steps keep every direction (span): its spectra are
+    // squares, and after a random start whatever lies below 1e-8 of the
+    // largest value is beyond the Gram matrix's resolution; dropped there, it
+    // ended HOTRG chi = 48 solves early (1e-7 norm errors).  Rayleigh-Ritz ->
+    // Cholesky QR in its loop: HOTRG chi 16 20.5 -> 14.6 ms, chi 32 59.1 ->
+    // 41.5 (7 steps), the same number of iterations.
     bool cholqr_y = true;
     bool cholqr_z = true;
-    bool cholqr_eigh = false;
+    bool cholqr_eigh = true;
     // Rayleigh-Ritz passes that rebuild V from the last Z (with Cholesky QR
     // on the Z side) and that extract the Ritz triplets from Y = M V.  V is
     // a Ritz basis of the converged subspace, so the columns of M V are
