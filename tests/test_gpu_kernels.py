@@ -307,6 +307,40 @@ def test_eigh_truncated(tk, n, k):
     assert np.max(np.abs(Pk - Pr)) < 1e-9
 
 
+# Direct SVDs from side 17 on precondition the Gram matrix twice before one
+# Jacobi pass: sides around the rule, the 16-column panels and both kernels, more
+# columns than rows, spectra beyond the Gram matrix's resolution, exact zeros.
+# Backward errors of a few n eps (96 eps = 2e-14); all of V is orthogonal (also
+# the null directions), U where the singular value is above roundoff.
+@pytest.mark.parametrize("n", [16, 17, 31, 33, 63, 64, 65, 81, 96])
+@pytest.mark.parametrize("spec", ["0.5", "gap", "rank", "flat", "zeros", "columns"])
+def test_direct_svd_preconditioned_edges(tk, n, spec):
+    rng = np.random.default_rng(n)
+    m = n + 7
+    j = np.arange(n)
+    U0, _ = np.linalg.qr(rng.standard_normal((m, n)))
+    V0, _ = np.linalg.qr(rng.standard_normal((n, n)))
+    w = {"0.5": 0.5 ** j, "gap": np.where(j < n // 3, 1.0, 1e-12) * 0.9 ** j,
+         "rank": np.where(j < n // 3, 0.7 ** j, 0.0)}.get(spec, np.ones(n))
+    M = (U0 * w) @ V0.T
+    if spec == "zeros":
+        M = np.zeros((m, n))
+        M[j[: n // 2] * 2 % m, j[: n // 2]] = 1.0 + j[: n // 2]
+    if spec == "columns":
+        M = rng.standard_normal((m, n)) * np.logspace(-9, 0, n)
+    for A in (M, np.ascontiguousarray(M.T)):
+        U, s, V, it = svd(tk, A, n)
+        assert it == 0
+        ref = np.linalg.svd(A, compute_uv=False)
+        assert np.max(np.abs(s - ref)) < 1e-13 * ref[0]
+        assert np.max(np.abs((U * s) @ V.T - A)) < 1e-13 * ref[0]
+        live = s > 1e-13 * ref[0]
+        if A is not M:
+            U, V = V, U   # the smaller side's vectors are the complete ones
+        assert np.max(np.abs(V.T @ V - np.eye(n))) < 1e-13
+        assert np.max(np.abs(U.T @ U - np.eye(n))[np.ix_(live, live)]) < 1e-13
+
+
 # The block iteration's Cholesky QR has to keep every direction of a steep
 # spectrum: after the random start all columns are within 1e-8 of the leading
 # eigenvectors, below what their Gram matrix resolves.  Spectra: steep ones

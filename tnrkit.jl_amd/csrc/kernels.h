@@ -243,6 +243,8 @@ void launch_gemm_reduce(hipStream_t st, const GemmDesc* d_descs, int nd, const i
 void launch_trace_normalize(hipStream_t st, const TraceDesc* d_descs, const TraceProb* d_probs,
                             int nprob, int64_t max_size);
 size_t jacobi_lds_bytes(int n);
+// orthogonal W = Q with (Y Q)^T (Y Q) closer to diagonal than G = Y^T Y
+void launch_precond(hipStream_t st, const JacobiDesc* d_descs, int nd, int nmin, int nmax);
 // pivoted Cholesky QR of Gram matrices (JacobiDesc: G in, W = P R^{-1} out,
 // lam = R_jj); columns below null_rel2 * max diag are dropped, or with span
 // (null_rel2 0) unresolved columns kept as they are.  With d_conv

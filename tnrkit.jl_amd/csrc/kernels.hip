@@ -2000,7 +2000,7 @@ struct CholLds {
     static constexpr int ROWS = (N + 63) / 64, BITS = N > 64 ? 7 : 6;
     static constexpr int WAVES = 8;
     static constexpr size_t BYTES =
-        2 * (size_t)N * LD * sizeof(double) + 2 * N * sizeof(double) + (2 * N + 2) * sizeof(int);
+        2 * (size_t)N * LD * sizeof(double) + 2 * N * sizeof(double) + (3 * N + 2) * sizeof(int);
 };
 
 // Largest of x over the wave: within each row of 16 lanes by lane swaps, then
@@ -2031,35 +2031,31 @@ __device__ __forceinline__ int wave_max_i32(int x) {
 // a column is the floor, the stopping rule is told.
 constexpr double SPAN_FLOOR = 1e-14;
 
-template <int N, bool SPAN>
-__global__ __launch_bounds__(64 * CholLds<N>::WAVES) void k_cholqr(const JacobiDesc* __restrict__ descs,
-                                                                  int nd, double null_rel2,
-                                                                  const ConvDesc* __restrict__ conv,
-                                                                  ConvRule rule) {
-    using L = CholLds<N>;
-    constexpr int LD = L::LD, ROWS = L::ROWS, NT = 64 * L::WAVES;
-    extern __shared__ double lds[];
-    const JacobiDesc D = descs[blockIdx.x];
-    // (the other sizes of the group are the other kernel's)
-    if (D.n > N || (N > CQ64 && D.n <= CQ64) || (D.skip && *D.skip)) return;
-    const int n = D.n, t = threadIdx.x, lane = t & 63, l0 = lane & 15, l1 = lane >> 4;
-    const int w = __builtin_amdgcn_readfirstlane(t >> 6);
-    const int T = (n + 15) / 16, m = 16 * T;
-    double* A = lds;              // A[i + k LD]; later R in pivot order
-    double* X = A + N * LD;       // L[i][j] at X[i LD + j]; later X[i + j LD]
-    double* piv = X + N * LD;     // pivot values, then R[j][j]
-    double* rinv = piv + N;       // 1 / R[j][j]
-    int* perm = (int*)(rinv + N);
-    int* iperm = perm + N;
-    int* rank_ = iperm + N;
-    // every lane loads (clamped, in bounds), so the loads are not predicated
-    // and stay in flight together
+// G into A, zero up to m x m.  Every lane loads (clamped, in bounds), so the
+// loads are not predicated and stay in flight together.
+template <int N>
+__device__ __forceinline__ void chol_load(const JacobiDesc& D, double* A, int n, int m) {
+    constexpr int LD = CholLds<N>::LD, NT = 64 * CholLds<N>::WAVES;
+    const int t = threadIdx.x;
 #pragma unroll 8
     for (int e = t; e < m * N; e += NT) {
         const int c = e / N, r = e - c * N;
         const double v = D.G[min(r, n - 1) + (int64_t)min(c, n - 1) * D.ldg];
         A[r + c * LD] = r < n && c < n ? v : 0.0;
     }
+}
+
+// The pivot steps on A (m columns of N rows in LDS, zero beyond n): perm, piv (pivot values),
+// *rank_ and the rows of L in X.  True if a column was noise (SPAN; in the
+// panel wave).
+template <int N, bool SPAN>
+__device__ __forceinline__ bool chol_panels(double* A, double* X, double* piv, int* perm, int* iperm, int* rank_,
+                                            int n, double null_rel2) {
+    using L = CholLds<N>;
+    constexpr int LD = L::LD, ROWS = L::ROWS;
+    const int t = threadIdx.x, lane = t & 63, l0 = lane & 15, l1 = lane >> 4;
+    const int w = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int T = (n + 15) / 16;
     if (t < N) iperm[t] = -1;
     if (t == 0) *rank_ = n;
     __syncthreads();
@@ -2181,7 +2177,19 @@ __global__ __launch_bounds__(64 * CholLds<N>::WAVES) void k_cholqr(const JacobiD
         }
         __syncthreads();
     }
-    const int rank = *rank_;
+    return noisy;
+}
+
+// R in pivot order into A's place, then X = R^{-1} (identity beyond rank);
+// piv becomes R[j][j].  Ends with a barrier.
+template <int N>
+__device__ __forceinline__ void chol_invert(double* A, double* X, double* piv, double* rinv, const int* perm,
+                                            int* iperm, int rank, int n) {
+    using L = CholLds<N>;
+    constexpr int LD = L::LD, NT = 64 * L::WAVES;
+    const int t = threadIdx.x, lane = t & 63, l0 = lane & 15, l1 = lane >> 4;
+    const int w = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int T = (n + 15) / 16, m = 16 * T;
     // R in pivot order: R[i + k LD] = R[i][k] for i <= k < rank, else 1 / 0
     // (in A's place)
 #pragma unroll 4
@@ -2235,6 +2243,31 @@ __global__ __launch_bounds__(64 * CholLds<N>::WAVES) void k_cholqr(const JacobiD
         }
         __syncthreads();
     }
+}
+
+template <int N, bool SPAN>
+__global__ __launch_bounds__(64 * CholLds<N>::WAVES) void k_cholqr(const JacobiDesc* __restrict__ descs,
+                                                                  int nd, double null_rel2,
+                                                                  const ConvDesc* __restrict__ conv,
+                                                                  ConvRule rule) {
+    using L = CholLds<N>;
+    constexpr int LD = L::LD, NT = 64 * L::WAVES;
+    extern __shared__ double lds[];
+    const JacobiDesc D = descs[blockIdx.x];
+    // (the other sizes of the group are the other kernel's)
+    if (D.n > N || (N > CQ64 && D.n <= CQ64) || (D.skip && *D.skip)) return;
+    const int n = D.n, t = threadIdx.x, m = 16 * ((n + 15) / 16);
+    double* A = lds;              // A[i + k LD]; later R in pivot order
+    double* X = A + N * LD;       // L[i][j] at X[i LD + j]; later X[i + j LD]
+    double* piv = X + N * LD;     // pivot values, then R[j][j]
+    double* rinv = piv + N;       // 1 / R[j][j]
+    int* perm = (int*)(rinv + N);
+    int* iperm = perm + N;
+    int* rank_ = iperm + N;
+    chol_load<N>(D, A, n, m);
+    const bool noisy = chol_panels<N, SPAN>(A, X, piv, perm, iperm, rank_, n, null_rel2);
+    const int rank = *rank_;
+    chol_invert<N>(A, X, piv, rinv, perm, iperm, rank, n);
     // W[perm[r]][c] = X[r][c] for r <= c < rank, zero elsewhere
 #pragma unroll 4
     for (int e = t; e < n * N; e += NT) {
@@ -2246,7 +2279,161 @@ __global__ __launch_bounds__(64 * CholLds<N>::WAVES) void k_cholqr(const JacobiD
     if (t < n) D.lam[t] = piv[t];
     if (t == 0 && D.sweeps) *D.sweeps = 0;
     // (a problem that is done needs no product with W any more)
-    if (conv && w == 0) conv_step(conv[blockIdx.x], piv, rule, lane, noisy);
+    if (conv && t < 64) conv_step(conv[blockIdx.x], piv, rule, t, noisy);
+}
+
+// ------------------------------------------- basis for a Jacobi solve
+// One workgroup per n x n Gram matrix G = Y^T Y (n <= LMAX): an orthogonal Q
+// (n x n, into W) for which (Y Q)^T (Y Q) is far closer to diagonal than G, in
+// decreasing order.  G = P R^T R P^T by diagonal pivoting; the QR factor of
+// R^T, from the Cholesky factor of H = R R^T, gives Q = P R^T P2 R2^{-1}:
+// one step of the QR iteration on G, which scales entry (i, j) by about
+// sigma_j^2 / sigma_i^2.  The rows of R are graded and well conditioned after
+// scaling, so Q is orthogonal to ~1e-14 whatever the spectrum; a Newton
+// step Q (3 - Q^T Q) / 2 makes it 1e-16.  What G does not resolve (below
+// 1e-8 of the largest singular value) is kept as it is (SPAN) and resolved
+// in a second round, on the Gram matrix of the graded columns Y Q.
+// Two rounds take the spectra of TRG and BTRG blocks (twelve decades) from
+// 20 + 8 Jacobi sweeps in two passes to 4 - 6 in one, and whole solves, copies
+// included, from 0.50 to 0.34 ms at n = 32, 1.15 to 0.49 at 64, 2.45 to 0.88 at
+// 85; singular values and vectors come out closer to orthogonal than from two
+// Jacobi passes.  Like k_cholqr bound by the chain of pivot steps.
+template <int N>
+__global__ __launch_bounds__(64 * CholLds<N>::WAVES) void k_precond(const JacobiDesc* __restrict__ descs,
+                                                                   int nd) {
+    using L = CholLds<N>;
+    constexpr int LD = L::LD, NT = 64 * L::WAVES, TMAX = N / 16;
+    extern __shared__ double lds[];
+    const JacobiDesc D = descs[blockIdx.x];
+    // (the other sizes of the group are the other kernel's)
+    if (D.n > N || (N > CQ64 && D.n <= CQ64) || (D.skip && *D.skip)) return;
+    const int n = D.n, t = threadIdx.x, lane = t & 63, l0 = lane & 15, l1 = lane >> 4;
+    const int w = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int T = (n + 15) / 16, m = 16 * T;
+    double* A = lds;
+    double* B = A + N * LD;
+    double* piv = B + N * LD;
+    double* rinv = piv + N;
+    int* perm = (int*)(rinv + N);
+    int* iperm = perm + N;
+    int* rank_ = iperm + N;
+    int* perm1 = rank_ + 2;
+    chol_load<N>(D, A, n, m);
+    chol_panels<N, true>(A, B, piv, perm1, iperm, rank_, n, 0.0);
+    const int rank = *rank_;
+    // (columns of zeros have no pivot: the rows left over, in order, with R = I)
+    if (t < rank) iperm[perm1[t]] = t;
+    __syncthreads();
+    if (t < n && iperm[t] < 0) {
+        int at = rank;
+        for (int i = 0; i < t; ++i) at += iperm[i] < 0;
+        if (at < n) perm1[at] = t;
+    }
+    // R[i + c LD], here and in W until Q is formed
+#pragma unroll 4
+    for (int e = t; e < m * N; e += NT) {
+        const int c = e / N, r = e - c * N;
+        const double v = B[(c < rank ? perm1[c] : 0) * LD + r];
+        const double x = c < rank && r < c ? v : (r != c ? 0.0 : c < rank ? sqrt(piv[c]) : 1.0);
+        A[r + c * LD] = x;
+        if (r < n && c < n) D.W[r + (int64_t)c * D.ldw] = x;
+    }
+    __syncthreads();
+    // H = R R^T, both triangles, zero below as chol_panels takes it
+    for (int e = t; e < m * N; e += NT)
+        if (e % N >= m) B[e % N + (e / N) * LD] = 0.0;
+    for (int u = w; u < T * (T + 1) / 2; u += L::WAVES) {
+        int J = 0;
+        while ((J + 1) * (J + 2) / 2 <= u) ++J;
+        const int I = u - J * (J + 1) / 2;
+        dbl4 c = dbl4{0, 0, 0, 0};
+        for (int K = J; K < T; ++K)
+#pragma unroll
+            for (int kk = 0; kk < 4; ++kk) {
+                const int at = (16 * K + 4 * kk + l1) * LD + l0;
+                c = __builtin_amdgcn_mfma_f64_16x16x4f64(A[16 * I + at], A[16 * J + at], c, 0, 0, 0);
+            }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int r = 16 * I + l1 + 4 * q, s = 16 * J + l0;
+            const double x = r < n && s < n ? c[q] : 0.0;
+            B[r + s * LD] = x;
+            if (I != J) B[s + r * LD] = x;
+        }
+    }
+    __syncthreads();
+    chol_panels<N, true>(B, A, piv, perm, iperm, rank_, n, 0.0);
+    chol_invert<N>(B, A, piv, rinv, perm, iperm, *rank_, n);
+    // the rows of R in H's pivot order (the bounds hold for a NaN, whose pivots
+    // are arbitrary, too)
+#pragma unroll 4
+    for (int e = t; e < m * N; e += NT) {
+        const int c = e / N, k = e - c * N;
+        const int row = (int)min((unsigned)perm[min(k, n - 1)], (unsigned)(n - 1));
+        const double v = D.W[row + (int64_t)min(c, n - 1) * D.ldw];
+        B[k + c * LD] = k < n && c < n ? v : 0.0;
+    }
+    __syncthreads();
+    // Q (rows in the order of perm1) = R^T X in tiles of 16, kept until all
+    // waves have read B
+    constexpr int PER = (TMAX * TMAX + L::WAVES - 1) / L::WAVES;
+    dbl4 q[PER];
+#pragma unroll
+    for (int s = 0; s < PER; ++s) {
+        const int u = w + s * L::WAVES;
+        q[s] = dbl4{0, 0, 0, 0};
+        if (u >= T * T) continue;
+        const int I = u % T, J = u / T;
+        for (int K = 0; K <= J; ++K)
+#pragma unroll
+            for (int kk = 0; kk < 4; ++kk) {
+                const int at = 16 * K + 4 * kk + l1;
+                q[s] = __builtin_amdgcn_mfma_f64_16x16x4f64(B[at + (16 * I + l0) * LD], A[at + (16 * J + l0) * LD],
+                                                            q[s], 0, 0, 0);
+            }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int s = 0; s < PER; ++s) {
+        const int u = w + s * L::WAVES;
+        if (u >= T * T) continue;
+#pragma unroll
+        for (int x = 0; x < 4; ++x) B[16 * (u % T) + l1 + 4 * x + (16 * (u / T) + l0) * LD] = q[s][x];
+    }
+    __syncthreads();
+    // S = Q^T Q in A's place
+    for (int u = w; u < T * (T + 1) / 2; u += L::WAVES) {
+        int J = 0;
+        while ((J + 1) * (J + 2) / 2 <= u) ++J;
+        const int I = u - J * (J + 1) / 2;
+        dbl4 c = dbl4{0, 0, 0, 0};
+        for (int k = l1; k < m; k += 4)
+            c = __builtin_amdgcn_mfma_f64_16x16x4f64(B[k + (16 * I + l0) * LD], B[k + (16 * J + l0) * LD], c, 0, 0,
+                                                     0);
+#pragma unroll
+        for (int x = 0; x < 4; ++x) {
+            const int r = 16 * I + l1 + 4 * x, s = 16 * J + l0;
+            A[r + s * LD] = c[x];
+            if (I != J) A[s + r * LD] = c[x];
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int s = 0; s < PER; ++s) {
+        const int u = w + s * L::WAVES;
+        if (u >= T * T) continue;
+        const int I = u % T, J = u / T;
+        dbl4 c = dbl4{0, 0, 0, 0};
+        for (int k = l1; k < m; k += 4)
+            c = __builtin_amdgcn_mfma_f64_16x16x4f64(B[16 * I + l0 + k * LD], A[k + (16 * J + l0) * LD], c, 0, 0, 0);
+#pragma unroll
+        for (int x = 0; x < 4; ++x) {
+            const int r = 16 * I + l1 + 4 * x, j = 16 * J + l0;
+            if (r < n && j < n)
+                D.W[min((unsigned)perm1[r], (unsigned)(n - 1)) + (int64_t)j * D.ldw] =
+                    fma(-0.5, c[x], 1.5 * q[s][x]);
+        }
+    }
 }
 
 // ------------------------------------------------- column norms / normalise
@@ -3239,6 +3426,22 @@ void launch_cholqr(hipStream_t st, const JacobiDesc* d_descs, int nd, int nmin, 
         st, d_descs, nd, null_rel2, d_conv, rule);
     if (nmax > CQ64) (span ? launch_cholqr_n<LMAX, true> : launch_cholqr_n<LMAX, false>)(
         st, d_descs, nd, null_rel2, d_conv, rule);
+}
+
+template <int N>
+static void launch_precond_n(hipStream_t st, const JacobiDesc* d_descs, int nd) {
+    static const hipError_t attr = hipFuncSetAttribute(
+        (const void*)k_precond<N>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)CholLds<N>::BYTES);
+    TNR_HIP(attr);
+    ProfScope ps(st, PK_JACOBI, 0.0, 0.0);
+    TNR_LAUNCH(ps, k_precond<N>, dim3(nd), dim3(64 * CholLds<N>::WAVES), CholLds<N>::BYTES, st, d_descs, nd);
+    TNR_HIP(hipGetLastError());
+}
+
+void launch_precond(hipStream_t st, const JacobiDesc* d_descs, int nd, int nmin, int nmax) {
+    if (nd <= 0) return;
+    if (nmin <= CQ64) launch_precond_n<CQ64>(st, d_descs, nd);
+    if (nmax > CQ64) launch_precond_n<LMAX>(st, d_descs, nd);
 }
 
 void launch_lincomb(hipStream_t st, const LinDesc* d_descs, int nd, int64_t total) {

@@ -106,7 +106,9 @@ struct RR {
 };
 
 // `passes` = 1 inside the block iteration (the next iteration corrects
-// what one pass leaves), 2 for the final Ritz extraction and direct solves;
+// what one pass leaves), 2 for the final Ritz extraction and direct solves of
+// the smallest matrices, 3 for the other direct ones: two k_precond passes
+// and one Jacobi pass on what they leave, total rotation in W2, columns in Y2;
 // `tight` = one pass at the final threshold, for columns that are already
 // orthogonal to the loop's threshold (the second pass of a two-pass step).
 struct RRPlan {
@@ -114,17 +116,17 @@ struct RRPlan {
     bool chol = false;          // one pass, pivoted Cholesky QR instead of Jacobi
     bool span = false;          // Cholesky QR that keeps every direction (null_rel2 = 0)
     bool tight = false;
-    GemmPlan gram[2], rot[2];
-    std::vector<JacobiDesc> jac[2];
+    GemmPlan gram[3], rot[3];
+    std::vector<JacobiDesc> jac[3];
     std::vector<ColDesc> col;
-    size_t o_jac[2] = {0, 0}, o_col = 0;
-    const JacobiDesc* d_jac[2] = {nullptr, nullptr};
+    size_t o_jac[3] = {0, 0, 0}, o_col = 0;
+    const JacobiDesc* d_jac[3] = {nullptr, nullptr, nullptr};
     const ColDesc* d_col = nullptr;
 };
 
 RRPlan rr_plan(Ctx& ctx, const std::vector<RR>& jobs, int passes, bool chol = false,
                bool tight = false) {
-    TNR_REQUIRE(passes == 1 || passes == 2, TNR_ERR_INTERNAL, "one or two passes");
+    TNR_REQUIRE(passes >= 1 && passes <= 3, TNR_ERR_INTERNAL, "one to three passes");
     TNR_REQUIRE(!chol || passes == 1, TNR_ERR_INTERNAL, "Cholesky QR is a one-pass step");
     TNR_REQUIRE(!tight || (passes == 1 && !chol), TNR_ERR_INTERNAL, "tight is a one-pass Jacobi step");
     RRPlan P;
@@ -140,8 +142,8 @@ RRPlan rr_plan(Ctx& ctx, const std::vector<RR>& jobs, int passes, bool chol = fa
     for (int pass = 0; pass < passes; ++pass) {
         std::vector<GemmJob> gj, rj;
         for (auto& j : jobs) {
-            double* Y = pass == 0 ? j.Y : j.Y2;
-            const int ld = pass == 0 ? j.ldy : j.rows;
+            double* Y = pass != 1 ? j.Y : j.Y2;
+            const int ld = pass != 1 ? j.ldy : j.rows;
             // one pass: its rotation is the total one
             double* W1 = passes == 1 && j.Wtot ? j.Wtot : j.W;
             GemmJob g{Y, Y, j.G, j.l, j.l, j.rows, ld, ld, j.l, 1, 0};   // G = Y^T Y
@@ -149,30 +151,36 @@ RRPlan rr_plan(Ctx& ctx, const std::vector<RR>& jobs, int passes, bool chol = fa
             gj.push_back(g);
             // Cholesky QR: the rotated columns are the orthonormal basis itself
             GemmJob r = chol ? GemmJob{j.Y, W1, j.U, j.rows, j.l, j.l, j.ldy, j.l, j.ldu, 0, 0}
-                        : pass == 0
+                        : pass != 1
                             ? GemmJob{j.Y, W1, j.Y2, j.rows, j.l, j.l, j.ldy, j.l, j.rows, 0, 0}
                             : GemmJob{j.Y2, j.W2, j.Y, j.rows, j.l, j.l, j.rows, j.l, j.ldy, 0, 0};
             r.skip = j.skip;
             rj.push_back(r);
-            if (pass == 1 && j.Wtot) {
-                GemmJob w{j.W, j.W2, j.Wtot, j.l, j.l, j.l, j.l, j.l, j.l, 0, 0};
+            if (pass >= 1 && j.Wtot) {
+                GemmJob w = pass == 1 ? GemmJob{j.W, j.W2, j.Wtot, j.l, j.l, j.l, j.l, j.l, j.l, 0, 0}
+                                      : GemmJob{j.Wtot, j.W, j.W2, j.l, j.l, j.l, j.l, j.l, j.l, 0, 0};
                 w.skip = j.skip;
                 rj.push_back(w);
             }
-            P.jac[pass].push_back(JacobiDesc{j.G, pass == 0 ? W1 : j.W2, j.lam, j.sweeps, j.l, j.l,
+            P.jac[pass].push_back(JacobiDesc{j.G, pass != 1 ? W1 : j.W2, j.lam, j.sweeps, j.l, j.l,
                                              j.l, j.skip, j.fail});
         }
         P.gram[pass] = gemm_plan(ctx, gj);
         P.rot[pass] = gemm_plan(ctx, rj);
     }
-    // rotated columns: Y2 after one pass, Y after two
+    // rotated columns: Y2 after one pass or three, Y after two
     if (!chol)
         for (auto& j : jobs)
-            P.col.push_back(passes == 1
+            P.col.push_back(passes != 2
                                 ? ColDesc{j.Y2, j.U, j.sigma, j.rows, j.l, j.rows, j.ldu, j.skip}
                                 : ColDesc{j.Y, j.U, j.sigma, j.rows, j.l, j.ldy, j.ldu, j.skip});
     return P;
 }
+
+// Smallest side from which a direct SVD takes k_precond before Jacobi: whole
+// solves with / without at 8 0.26 / 0.26 ms, 16 0.27 / 0.27, 18 0.31 / 0.34, 25
+// 0.33 / 0.44, 32 0.34 / 0.50.
+constexpr int kPrecondFrom = 17;
 
 void rr_stage(RRPlan& P, DescArena& a) {
     for (int pass = 0; pass < P.passes; ++pass) {
@@ -203,6 +211,8 @@ void rr_issue(Ctx& ctx, RRPlan& P, bool first = false, const ConvDesc* conv = nu
         if (P.chol)
             launch_cholqr(ctx.stream, P.d_jac[pass], (int)P.jac[pass].size(), P.lmin, P.lmax,
                           P.span ? 0.0 : cfg.null_rtol * cfg.null_rtol, P.span, conv, conv_rule(cfg));
+        else if (P.passes == 3 && pass < 2)
+            launch_precond(ctx.stream, P.d_jac[pass], (int)P.jac[pass].size(), P.lmin, P.lmax);
         else
             launch_jacobi(ctx.stream, P.d_jac[pass], (int)P.jac[pass].size(), P.lmax,
                           !in_loop ? cfg.jacobi_tol
@@ -813,7 +823,7 @@ void svd_grouped(Ctx& ctx, const std::vector<SvdIn>& in, std::vector<SvdOut>& ou
         struct DW { Buf Y, Y2, G, W, W2, Wt, lam, sig, sw; };
         std::vector<DW> w(direct.size());
         std::vector<GatherDesc> gd;
-        std::vector<RR> rr;
+        std::vector<RR> rr, rp;   // two Jacobi passes; k_precond first
         for (size_t i = 0; i < direct.size(); ++i) {
             const SvdIn& s = in[direct[i]];
             const bool tr = s.n > s.m;
@@ -832,23 +842,26 @@ void svd_grouped(Ctx& ctx, const std::vector<SvdIn>& in, std::vector<SvdOut>& ou
             g.in = s.M; g.out = x.Y.d(); g.rows = rows; g.cols = l;
             g.ldi = s.ld; g.ldo = rows; g.trans = tr ? 1 : 0;
             gd.push_back(g);
-            rr.push_back(RR{x.Y.d(), rows, l, rows, x.Y2.d(), x.G.d(), x.W.d(), x.W2.d(),
-                            x.lam.d(), x.sw.as<int>(), x.Wt.d(), x.Y.d(), rows, x.sig.d()});
-            rr.back().fail = failv.d() + direct[i];
+            RR r{x.Y.d(), rows, l, rows, x.Y2.d(), x.G.d(), x.W.d(), x.W2.d(),
+                 x.lam.d(), x.sw.as<int>(), x.Wt.d(), x.Y.d(), rows, x.sig.d()};
+            r.fail = failv.d() + direct[i];
+            (l >= kPrecondFrom ? rp : rr).push_back(r);
         }
         gather_many(ctx, gd);
         rr_grouped(ctx, rr, 2);
+        rr_grouped(ctx, rp, 3);
         for (size_t i = 0; i < direct.size(); ++i) {
             const SvdIn& s = in[direct[i]];
             SvdOut& o = out[direct[i]];
             DW& x = w[i];
             const bool tr = s.n > s.m;
             const int rows = std::max(s.m, s.n), l = std::min(s.m, s.n);
+            Buf& wt = l >= kPrecondFrom ? x.W2 : x.Wt;
             if (!tr) {
                 o.U = std::move(x.Y); o.ldu = rows;
-                o.V = std::move(x.Wt); o.ldv = l;
+                o.V = std::move(wt); o.ldv = l;
             } else {
-                o.U = std::move(x.Wt); o.ldu = l;
+                o.U = std::move(wt); o.ldu = l;
                 o.V = std::move(x.Y); o.ldv = rows;
             }
             o.s = std::move(x.sig);

@@ -1,9 +1,9 @@
 // Grouped truncated SVD and symmetric eigensolver on the device (FP64).
 //
-// Small problems (min(m, n) <= LMAX) are solved directly: Gram matrix on
-// MFMA, parallel-order Jacobi in LDS, a second Gram/Jacobi pass on the
-// rotated columns (which are then nearly orthogonal, so the second pass is
-// relatively accurate), column norms.  Larger problems run block subspace
+// Small problems (min(m, n) <= LMAX) are solved directly: two passes of Gram
+// matrix on MFMA, k_precond, rotation, which leave graded, nearly orthogonal
+// columns (whose Gram matrix is then relatively accurate), one of parallel-order
+// Jacobi in LDS, column norms; the smallest by two Jacobi passes.  Larger problems run block subspace
 // iteration (Y = M V, Z = M^T U; Y = M V for eigenpairs) with a pivoted
 // Cholesky QR step after every product, until the top-k subspace has
 // converged to working precision; the Ritz triplets (pairs) are then extracted
