@@ -187,6 +187,27 @@ def test_convcrit_run_stops_like_the_reference(tk):
     assert np.array_equal(d, ref)
 
 
+# Permutes at odd, unit and unequal extents (legs of sector sizes `dw`, `ds`):
+# first steps of random positive tensors, whose copies merge and decode every
+# rank up to 6, weighted (BTRG) and not, against the oracle (at this module's
+# tolerance: some cut a spectrum; a unit leg beside one above 4 would cut
+# between equal products of eigenvalues).
+@pytest.mark.parametrize("name", ["TRG", "BTRG", "HOTRG", "ATRG"])
+@pytest.mark.parametrize("N,dw,ds", [(1, (3,), (2,)), (1, (1,), (4,)), (2, (1, 2), (2, 1)),
+                                     (2, (3, 0), (1, 2)), (3, (1, 1, 1), (1, 0, 1))])
+def test_permutes_of_odd_extents(tk, name, N, dw, ds):
+    rng = np.random.default_rng(sum(dw) + 10 * sum(ds))
+    w, s = (np.repeat(np.arange(N), d) for d in (dw, ds))
+    q = [w, s, -s % N, -w % N]
+    tot = w[:, None, None, None] + s[:, None, None] + q[2][:, None] + q[3]
+    T = ZT(np.where(tot % N == 0, rng.uniform(0.5, 1.5, tot.shape), 0.0), q, N)
+    ref = osch.run(getattr(osch, name)(T), 16, 1)
+    sc = getattr(tk, name)(to_sym(tk, T))
+    got = tk.run(sc, tk.truncrank(16), tk.maxiter(1), verbosity=0)
+    sc.close()
+    assert np.max(np.abs(np.array(got) / np.array(ref) - 1)) < TOL
+
+
 def _close_rows(got, ref, cols=None, rtol=1e-10):
     """Row-wise: every compared component within rtol of the oracle, or
     within rtol * 1e-4 of the row's first value when it is smaller."""

@@ -230,6 +230,53 @@ static void permute_descs(const BT& src, BT& dst, const std::vector<int>& perm, 
     });
 }
 
+// Dims of extent 1 dropped, neighbours that are neighbours in the source too
+// merged; a weighted dim stays by itself (its index reads the weights).
+static void merge_dims(CopyDesc& d) {
+    int k = 0, wl[2] = {-1, -1};
+    bool weighted_last = false;
+    for (int j = 0; j < d.nd; ++j) {
+        if (d.dim[j] == 1) continue;   // (its weight index stays 0)
+        const bool weighted = d.wleg[0] == j || d.wleg[1] == j;
+        if (k > 0 && !weighted && !weighted_last && d.sstr[j] == d.sstr[k - 1] * d.dim[k - 1] &&
+            d.dstr[j] == d.dstr[k - 1] * d.dim[k - 1] &&
+            (int64_t)d.dim[k - 1] * d.dim[j] < ((int64_t)1 << 31)) {
+            d.dim[k - 1] *= d.dim[j];
+            continue;
+        }
+        d.dim[k] = d.dim[j];
+        d.sstr[k] = d.sstr[j];
+        d.dstr[k] = d.dstr[j];
+        for (int w = 0; w < 2; ++w)
+            if (d.wleg[w] == j) wl[w] = k;
+        weighted_last = weighted;
+        ++k;
+    }
+    for (int j = k; j < d.nd; ++j) {
+        d.dim[j] = 1;
+        d.sstr[j] = d.dstr[j] = 0;
+    }
+    d.nd = k;
+    d.wleg[0] = wl[0];
+    d.wleg[1] = wl[1];
+}
+
+// Reciprocals for the kernel's divisions: with s = ceil(log2 dim) >= 1 and
+// m = ceil(2^(31+s) / dim) < 2^32, floor(n m / 2^(31+s)) = floor(n / dim) for
+// every n < 2^31 (m dim exceeds 2^(31+s) by less than dim <= 2^s).
+static void set_reciprocals(CopyDesc& d) {
+    int64_t so = 0, dof = 0;
+    for (int j = 0; j < d.nd; ++j) {
+        int s = 1;
+        while (((int64_t)1 << s) < d.dim[j]) ++s;
+        d.sh[j] = s - 1;
+        d.mul[j] = (uint32_t)((((uint64_t)1 << (31 + s)) + d.dim[j] - 1) / d.dim[j]);
+        so += (int64_t)(d.dim[j] - 1) * d.sstr[j];
+        dof += (int64_t)(d.dim[j] - 1) * d.dstr[j];
+    }
+    d.wide = so >= ((int64_t)1 << 31) || dof >= ((int64_t)1 << 31);
+}
+
 // Sub-blocks whose source- and destination-contiguous dims differ (and are
 // both long enough) go to the tiled transpose; the rest to the element copy.
 static void issue_copies(Ctx& ctx, const std::vector<CopyDesc>& descs, int64_t total) {
@@ -237,7 +284,9 @@ static void issue_copies(Ctx& ctx, const std::vector<CopyDesc>& descs, int64_t t
     std::vector<CopyDesc> elem;
     std::vector<TransDesc> tr;
     int64_t estart = 0, eelems = 0, tiles = 0, telems = 0;
-    for (const CopyDesc& d : descs) {
+    for (CopyDesc d : descs) {
+        const bool weighted = d.w[0] || d.w[1];
+        merge_dims(d);
         int s0 = -1, d0 = -1;
         for (int j = 0; j < d.nd; ++j) {
             if (d.dim[j] <= 1) continue;
@@ -246,7 +295,6 @@ static void issue_copies(Ctx& ctx, const std::vector<CopyDesc>& descs, int64_t t
         }
         int64_t cnt = 1;
         for (int j = 0; j < d.nd; ++j) cnt *= d.dim[j];
-        const bool weighted = d.wleg[0] >= 0 || d.wleg[1] >= 0;
         if (!weighted && s0 >= 0 && d0 >= 0 && s0 != d0 && d.dim[s0] >= 8 && d.dim[d0] >= 8 &&
             d.nd - 2 <= TR_BATCH) {
             TransDesc t;
@@ -281,11 +329,11 @@ static void issue_copies(Ctx& ctx, const std::vector<CopyDesc>& descs, int64_t t
             tr.push_back(t);
         } else {
             TNR_REQUIRE(cnt < ((int64_t)1 << 31), TNR_ERR_INTERNAL, "copy job too large");
-            CopyDesc e = d;
-            e.start = estart;              // in 4096-element chunks
-            estart += (cnt + 4095) / 4096;
+            set_reciprocals(d);
+            d.start = estart;
+            estart += (cnt + COPY_CHUNK - 1) / COPY_CHUNK;
             eelems += cnt;
-            elem.push_back(e);
+            elem.push_back(d);
         }
     }
     (void)total;

@@ -14,10 +14,15 @@ struct CopyDesc {
     int64_t sstr[MAXLEG];         // src stride per dst-ordered dim
     int64_t dstr[MAXLEG];         // dst stride per dst-ordered dim
     int32_t dim[MAXLEG];          // extents (dst order)
+    // n / dim = umulhi(n, mul) >> sh for 0 <= n < 2^31 (all dims but the last)
+    uint32_t mul[MAXLEG];
+    int32_t sh[MAXLEG];
     int32_t nd;                   // number of dims
     int32_t wleg[2];              // dims (dst order) carrying weights, -1 = none
-    int64_t start;                // prefix sum of 4096-element chunks
+    int32_t wide;                 // an offset inside the job exceeds 31 bits
+    int64_t start;                // prefix sum of COPY_CHUNK-element chunks
 };
+constexpr int COPY_CHUNK = 1024;
 
 // Tiled transpose job: a sub-block whose source-contiguous dim (extent n0,
 // source stride 1, destination stride ds0) differs from its

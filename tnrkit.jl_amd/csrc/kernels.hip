@@ -32,87 +32,86 @@ __device__ __forceinline__ gmut_double* as_global(double* p) { return (gmut_doub
 typedef double dbl4 __attribute__((ext_vector_type(4)));
 typedef float flt4 __attribute__((ext_vector_type(4)));
 
-// ------------------------------------------------------------------ helpers
-__device__ __forceinline__ int find_desc_copy(const CopyDesc* d, int n, int64_t e) {
-    int lo = 0, hi = n - 1;
-    while (lo < hi) {
-        int mid = (lo + hi + 1) >> 1;
-        if (d[mid].start <= e) lo = mid; else hi = mid - 1;
-    }
-    return lo;
-}
-
 // ------------------------------------------------------------------ permute
 // dst[sum i_k dstr_k] = src[sum i_k sstr_k] * w0[i_wleg0] * w1[i_wleg1]
-// One chunk of COPY_CHUNK consecutive elements (destination order) of one
-// job per workgroup iteration: the job is looked up once per chunk, and the
-// index decomposition runs in 32-bit arithmetic (a job holds < 2^31
-// elements; checked on the host).  Each thread decodes COPY_GROUP elements,
-// issues their loads together, then scales and stores them, so that many
-// loads are in flight per thread.
-constexpr int COPY_CHUNK = 4096;
-constexpr int COPY_GROUP = 8;
+// One chunk of COPY_CHUNK consecutive elements (destination order) of one job
+// per workgroup iteration.  What bounds it is decoding the index: the host
+// merges dims that stay neighbours, divisions are multiplications by
+// precomputed reciprocals, offsets take 32 bits where they fit, and the code
+// is unrolled for the number of dims left.  Four elements a thread, whose loads
+// are issued together: small jobs spread over more CUs than with eight or
+// sixteen.  A wave finds its job 64 entries at a time.
+template <int ND, class I>
+__device__ __forceinline__ void copy_chunk(const CopyDesc& D, uint32_t base, int t) {
+    constexpr int G = COPY_CHUNK / 256;
+    const int ndim = D.nd;
+    uint32_t cnt = 1;
+#pragma unroll
+    for (int q = 0; q < ND; ++q) cnt *= q < ndim ? (uint32_t)D.dim[q] : 1u;
+    gconst_double* src = as_global(D.src);
+    gmut_double* dst = as_global(D.dst);
+    uint32_t r[G], iw0[G], iw1[G];
+    I so[G], dof[G];
+    bool ok[G];
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+        r[g] = base + (uint32_t)(t + 256 * g);
+        ok[g] = r[g] < cnt;
+        if (!ok[g]) r[g] = 0;   // element 0: a valid address, not stored
+        so[g] = dof[g] = 0;
+        iw0[g] = iw1[g] = 0;
+    }
+#pragma unroll
+    for (int q = 0; q < ND; ++q) {
+        if (q >= ndim) continue;
+        const uint32_t dim = (uint32_t)D.dim[q], mul = D.mul[q];
+        const int sh = D.sh[q];
+        const I ss = (I)D.sstr[q], ds = (I)D.dstr[q];
+        const bool last = q + 1 == ndim, w0 = D.wleg[0] == q, w1 = D.wleg[1] == q;
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            const uint32_t n = last ? 0u : __umulhi(r[g], mul) >> sh;
+            const uint32_t i = r[g] - n * dim;
+            r[g] = n;
+            so[g] += (I)i * ss;
+            dof[g] += (I)i * ds;
+            if (w0) iw0[g] = i;
+            if (w1) iw1[g] = i;
+        }
+    }
+    double v[G];
+#pragma unroll
+    for (int g = 0; g < G; ++g) v[g] = src[so[g]];
+    if (D.w[0])
+#pragma unroll
+        for (int g = 0; g < G; ++g) v[g] *= as_global(D.w[0])[iw0[g]];
+    if (D.w[1])
+#pragma unroll
+        for (int g = 0; g < G; ++g) v[g] *= as_global(D.w[1])[iw1[g]];
+#pragma unroll
+    for (int g = 0; g < G; ++g)
+        if (ok[g]) dst[dof[g]] = v[g];
+}
 
 __global__ __launch_bounds__(256) void k_copy(const CopyDesc* __restrict__ descs, int nd,
                                               int64_t chunks) {
-    const int t = threadIdx.x;
+    const int t = threadIdx.x, lane = t & 63;
     for (int64_t c = blockIdx.x; c < chunks; c += gridDim.x) {
-        int lo = 0, hi = nd - 1;
-        while (lo < hi) {
-            const int mid = (lo + hi + 1) >> 1;
-            if (descs[mid].start <= c) lo = mid; else hi = mid - 1;
+        // the last job that starts at or before chunk c
+        int lo = 0, n = nd;
+        while (n > 1) {
+            const int step = (n + 63) / 64, at = lane * step;
+            const bool le = at < n && descs[lo + min(at, n - 1)].start <= c;
+            const int k = __builtin_amdgcn_readfirstlane(__popcll(__ballot(le))) - 1;
+            lo += k * step;
+            n = min(step, n - k * step);
         }
         const CopyDesc& D = descs[lo];
-        const int ndim = D.nd;
-        uint32_t dim[MAXLEG];
-        uint32_t cnt = 1;
-#pragma unroll
-        for (int q = 0; q < MAXLEG; ++q) {
-            dim[q] = q < ndim ? (uint32_t)D.dim[q] : 1u;
-            cnt *= dim[q];
-        }
         const uint32_t base = (uint32_t)(c - D.start) * COPY_CHUNK;
-        const int wl0 = D.wleg[0], wl1 = D.wleg[1];
-        gconst_double* src = as_global(D.src);
-        gmut_double* dst = as_global(D.dst);
-        for (int u0 = 0; u0 < COPY_CHUNK / 256; u0 += COPY_GROUP) {
-            if (base + (uint32_t)(256 * u0) >= cnt) break;
-            int64_t so[COPY_GROUP], dof[COPY_GROUP];
-            uint32_t iw0[COPY_GROUP], iw1[COPY_GROUP];
-            bool ok[COPY_GROUP];
-#pragma unroll
-            for (int g = 0; g < COPY_GROUP; ++g) {
-                uint32_t r = base + (uint32_t)(t + 256 * (u0 + g));
-                ok[g] = r < cnt;
-                if (!ok[g]) r = 0;          // element 0: a valid address, not stored
-                so[g] = 0;
-                dof[g] = 0;
-                iw0[g] = 0;
-                iw1[g] = 0;
-#pragma unroll
-                for (int q = 0; q < MAXLEG; ++q) {
-                    if (q < ndim) {
-                        const uint32_t nq = r / dim[q];
-                        const uint32_t iq = r - nq * dim[q];
-                        r = nq;
-                        so[g] += (int64_t)iq * D.sstr[q];
-                        dof[g] += (int64_t)iq * D.dstr[q];
-                        if (q == wl0) iw0[g] = iq;
-                        if (q == wl1) iw1[g] = iq;
-                    }
-                }
-            }
-            double v[COPY_GROUP];
-#pragma unroll
-            for (int g = 0; g < COPY_GROUP; ++g) v[g] = src[so[g]];
-#pragma unroll
-            for (int g = 0; g < COPY_GROUP; ++g) {
-                double x = v[g];
-                if (wl0 >= 0) x *= D.w[0][iw0[g]];
-                if (wl1 >= 0) x *= D.w[1][iw1[g]];
-                if (ok[g]) dst[dof[g]] = x;
-            }
-        }
+        if (D.wide) copy_chunk<MAXLEG, int64_t>(D, base, t);
+        else if (D.nd <= 2) copy_chunk<2, uint32_t>(D, base, t);
+        else if (D.nd <= 4) copy_chunk<4, uint32_t>(D, base, t);
+        else copy_chunk<MAXLEG, uint32_t>(D, base, t);
     }
 }
 
