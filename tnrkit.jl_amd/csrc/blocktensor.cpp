@@ -186,8 +186,7 @@ static Layout permuted_layout(const Layout& S, const std::vector<int>& perm, int
 
 // append the sub-block copy descriptors of one permute job
 static void permute_descs(const BT& src, BT& dst, const std::vector<int>& perm, bool conj,
-                          const std::vector<WeightSpec>& ws, std::vector<CopyDesc>& descs,
-                          int64_t& start) {
+                          const std::vector<WeightSpec>& ws, std::vector<CopyDesc>& descs) {
     const Layout& S = src.L;
     const int n = S.nleg, N = S.N;
     TNR_REQUIRE(ws.size() <= 2, TNR_ERR_INTERNAL, "at most two weighted legs");
@@ -204,12 +203,10 @@ static void permute_descs(const BT& src, BT& dst, const std::vector<int>& perm, 
         d.src = src.d() + sbase;
         d.dst = dst.d() + dbase;
         d.nd = n;
-        int64_t cnt = 1;
         for (int j = 0; j < n; ++j) {
             d.dim[j] = S.legs[perm[j]].d[q[perm[j]]];
             d.sstr[j] = ss[perm[j]];
             d.dstr[j] = ds[j];
-            cnt *= d.dim[j];
         }
         // every access of the job must stay inside both tensors
         int64_t smax = sbase, dmax = dbase;
@@ -224,8 +221,6 @@ static void permute_descs(const BT& src, BT& dst, const std::vector<int>& perm, 
             d.wleg[w] = inv[ws[w].leg];
             d.w[w] = ws[w].w.w + ws[w].w.off[q[ws[w].leg]];
         }
-        d.start = start;
-        start += cnt;
         descs.push_back(d);
     });
 }
@@ -279,11 +274,18 @@ static void set_reciprocals(CopyDesc& d) {
 
 // Sub-blocks whose source- and destination-contiguous dims differ (and are
 // both long enough) go to the tiled transpose; the rest to the element copy.
-static void issue_copies(Ctx& ctx, const std::vector<CopyDesc>& descs, int64_t total) {
-    if (total <= 0 || descs.empty()) return;
+struct CopyPlan {
     std::vector<CopyDesc> elem;
     std::vector<TransDesc> tr;
     int64_t estart = 0, eelems = 0, tiles = 0, telems = 0;
+    size_t o_elem = 0, o_tr = 0;
+};
+
+static CopyPlan copy_plan(const std::vector<CopyDesc>& descs, DescArena& arena) {
+    CopyPlan P;
+    std::vector<CopyDesc>& elem = P.elem;
+    std::vector<TransDesc>& tr = P.tr;
+    int64_t &estart = P.estart, &eelems = P.eelems, &tiles = P.tiles, &telems = P.telems;
     for (CopyDesc d : descs) {
         const bool weighted = d.w[0] || d.w[1];
         merge_dims(d);
@@ -336,27 +338,35 @@ static void issue_copies(Ctx& ctx, const std::vector<CopyDesc>& descs, int64_t t
             elem.push_back(d);
         }
     }
-    (void)total;
-    if (!tr.empty()) {
-        TransDesc* dt = ctx.stage->put(ctx.stream, tr);
-        launch_transpose(ctx.stream, dt, (int)tr.size(), tiles, telems);
+    P.o_tr = arena.add(tr);
+    P.o_elem = arena.add(elem);
+    return P;
+}
+
+static void copy_issue(Ctx& ctx, const CopyPlan& P, const DescArena& arena) {
+    if (!P.tr.empty())
+        launch_transpose(ctx.stream, arena.at<TransDesc>(P.o_tr), (int)P.tr.size(), P.tiles, P.telems);
+    if (!P.elem.empty())
+        launch_copy(ctx.stream, arena.at<CopyDesc>(P.o_elem), (int)P.elem.size(), P.estart, P.eelems);
+}
+
+// The permuted tensors' storage, and the copies that fill it.
+static CopyPlan permute_plan(Ctx& ctx, const std::vector<PermJob>& jobs, std::vector<BT>& out, DescArena& arena) {
+    out.reserve(jobs.size());
+    std::vector<CopyDesc> descs;
+    for (const PermJob& j : jobs) {
+        out.emplace_back(ctx, permuted_layout(j.src->L, j.perm, j.ncod, j.conj));
+        permute_descs(*j.src, out.back(), j.perm, j.conj, j.ws, descs);
     }
-    if (!elem.empty()) {
-        CopyDesc* dd = ctx.stage->put(ctx.stream, elem);
-        launch_copy(ctx.stream, dd, (int)elem.size(), estart, eelems);
-    }
+    return copy_plan(descs, arena);
 }
 
 std::vector<BT> permute_many(Ctx& ctx, const std::vector<PermJob>& jobs) {
     std::vector<BT> out;
-    out.reserve(jobs.size());
-    std::vector<CopyDesc> descs;
-    int64_t start = 0;
-    for (const PermJob& j : jobs) {
-        out.emplace_back(ctx, permuted_layout(j.src->L, j.perm, j.ncod, j.conj));
-        permute_descs(*j.src, out.back(), j.perm, j.conj, j.ws, descs, start);
-    }
-    issue_copies(ctx, descs, start);
+    DescArena arena;
+    const CopyPlan P = permute_plan(ctx, jobs, out, arena);
+    arena.commit(ctx);
+    copy_issue(ctx, P, arena);
     return out;
 }
 
@@ -778,7 +788,11 @@ std::vector<BT> contract_many(Ctx& ctx, const std::vector<ContractJob>& jobs) {
             P.pc.push_back(pos);
         }
     }
-    std::vector<BT> ops = permute_many(ctx, pj);
+    // operand copies, products and output copies are planned before the first
+    // of them is issued: one upload for all their descriptors
+    DescArena arena;
+    std::vector<BT> ops;
+    const CopyPlan pin = permute_plan(ctx, pj, ops, arena);
     std::vector<BT> Cs;
     Cs.reserve(J);
     std::vector<GemmJob> gj;
@@ -806,7 +820,8 @@ std::vector<BT> contract_many(Ctx& ctx, const std::vector<ContractJob>& jobs) {
             gj.push_back(j);
         }
     }
-    gemm_grouped(ctx, gj, ctx.precision == TNR_PREC_SPLIT32);
+    GemmPlan pg = gemm_plan(ctx, gj, ctx.precision == TNR_PREC_SPLIT32);
+    gemm_stage(pg, arena);
     // output arrangement
     std::vector<PermJob> fj;
     std::vector<int> fidx(J, -1);
@@ -816,7 +831,13 @@ std::vector<BT> contract_many(Ctx& ctx, const std::vector<ContractJob>& jobs) {
         fidx[x] = (int)fj.size();
         fj.push_back(PermJob{&Cs[x], P.pc, jobs[x].out_ncod, false, {}});
     }
-    std::vector<BT> fin = permute_many(ctx, fj);
+    std::vector<BT> fin;
+    const CopyPlan pout = permute_plan(ctx, fj, fin, arena);
+    arena.commit(ctx);
+    gemm_bind(pg, arena);
+    copy_issue(ctx, pin, arena);
+    gemm_issue(ctx, pg);
+    copy_issue(ctx, pout, arena);
     std::vector<BT> out;
     out.reserve(J);
     for (size_t x = 0; x < J; ++x)
@@ -906,9 +927,11 @@ void trace_normalize_many(Ctx& ctx, const std::vector<TraceJob>& jobs) {
         max_size = std::max(max_size, L.size);
     }
     if (probs.empty()) return;
-    TraceDesc* dd = ctx.stage->put(ctx.stream, descs);
-    TraceProb* dp = ctx.stage->put(ctx.stream, probs);
-    launch_trace_normalize(ctx.stream, dd, dp, (int)probs.size(), max_size);
+    DescArena arena;
+    const size_t od = arena.add(descs), op = arena.add(probs);
+    arena.commit(ctx);
+    launch_trace_normalize(ctx.stream, arena.at<TraceDesc>(od), arena.at<TraceProb>(op), (int)probs.size(),
+                           max_size);
 }
 
 // ------------------------------------------------------ linear combinations
@@ -938,18 +961,28 @@ void lincomb_many(Ctx& ctx, const std::vector<LinJob>& jobs) {
 }
 
 // ------------------------------------------------------------------ gather
-void gather_many(Ctx& ctx, std::vector<GatherDesc> descs) {
-    int64_t start = 0;
-    std::vector<GatherDesc> d;
-    for (auto& g : descs) {
-        if (g.rows <= 0 || g.cols <= 0) continue;
-        g.start = start;
-        start += (int64_t)g.rows * g.cols;
-        d.push_back(g);
+GatherPlan gather_plan(const std::vector<GatherDesc>& descs, DescArena& arena) {
+    GatherPlan P;
+    for (const GatherDesc& x : descs) {
+        if (x.rows <= 0 || x.cols <= 0) continue;
+        P.d.push_back(x);
+        P.d.back().start = P.total;
+        P.total += (int64_t)x.rows * x.cols;
     }
-    if (d.empty()) return;
-    GatherDesc* dd = ctx.stage->put(ctx.stream, d);
-    launch_gather(ctx.stream, dd, (int)d.size(), start);
+    P.off = arena.add(P.d);
+    return P;
+}
+
+void gather_issue(Ctx& ctx, const GatherPlan& P, const DescArena& arena) {
+    if (!P.d.empty()) launch_gather(ctx.stream, arena.at<GatherDesc>(P.off), (int)P.d.size(), P.total);
+}
+
+void gather_many(Ctx& ctx, const std::vector<GatherDesc>& descs) {
+    DescArena arena;
+    const GatherPlan P = gather_plan(descs, arena);
+    if (P.d.empty()) return;
+    arena.commit(ctx);
+    gather_issue(ctx, P, arena);
 }
 
 void readback_vectors(Ctx& ctx, const std::vector<const double*>& src,
@@ -960,14 +993,15 @@ void readback_vectors(Ctx& ctx, const std::vector<const double*>& src,
         total += (size_t)std::max(cnt[p], 0);
     }
     if (!total) return;
-    Buf packed(&ctx.pool, total * sizeof(double));
+    // (the kernel writes pinned host memory)
+    double* h = static_cast<double*>(ctx.bounce(total * sizeof(double)));
     std::vector<GatherDesc> gd;
     size_t o = 0;
     for (size_t p = 0; p < src.size(); ++p) {
         if (cnt[p] <= 0) continue;
         GatherDesc g{};
         g.in = src[p];
-        g.out = packed.d() + o;
+        g.out = h + o;
         g.rows = cnt[p];
         g.cols = 1;
         g.ldi = cnt[p];
@@ -976,12 +1010,11 @@ void readback_vectors(Ctx& ctx, const std::vector<const double*>& src,
         o += (size_t)cnt[p];
     }
     gather_many(ctx, gd);
-    std::vector<double> h(total);
-    ctx.fetch(h.data(), packed.d(), total * sizeof(double));
+    ctx.sync();
     o = 0;
     for (size_t p = 0; p < src.size(); ++p) {
         if (cnt[p] <= 0) continue;
-        std::copy(h.begin() + o, h.begin() + o + cnt[p], dst[p]->begin());
+        std::copy(h + o, h + o + cnt[p], dst[p]->begin());
         o += (size_t)cnt[p];
     }
 }

@@ -169,6 +169,15 @@ class DescArena {
     char* base_ = nullptr;
 };
 
+// A grouped gather to be uploaded with other descriptors.
+struct GatherPlan {
+    std::vector<GatherDesc> d;
+    int64_t total = 0;
+    size_t off = 0;
+};
+GatherPlan gather_plan(const std::vector<GatherDesc>& descs, DescArena& arena);
+void gather_issue(Ctx& ctx, const GatherPlan& P, const DescArena& arena);
+
 // A grouped GEMM prepared once and issued many times.
 struct GemmPlan {
     std::vector<GemmDesc> descs, red;
@@ -216,7 +225,7 @@ void lincomb_many(Ctx& ctx, const std::vector<LinJob>& jobs);
 void trace_normalize_many(Ctx& ctx, const std::vector<TraceJob>& jobs);
 
 // Grouped strided matrix copies with optional row/column weights.
-void gather_many(Ctx& ctx, std::vector<GatherDesc> descs);
+void gather_many(Ctx& ctx, const std::vector<GatherDesc>& descs);
 // cnt[p] doubles at device src[p] into *dst[p]: packed on the device, one
 // copy to the host, one synchronisation
 void readback_vectors(Ctx& ctx, const std::vector<const double*>& src,

@@ -100,8 +100,12 @@ class Staging {
     template <class T> T* put(hipStream_t st, const std::vector<T>& v) {
         return static_cast<T*>(put(st, v.data(), v.size() * sizeof(T)));
     }
+    // the same into device memory of the caller's
+    void put_to(hipStream_t st, void* dst, const void* src, size_t bytes);
 
   private:
+    size_t reserve(hipStream_t st, size_t bytes);   // offset of a free chunk
+    void put_at(hipStream_t st, size_t at, void* dst, const void* src, size_t bytes);
     void alloc(size_t bytes);
     void release();
     char* host_ = nullptr;
@@ -126,6 +130,9 @@ struct Ctx {
     // device -> host copy that waits for the stream (through a pinned
     // bounce buffer, so the DMA engine writes host memory directly)
     void fetch(void* dst, const void* src, size_t bytes);
+    // at least `bytes` of that buffer, for kernels to write to; read it after
+    // sync()
+    void* bounce(size_t bytes);
 
   private:
     void* bounce_ = nullptr;

@@ -83,7 +83,7 @@ Staging::Staging(size_t bytes) { alloc(bytes); }
 
 Staging::~Staging() { release(); }
 
-void* Staging::put(hipStream_t st, const void* src, size_t bytes) {
+size_t Staging::reserve(hipStream_t st, size_t bytes) {
     size_t need = (bytes + 255) & ~size_t(255);
     if (need == 0) need = 256;
     if (need > cap_) {
@@ -98,14 +98,25 @@ void* Staging::put(hipStream_t st, const void* src, size_t bytes) {
         TNR_HIP(hipStreamSynchronize(st));
         head_ = 0;
     }
-    char* h = host_ + head_;
-    char* d = dev_ + head_;
+    const size_t at = head_;
     head_ += need;
-    if (bytes) {
-        std::memcpy(h, src, bytes);
-        TNR_HIP(hipMemcpyAsync(d, h, bytes, hipMemcpyHostToDevice, st));
-    }
-    return d;
+    return at;
+}
+
+void* Staging::put(hipStream_t st, const void* src, size_t bytes) {
+    const size_t at = reserve(st, bytes);
+    put_at(st, at, dev_ + at, src, bytes);
+    return dev_ + at;
+}
+
+void Staging::put_to(hipStream_t st, void* dst, const void* src, size_t bytes) {
+    put_at(st, reserve(st, bytes), dst, src, bytes);
+}
+
+void Staging::put_at(hipStream_t st, size_t at, void* dst, const void* src, size_t bytes) {
+    if (!bytes) return;
+    std::memcpy(host_ + at, src, bytes);
+    TNR_HIP(hipMemcpyAsync(dst, host_ + at, bytes, hipMemcpyHostToDevice, st));
 }
 
 // -------------------------------------------------------------------- Ctx
@@ -152,8 +163,7 @@ void Ctx::ensure_stream() {
     if (!stream) TNR_HIP(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
 }
 
-void Ctx::fetch(void* dst, const void* src, size_t bytes) {
-    if (!bytes) return;
+void* Ctx::bounce(size_t bytes) {
     if (bytes > bounce_cap_) {
         TNR_HIP(hipStreamSynchronize(stream));
         if (bounce_) TNR_HIP(hipHostFree(bounce_));
@@ -163,9 +173,15 @@ void Ctx::fetch(void* dst, const void* src, size_t bytes) {
         TNR_HIP(hipHostMalloc(&bounce_, cap, hipHostMallocDefault));
         bounce_cap_ = cap;
     }
-    TNR_HIP(hipMemcpyAsync(bounce_, src, bytes, hipMemcpyDeviceToHost, stream));
+    return bounce_;
+}
+
+void Ctx::fetch(void* dst, const void* src, size_t bytes) {
+    if (!bytes) return;
+    void* h = bounce(bytes);
+    TNR_HIP(hipMemcpyAsync(h, src, bytes, hipMemcpyDeviceToHost, stream));
     TNR_HIP(hipStreamSynchronize(stream));
-    std::memcpy(dst, bounce_, bytes);
+    std::memcpy(dst, h, bytes);
 }
 
 }  // namespace tnr

@@ -47,11 +47,7 @@ std::vector<BondVec> make_bonds(Ctx& ctx, const std::vector<int>& Ns,
         all.insert(all.end(), vals[b]->begin(), vals[b]->end());
     }
     auto store = std::make_shared<Buf>(&ctx.pool, std::max<size_t>(1, all.size()) * sizeof(double));
-    if (!all.empty()) {
-        void* tmp = ctx.stage->put(ctx.stream, all.data(), all.size() * sizeof(double));
-        TNR_HIP(hipMemcpyAsync(store->d(), tmp, all.size() * sizeof(double),
-                               hipMemcpyDeviceToDevice, ctx.stream));
-    }
+    ctx.stage->put_to(ctx.stream, store->d(), all.data(), all.size() * sizeof(double));
     for (auto& v : out) v.store = store;
     return out;
 }

@@ -223,27 +223,21 @@ void rr_issue(Ctx& ctx, RRPlan& P, bool first = false, const ConvDesc* conv = nu
     if (!P.chol) launch_colnorm(ctx.stream, P.d_col, (int)P.col.size(), P.lmax, cfg.null_rtol);
 }
 
-void rr_grouped(Ctx& ctx, const std::vector<RR>& jobs, int passes, bool tight = false, bool chol = false) {
-    if (jobs.empty()) return;
-    RRPlan P = rr_plan(ctx, jobs, passes, chol, tight);
-    P.span = chol;
-    DescArena a;
-    rr_stage(P, a);
-    a.commit(ctx);
-    rr_bind(P, a);
-    rr_issue(ctx, P);
-}
-
-void randfill(Ctx& ctx, const std::vector<FillDesc>& fills) {
-    if (fills.empty()) return;
-    std::vector<FillDesc> f(fills);
+// prefix sums of the fills' elements; returns the total
+int64_t fill_starts(std::vector<FillDesc>& f) {
     int64_t start = 0;
     for (auto& x : f) {
         x.start = start;
         start += (int64_t)x.rows * x.cols;
     }
+    return start;
+}
+
+void randfill(Ctx& ctx, std::vector<FillDesc> f) {
+    if (f.empty()) return;
+    const int64_t total = fill_starts(f);
     FillDesc* d = ctx.stage->put(ctx.stream, f);
-    launch_randfill(ctx.stream, d, (int)f.size(), start);
+    launch_randfill(ctx.stream, d, (int)f.size(), total);
 }
 
 // One double per problem, zeroed on the stream: the Jacobi kernels set a
@@ -251,8 +245,7 @@ void randfill(Ctx& ctx, const std::vector<FillDesc>& fills) {
 Buf fail_flags(Ctx& ctx, size_t P) {
     Buf f(&ctx.pool, std::max<size_t>(1, P) * sizeof(double));
     std::vector<double> z(std::max<size_t>(1, P), 0.0);
-    void* a = ctx.stage->put(ctx.stream, z.data(), z.size() * sizeof(double));
-    TNR_HIP(hipMemcpyAsync(f.d(), a, z.size() * sizeof(double), hipMemcpyDeviceToDevice, ctx.stream));
+    ctx.stage->put_to(ctx.stream, f.d(), z.data(), z.size() * sizeof(double));
     return f;
 }
 
@@ -279,25 +272,27 @@ int block_size(int kmax) {
     return std::min(LMAX, std::max(l, kmax + 2 <= LMAX ? kmax + 2 : LMAX));
 }
 
-// Per-call device state of the stopping rule: it, done (ints), prod (double).
+// Per-call device state of the stopping rule: prod (doubles), it, done (ints).
 struct ConvState {
-    Buf ints, prods;
+    Buf state;
     int P = 0;
     ConvState(Ctx& ctx, int P_) : P(P_) {
-        ints = Buf(&ctx.pool, (size_t)2 * P * sizeof(int));
-        prods = Buf(&ctx.pool, (size_t)P * sizeof(double));
-        std::vector<int> zi(2 * P, 0);
-        std::vector<double> one(P, 1.0);
-        void* a = ctx.stage->put(ctx.stream, zi.data(), zi.size() * sizeof(int));
-        void* b = ctx.stage->put(ctx.stream, one.data(), one.size() * sizeof(double));
-        TNR_HIP(hipMemcpyAsync(ints.d(), a, zi.size() * sizeof(int), hipMemcpyDeviceToDevice,
-                               ctx.stream));
-        TNR_HIP(hipMemcpyAsync(prods.d(), b, one.size() * sizeof(double),
-                               hipMemcpyDeviceToDevice, ctx.stream));
+        state = Buf(&ctx.pool, (size_t)2 * P * sizeof(double));
+        std::vector<double> s(2 * P, 0.0);   // (all bits zero: the ints)
+        std::fill(s.begin(), s.begin() + P, 1.0);
+        ctx.stage->put_to(ctx.stream, state.d(), s.data(), s.size() * sizeof(double));
     }
-    int* it(int p) const { return ints.as<int>() + p; }
-    int* done(int p) const { return ints.as<int>() + P + p; }
-    double* prod(int p) const { return prods.d() + p; }
+    int* it(int p) const { return reinterpret_cast<int*>(state.d() + P) + p; }
+    int* done(int p) const { return it(P + p); }
+    double* prod(int p) const { return state.d() + p; }
+    // iterations and accumulated contractions, once the loop has ended
+    void fetch(Ctx& ctx, std::vector<int>& its, std::vector<double>& prods) const {
+        std::vector<double> s(2 * P);
+        ctx.fetch(s.data(), state.d(), s.size() * sizeof(double));
+        prods.assign(s.begin(), s.begin() + P);
+        its.resize(P);
+        std::memcpy(its.data(), s.data() + P, P * sizeof(int));
+    }
 };
 
 // Issue `issue_one` chunk by chunk until the device marks every problem done.
@@ -369,9 +364,7 @@ std::vector<int> wide_rr(Ctx& ctx, const std::vector<WideRR>& jobs, double tol, 
         const int l = jobs[j].l;
         std::vector<double> id((size_t)l * l, 0.0);
         for (int i = 0; i < l; ++i) id[(size_t)i * l + i] = 1.0;
-        void* t = ctx.stage->put(ctx.stream, id.data(), id.size() * sizeof(double));
-        TNR_HIP(hipMemcpyAsync(jobs[j].Wtot, t, id.size() * sizeof(double), hipMemcpyDeviceToDevice,
-                               ctx.stream));
+        ctx.stage->put_to(ctx.stream, jobs[j].Wtot, id.data(), id.size() * sizeof(double));
     }
     std::vector<char> live(J, 1);
     for (int sw = 0;; ++sw) {
@@ -546,8 +539,7 @@ std::vector<int> wide_rr(Ctx& ctx, const std::vector<WideRR>& jobs, double tol, 
                 perm.push_back(w);
             }
         }
-        void* t = ctx.stage->put(ctx.stream, sorted_all.data() + soff[j], (size_t)R.l * 8);
-        TNR_HIP(hipMemcpyAsync(R.sigma, t, (size_t)R.l * 8, hipMemcpyDeviceToDevice, ctx.stream));
+        ctx.stage->put_to(ctx.stream, R.sigma, sorted_all.data() + soff[j], (size_t)R.l * 8);
     }
     gather_many(ctx, perm);
     return status;
@@ -789,8 +781,7 @@ void eigh_wide(Ctx& ctx, const std::vector<EighIn>& in, const std::vector<int>& 
             if (d < 0.0) hs[c] = -hs[c];
         }
         o.lam = Buf(&ctx.pool, (size_t)x.l * 8);
-        void* t = ctx.stage->put(ctx.stream, hs.data(), (size_t)x.l * 8);
-        TNR_HIP(hipMemcpyAsync(o.lam.d(), t, (size_t)x.l * 8, hipMemcpyDeviceToDevice, ctx.stream));
+        ctx.stage->put_to(ctx.stream, o.lam.d(), hs.data(), (size_t)x.l * 8);
         o.U = Buf(&ctx.pool, (size_t)s.n * x.l * 8);
         o.ncols = x.l;
         o.direct = whole;     // all n eigenvalues: the truncation error is exact
@@ -847,9 +838,17 @@ void svd_grouped(Ctx& ctx, const std::vector<SvdIn>& in, std::vector<SvdOut>& ou
             r.fail = failv.d() + direct[i];
             (l >= kPrecondFrom ? rp : rr).push_back(r);
         }
-        gather_many(ctx, gd);
-        rr_grouped(ctx, rr, 2);
-        rr_grouped(ctx, rp, 3);
+        DescArena a;
+        const GatherPlan pg = gather_plan(gd, a);
+        RRPlan p2 = rr_plan(ctx, rr, 2), p3 = rr_plan(ctx, rp, 3);
+        rr_stage(p2, a);
+        rr_stage(p3, a);
+        a.commit(ctx);
+        rr_bind(p2, a);
+        rr_bind(p3, a);
+        gather_issue(ctx, pg, a);
+        if (!rr.empty()) rr_issue(ctx, p2);
+        if (!rp.empty()) rr_issue(ctx, p3);
         for (size_t i = 0; i < direct.size(); ++i) {
             const SvdIn& s = in[direct[i]];
             SvdOut& o = out[direct[i]];
@@ -931,7 +930,6 @@ void svd_grouped(Ctx& ctx, const std::vector<SvdIn>& in, std::vector<SvdOut>& ou
                             x.sw.as<int>(), x.Wt.d(), x.U.d(), s.m, x.sigU.d(), nullptr, fl});
             jV.push_back(GemmJob{x.V.d(), x.Wt.d(), x.Z.d(), s.n, l, l, s.n, l, s.n, 0, 0});
         }
-        randfill(ctx, fills);
         // the random start block is not orthonormalised: the first
         // Rayleigh-Ritz step on Y = M V builds an orthonormal basis of its span
         GemmPlan pMV = gemm_plan(ctx, jMV), pMtU = gemm_plan(ctx, jMtU);
@@ -939,18 +937,26 @@ void svd_grouped(Ctx& ctx, const std::vector<SvdIn>& in, std::vector<SvdOut>& ou
         // needs (pivoted Cholesky QR); Z side: Rayleigh-Ritz, whose values
         // drive the stopping rule
         RRPlan pY = rr_plan(ctx, rY, 1, cfg.cholqr_y), pZ = rr_plan(ctx, rZ, 1, cfg.cholqr_z);
+        // the loop orthonormalises only to its looser Jacobi threshold: V is
+        // rebuilt at full accuracy before the final extraction relies on
+        // V^T V = I.  Its last rotated Z has columns orthogonal to that
+        // threshold, so one pass at the final threshold does what the second
+        // pass of a two-pass step does.
+        const int vpass = cfg.cholqr_z ? cfg.rv_passes : 1;
+        RRPlan pV = rr_plan(ctx, rV, vpass, false, vpass == 1);
+        RRPlan pF = rr_plan(ctx, rF, cfg.rf_passes, false, cfg.rf_passes == 1);
+        GemmPlan pjF = gemm_plan(ctx, jF), pjV = gemm_plan(ctx, jV);
+        // all of the solve's descriptors in one upload
+        const int64_t nfill = fill_starts(fills);
         DescArena a;
-        gemm_stage(pMV, a);
-        gemm_stage(pMtU, a);
-        rr_stage(pY, a);
-        rr_stage(pZ, a);
-        const size_t o_conv = a.add(conv);
+        for (GemmPlan* g : {&pMV, &pMtU, &pjF, &pjV}) gemm_stage(*g, a);
+        for (RRPlan* r : {&pY, &pZ, &pV, &pF}) rr_stage(*r, a);
+        const size_t o_conv = a.add(conv), o_fill = a.add(fills);
         a.commit(ctx);
-        gemm_bind(pMV, a);
-        gemm_bind(pMtU, a);
-        rr_bind(pY, a);
-        rr_bind(pZ, a);
+        for (GemmPlan* g : {&pMV, &pMtU, &pjF, &pjV}) gemm_bind(*g, a);
+        for (RRPlan* r : {&pY, &pZ, &pV, &pF}) rr_bind(*r, a);
         const ConvDesc* d_conv = a.at<ConvDesc>(o_conv);
+        launch_randfill(ctx.stream, a.at<FillDesc>(o_fill), (int)fills.size(), nfill);
         iterate(ctx, cs, [&](int it) {
             gemm_issue(ctx, pMV);
             rr_issue(ctx, pY, it == 0);
@@ -958,20 +964,13 @@ void svd_grouped(Ctx& ctx, const std::vector<SvdIn>& in, std::vector<SvdOut>& ou
             rr_issue(ctx, pZ, it == 0, cfg.cholqr_z ? d_conv : nullptr);
             if (!cfg.cholqr_z) launch_conv(ctx.stream, d_conv, P, conv_rule(cfg));
         });
-        // the loop orthonormalises only to its looser Jacobi threshold: V is
-        // rebuilt at full accuracy before the final extraction relies on
-        // V^T V = I.  Its last rotated Z has columns orthogonal to that
-        // threshold, so one pass at the final threshold does what the second
-        // pass of a two-pass step does.
-        if (cfg.cholqr_z) rr_grouped(ctx, rV, cfg.rv_passes, cfg.rv_passes == 1);
-        else rr_grouped(ctx, rV, 1, true);
-        gemm_grouped(ctx, jF);
-        rr_grouped(ctx, rF, cfg.rf_passes, cfg.rf_passes == 1);
-        gemm_grouped(ctx, jV);
-        std::vector<int> its(P);
-        std::vector<double> prods(P);
-        ctx.fetch(its.data(), cs.it(0), P * sizeof(int));
-        ctx.fetch(prods.data(), cs.prod(0), P * sizeof(double));
+        rr_issue(ctx, pV);
+        gemm_issue(ctx, pjF);
+        rr_issue(ctx, pF);
+        gemm_issue(ctx, pjV);
+        std::vector<int> its;
+        std::vector<double> prods;
+        cs.fetch(ctx, its, prods);
         std::vector<int> stalled;
         for (int i = 0; i < P; ++i) {
             SvdOut& o = out[iter[i]];
@@ -1101,65 +1100,59 @@ void eigh_grouped(Ctx& ctx, const std::vector<EighIn>& in, std::vector<EighOut>&
             jH.push_back(GemmJob{x.V.d(), x.Y.d(), x.G.d(), l, l, s.n, s.n, s.n, l, 1, 0});
             nmax = std::max(nmax, s.n);
         }
-        ColDesc* dsym = ctx.stage->put(ctx.stream, sym);
-        launch_symmetrize(ctx.stream, dsym, (int)sym.size(), nmax);
-        randfill(ctx, fills);
         // (random start block used as is, see svd_grouped)
         GemmPlan pMV = gemm_plan(ctx, jMV);
         RRPlan pY = rr_plan(ctx, rY, 1, cfg.cholqr_eigh);
         pY.span = cfg.cholqr_eigh;
+        // V at full orthonormality from the loop's last rotated Y = M V W
+        // (the loop uses a looser Jacobi threshold; one pass at the final
+        // threshold, as in svd_grouped) or from the last Cholesky QR basis,
+        // then the Ritz pairs: H = V^T (M V), eigendecompose, U = V W
+        RRPlan pV = rr_plan(ctx, rV, 1, cfg.cholqr_eigh, !cfg.cholqr_eigh);
+        pV.span = cfg.cholqr_eigh;
+        std::vector<JacobiDesc> jd;
+        std::vector<GemmJob> jU;
+        int lmax = 0;
+        for (int i = 0; i < P; ++i) {
+            const EighIn& s = in[iter[i]];
+            IW& x = w[i];
+            EighOut& o = out[iter[i]];
+            o.lam = Buf(&ctx.pool, (size_t)x.l * 8);
+            o.U = Buf(&ctx.pool, (size_t)s.n * x.l * 8);
+            o.ncols = x.l;
+            o.direct = false;
+            jd.push_back(JacobiDesc{x.G.d(), x.W.d(), o.lam.d(), x.sw.as<int>(), x.l, x.l, x.l, nullptr,
+                                    failv.d() + iter[i]});
+            jU.push_back(GemmJob{x.V.d(), x.W.d(), o.U.d(), s.n, x.l, x.l, s.n, x.l, s.n, 0, 0});
+            lmax = std::max(lmax, x.l);
+        }
+        GemmPlan pQ = gemm_plan(ctx, jQ), pjF = gemm_plan(ctx, jF), pH = gemm_plan(ctx, jH), pU = gemm_plan(ctx, jU);
+        // all of the solve's descriptors in one upload
+        const int64_t nfill = fill_starts(fills);
         DescArena a;
-        gemm_stage(pMV, a);
-        rr_stage(pY, a);
-        const size_t o_conv = a.add(conv);
+        for (GemmPlan* g : {&pMV, &pQ, &pjF, &pH, &pU}) gemm_stage(*g, a);
+        for (RRPlan* r : {&pY, &pV}) rr_stage(*r, a);
+        const size_t o_conv = a.add(conv), o_fill = a.add(fills), o_sym = a.add(sym), o_jd = a.add(jd);
         a.commit(ctx);
-        gemm_bind(pMV, a);
-        rr_bind(pY, a);
+        for (GemmPlan* g : {&pMV, &pQ, &pjF, &pH, &pU}) gemm_bind(*g, a);
+        for (RRPlan* r : {&pY, &pV}) rr_bind(*r, a);
         const ConvDesc* d_conv = a.at<ConvDesc>(o_conv);
+        launch_symmetrize(ctx.stream, a.at<ColDesc>(o_sym), (int)sym.size(), nmax);
+        launch_randfill(ctx.stream, a.at<FillDesc>(o_fill), (int)fills.size(), nfill);
         iterate(ctx, cs, [&](int it) {
             gemm_issue(ctx, pMV);
             rr_issue(ctx, pY, it == 0, cfg.cholqr_eigh ? d_conv : nullptr);
             if (!cfg.cholqr_eigh) launch_conv(ctx.stream, d_conv, P, conv_rule(cfg));
         });
-        // V at full orthonormality from the loop's last rotated Y = M V W
-        // (the loop uses a looser Jacobi threshold; one pass at the final
-        // threshold, as in svd_grouped) or from the last Cholesky QR basis
-        if (cfg.cholqr_eigh) {
-            gemm_grouped(ctx, jQ);
-            rr_grouped(ctx, rV, 1, false, true);
-        } else {
-            rr_grouped(ctx, rV, 1, true);
-        }
-        // Ritz pairs: H = V^T (M V), eigendecompose, U = V W
-        gemm_grouped(ctx, jF);
-        gemm_grouped(ctx, jH);
-        std::vector<JacobiDesc> jd;
-        int lmax = 0;
-        for (int i = 0; i < P; ++i) {
-            IW& x = w[i];
-            EighOut& o = out[iter[i]];
-            o.lam = Buf(&ctx.pool, (size_t)x.l * 8);
-            jd.push_back(JacobiDesc{x.G.d(), x.W.d(), o.lam.d(), x.sw.as<int>(), x.l, x.l, x.l, nullptr,
-                                    failv.d() + iter[i]});
-            lmax = std::max(lmax, x.l);
-        }
-        JacobiDesc* djd = ctx.stage->put(ctx.stream, jd);
-        launch_jacobi(ctx.stream, djd, (int)jd.size(), lmax, cfg.jacobi_tol, cfg.jacobi_sweeps);
-        std::vector<GemmJob> jU;
-        for (int i = 0; i < P; ++i) {
-            const EighIn& s = in[iter[i]];
-            IW& x = w[i];
-            EighOut& o = out[iter[i]];
-            o.U = Buf(&ctx.pool, (size_t)s.n * x.l * 8);
-            o.ncols = x.l;
-            o.direct = false;
-            jU.push_back(GemmJob{x.V.d(), x.W.d(), o.U.d(), s.n, x.l, x.l, s.n, x.l, s.n, 0, 0});
-        }
-        gemm_grouped(ctx, jU);
-        std::vector<int> its(P);
-        std::vector<double> prods(P);
-        ctx.fetch(its.data(), cs.it(0), P * sizeof(int));
-        ctx.fetch(prods.data(), cs.prod(0), P * sizeof(double));
+        gemm_issue(ctx, pQ);
+        rr_issue(ctx, pV);
+        gemm_issue(ctx, pjF);
+        gemm_issue(ctx, pH);
+        launch_jacobi(ctx.stream, a.at<JacobiDesc>(o_jd), (int)jd.size(), lmax, cfg.jacobi_tol, cfg.jacobi_sweeps);
+        gemm_issue(ctx, pU);
+        std::vector<int> its;
+        std::vector<double> prods;
+        cs.fetch(ctx, its, prods);
         std::vector<int> stalled;
         for (int i = 0; i < P; ++i) {
             out[iter[i]].iters = its[i];
