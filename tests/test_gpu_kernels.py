@@ -290,6 +290,27 @@ def test_svd_cholesky_panel_edges(tk, k, extra):
     assert np.max(np.abs(V.T @ V - np.eye(k))) < 1e-12
 
 
+# Cholesky QR steps that form Y^T Y and Y W themselves: sides around the rule (at
+# most 511 rows, 8960 doubles of padded Y, width 64), one side or both, ragged
+# rows and widths.  Tolerances as above (geometric spectrum, gap 0.82 at k).
+@pytest.mark.parametrize("m,n,k", [
+    (97, 101, 1), (100, 97, 3), (128, 128, 32), (128, 146, 32), (256, 255, 16), (272, 257, 16),
+    (273, 288, 15), (511, 130, 5), (512, 511, 5), (131, 120, 31), (113, 111, 33)])
+def test_svd_fused_cholesky_edges(tk, m, n, k):
+    rng = np.random.default_rng(m + n + k)
+    r = min(m, n)
+    Ua, _ = np.linalg.qr(rng.standard_normal((m, r)))
+    Va, _ = np.linalg.qr(rng.standard_normal((n, r)))
+    M = (Ua * np.exp(-0.2 * np.arange(r))) @ Va.T
+    U, s, V, it = svd(tk, M, k)
+    assert it > 0
+    Ur, sr, Vtr = np.linalg.svd(M, full_matrices=False)
+    assert np.max(np.abs(s - sr[:k])) < 1e-13 * sr[0]
+    assert np.max(np.abs((U * s) @ V.T - (Ur[:, :k] * sr[:k]) @ Vtr[:k])) < 1e-12 * sr[0]
+    assert np.max(np.abs(U.T @ U - np.eye(k))) < 1e-12
+    assert np.max(np.abs(V.T @ V - np.eye(k))) < 1e-12
+
+
 @pytest.mark.parametrize("n,k", [(64, 16), (512, 32), (400, 120)])
 def test_eigh_truncated(tk, n, k):
     rng = np.random.default_rng(n)

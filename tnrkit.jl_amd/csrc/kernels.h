@@ -112,7 +112,19 @@ struct JacobiDesc {
                                   // accumulated rotation, close to the
                                   // identity for a nearly diagonal G) instead
                                   // of ordering by |lambda| descending
+    // Cholesky QR of a small Y (cholqr_fused): G is Y^T Y and U = Y W follows
+    const double* Y = nullptr;
+    double* U = nullptr;
+    int32_t rows = 0, ldy = 0, ldu = 0;
 };
+// k_cholqr's LDS copy of Y, in doubles: columns and rows up to 16, + 2
+__host__ __device__ inline int cholqr_ldy(int rows) { return (rows + 15) / 16 * 16 + 2; }
+constexpr int CQ64 = 64;            // Gram matrices up to this size take the 64-row kernel
+constexpr int CHOLQR_YLDS = 8960;   // 70 KB beside its 68 KB: 128 x 64, 256 x 32, 350 x 16
+__host__ __device__ inline int64_t cholqr_ylds(int rows, int n) { return (int64_t)cholqr_ldy(rows) * ((n + 15) / 16 * 16); }
+inline bool cholqr_fused(int rows, int n) {
+    return n <= CQ64 && rows < 512 && cholqr_ylds(rows, n) <= CHOLQR_YLDS;
+}
 
 // Column-norm / normalise job (also the Frobenius-norm job).
 struct ColDesc {
@@ -252,11 +264,12 @@ size_t jacobi_lds_bytes(int n);
 void launch_precond(hipStream_t st, const JacobiDesc* d_descs, int nd, int nmin, int nmax);
 // pivoted Cholesky QR of Gram matrices (JacobiDesc: G in, W = P R^{-1} out,
 // lam = R_jj); columns below null_rel2 * max diag are dropped, or with span
-// (null_rel2 0) unresolved columns kept as they are.  With d_conv
+// (null_rel2 0) unresolved columns kept as they are.  ylds: the
+// largest cholqr_ylds of the jobs that bring Y.  With d_conv
 // the stopping rule follows, on each problem's R_jj.
 void launch_cholqr(hipStream_t st, const JacobiDesc* d_descs, int nd, int nmin, int nmax,
                    double null_rel2, bool span = false, const ConvDesc* d_conv = nullptr,
-                   const ConvRule& rule = ConvRule());
+                   const ConvRule& rule = ConvRule(), int64_t ylds = 0);
 void launch_jacobi(hipStream_t st, const JacobiDesc* d_descs, int nd, int nmax, double tol,
                    int max_sweeps);
 void launch_colnorm(hipStream_t st, const ColDesc* d_descs, int nd, int ncol_max, double rtol);

@@ -1991,7 +1991,6 @@ __device__ __forceinline__ void conv_step(const ConvDesc& D, const double* sv, c
 // wave (n <= 64) or four: 39.6 -> 11.6 us at n = 32, 77 -> 22 at 64, 154 -> 46
 // at 96.  A pivot step takes 0.23 us (0.38 with the control flow in vector
 // registers and keys converted to single precision).
-constexpr int CQ64 = 64;   // Gram matrices up to this size take the 64-row kernel
 
 template <int N>
 struct CholLds {
@@ -2021,6 +2020,13 @@ __device__ __forceinline__ int wave_max_i32(int x) {
 }
 
 //
+// A small Y (cholqr_fused: its copy fits the LDS beside A and X) comes with the
+// job: G = Y^T Y and U = Y W are formed here, without their two launches (5 us
+// each and the gaps between).  The one workgroup takes 5 us longer at 128 x 32, 8
+// at 256 x 32; larger Y are the GEMM's, which has the whole chip.  Measured: ATRG
+// Z2 chi 16 (128 x 32) 23.5 -> 21.0 ms, BTRG Z2 chi 16 11.7 -> 10.9, HOTRG chi 16
+// (256 x 32) 12.4 -> 12.0.
+//
 // SPAN: the basis must keep all n directions.  G resolves a column down to
 // 1e-7 of its own norm; what it has left below that (d <= SPAN_FLOOR G_pp) is
 // noise, and dropping or eliminating with such a column would lose its direction
@@ -2041,6 +2047,84 @@ __device__ __forceinline__ void chol_load(const JacobiDesc& D, double* A, int n,
         const int c = e / N, r = e - c * N;
         const double v = D.G[min(r, n - 1) + (int64_t)min(c, n - 1) * D.ldg];
         A[r + c * LD] = r < n && c < n ? v : 0.0;
+    }
+}
+
+// A = Y^T Y (zero beyond n) by way of a copy of Y in LDS, summed over the rows
+// in the order of the GEMM kernels (rows < 512: one K chunk).
+template <int N>
+__device__ __forceinline__ void chol_gram(const JacobiDesc& D, double* A, double* Yl, int n) {
+    constexpr int LD = CholLds<N>::LD, NT = 64 * CholLds<N>::WAVES;
+    const int t = threadIdx.x, lane = t & 63, l0 = lane & 15, l1 = lane >> 4;
+    const int w = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int T = (n + 15) / 16, m = 16 * T, ld = cholqr_ldy(D.rows), rows16 = ld - 2;
+    gconst_double* Y = as_global(D.Y);
+    // 64 rows of a column a wave and load, eight loads in flight (p / rc by a
+    // 16-bit reciprocal, exact below 65536 / rc)
+    const int rc = (rows16 + 63) / 64, inv = 65536 / rc + 1;
+    for (int p0 = w; p0 < m * rc; p0 += 8 * CholLds<N>::WAVES) {
+        double v[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const int p = min(p0 + i * CholLds<N>::WAVES, m * rc - 1), c = (p * inv) >> 16;
+            const int r = 64 * (p - c * rc) + lane;
+            v[i] = Y[min(r, D.rows - 1) + (int64_t)min(c, n - 1) * D.ldy];
+            if (r >= D.rows || c >= n) v[i] = 0.0;
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const int p = p0 + i * CholLds<N>::WAVES, c = (p * inv) >> 16, r = 64 * (p - c * rc) + lane;
+            if (p < m * rc && r < rows16) Yl[r + c * ld] = v[i];
+        }
+    }
+    for (int e = t; e < m * N; e += NT)
+        if (e % N >= m) A[e % N + (e / N) * LD] = 0.0;
+    __syncthreads();
+    for (int u = w; u < T * (T + 1) / 2; u += CholLds<N>::WAVES) {
+        int J = 0;
+        while ((J + 1) * (J + 2) / 2 <= u) ++J;
+        const int I = u - J * (J + 1) / 2;
+        dbl4 c = dbl4{0, 0, 0, 0};
+        const double *a = Yl + l1 + (16 * I + l0) * ld, *b = Yl + l1 + (16 * J + l0) * ld;
+        for (int k = 0; k < rows16; k += 16) {
+            double x[4], y[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) x[q] = a[k + 4 * q], y[q] = b[k + 4 * q];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) c = __builtin_amdgcn_mfma_f64_16x16x4f64(x[q], y[q], c, 0, 0, 0);
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int r = 16 * I + l1 + 4 * q, s = 16 * J + l0;
+            A[r + s * LD] = c[q];
+            if (I != J) A[s + r * LD] = c[q];
+        }
+    }
+}
+
+// U = Y W = Y P X from the copy of Y.
+template <int N>
+__device__ __forceinline__ void chol_rotate(const JacobiDesc& D, const double* X, const double* Yl, const int* perm,
+                                            int rank, int n) {
+    constexpr int LD = CholLds<N>::LD;
+    const int lane = threadIdx.x & 63, l0 = lane & 15, l1 = lane >> 4;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int T = (n + 15) / 16, ld = cholqr_ldy(D.rows), RT = (D.rows + 15) / 16;
+    for (int u = w; u < RT * T; u += CholLds<N>::WAVES) {
+        const int I = u % RT, J = u / RT, row = 16 * I + l0;
+        dbl4 c = dbl4{0, 0, 0, 0};
+        for (int K = 0; K <= J; ++K)
+#pragma unroll
+            for (int kk = 0; kk < 4; ++kk) {
+                const int k = 16 * K + 4 * kk + l1;
+                const double a = k < rank ? Yl[row + perm[min(k, rank - 1)] * ld] : 0.0;
+                c = __builtin_amdgcn_mfma_f64_16x16x4f64(a, X[k + (16 * J + l0) * LD], c, 0, 0, 0);
+            }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int r = 16 * I + l1 + 4 * q, j = 16 * J + l0;
+            if (r < D.rows && j < n) as_global(D.U)[r + (int64_t)j * D.ldu] = c[q];
+        }
     }
 }
 
@@ -2263,7 +2347,9 @@ __global__ __launch_bounds__(64 * CholLds<N>::WAVES) void k_cholqr(const JacobiD
     int* perm = (int*)(rinv + N);
     int* iperm = perm + N;
     int* rank_ = iperm + N;
-    chol_load<N>(D, A, n, m);
+    double* Yl = lds + CholLds<N>::BYTES / sizeof(double);
+    if (D.Y) chol_gram<N>(D, A, Yl, n);
+    else chol_load<N>(D, A, n, m);
     const bool noisy = chol_panels<N, SPAN>(A, X, piv, perm, iperm, rank_, n, null_rel2);
     const int rank = *rank_;
     chol_invert<N>(A, X, piv, rinv, perm, iperm, rank, n);
@@ -2275,6 +2361,7 @@ __global__ __launch_bounds__(64 * CholLds<N>::WAVES) void k_cholqr(const JacobiD
         if (r < n)
             D.W[r + (int64_t)c * D.ldw] = ip >= 0 && ip <= c && c < rank ? X[ip + c * LD] : 0.0;
     }
+    if (D.Y) chol_rotate<N>(D, X, Yl, perm, rank, n);
     if (t < n) D.lam[t] = piv[t];
     if (t == 0 && D.sweeps) *D.sweeps = 0;
     // (a problem that is done needs no product with W any more)
@@ -3408,23 +3495,24 @@ void launch_jacobi(hipStream_t st, const JacobiDesc* d_descs, int nd, int nmax, 
 // depends on its own size only, never on the rest of its launch group.
 template <int N, bool SPAN>
 static void launch_cholqr_n(hipStream_t st, const JacobiDesc* d_descs, int nd, double null_rel2,
-                            const ConvDesc* d_conv, const ConvRule& rule) {
+                            const ConvDesc* d_conv, const ConvRule& rule, int64_t ylds) {
     static const hipError_t attr = hipFuncSetAttribute(
-        (const void*)k_cholqr<N, SPAN>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)CholLds<N>::BYTES);
+        (const void*)k_cholqr<N, SPAN>, hipFuncAttributeMaxDynamicSharedMemorySize,
+        (int)(CholLds<N>::BYTES + (N == CQ64 ? CHOLQR_YLDS * sizeof(double) : 0)));
     TNR_HIP(attr);
     ProfScope ps(st, PK_JACOBI, 0.0, 0.0);
-    TNR_LAUNCH(ps, (k_cholqr<N, SPAN>), dim3(nd), dim3(64 * CholLds<N>::WAVES), CholLds<N>::BYTES, st, d_descs,
-               nd, null_rel2, d_conv, rule);
+    TNR_LAUNCH(ps, (k_cholqr<N, SPAN>), dim3(nd), dim3(64 * CholLds<N>::WAVES),
+               CholLds<N>::BYTES + (N == CQ64 ? ylds * sizeof(double) : 0), st, d_descs, nd, null_rel2, d_conv, rule);
     TNR_HIP(hipGetLastError());
 }
 
 void launch_cholqr(hipStream_t st, const JacobiDesc* d_descs, int nd, int nmin, int nmax,
-                   double null_rel2, bool span, const ConvDesc* d_conv, const ConvRule& rule) {
+                   double null_rel2, bool span, const ConvDesc* d_conv, const ConvRule& rule, int64_t ylds) {
     if (nd <= 0) return;
     if (nmin <= CQ64) (span ? launch_cholqr_n<CQ64, true> : launch_cholqr_n<CQ64, false>)(
-        st, d_descs, nd, null_rel2, d_conv, rule);
+        st, d_descs, nd, null_rel2, d_conv, rule, ylds);
     if (nmax > CQ64) (span ? launch_cholqr_n<LMAX, true> : launch_cholqr_n<LMAX, false>)(
-        st, d_descs, nd, null_rel2, d_conv, rule);
+        st, d_descs, nd, null_rel2, d_conv, rule, 0);
 }
 
 template <int N>

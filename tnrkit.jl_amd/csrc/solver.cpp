@@ -116,6 +116,7 @@ struct RRPlan {
     bool chol = false;          // one pass, pivoted Cholesky QR instead of Jacobi
     bool span = false;          // Cholesky QR that keeps every direction (null_rel2 = 0)
     bool tight = false;
+    int64_t ylds = 0;           // LDS for the jobs whose Cholesky QR is one launch
     GemmPlan gram[3], rot[3];
     std::vector<JacobiDesc> jac[3];
     std::vector<ColDesc> col;
@@ -148,14 +149,16 @@ RRPlan rr_plan(Ctx& ctx, const std::vector<RR>& jobs, int passes, bool chol = fa
             double* W1 = passes == 1 && j.Wtot ? j.Wtot : j.W;
             GemmJob g{Y, Y, j.G, j.l, j.l, j.rows, ld, ld, j.l, 1, 0};   // G = Y^T Y
             g.skip = j.skip;
-            gj.push_back(g);
+            // a small Y is read once: k_cholqr does the products, too
+            const bool fused = chol && cholqr_fused(j.rows, j.l);
+            if (!fused) gj.push_back(g);
             // Cholesky QR: the rotated columns are the orthonormal basis itself
             GemmJob r = chol ? GemmJob{j.Y, W1, j.U, j.rows, j.l, j.l, j.ldy, j.l, j.ldu, 0, 0}
                         : pass != 1
                             ? GemmJob{j.Y, W1, j.Y2, j.rows, j.l, j.l, j.ldy, j.l, j.rows, 0, 0}
                             : GemmJob{j.Y2, j.W2, j.Y, j.rows, j.l, j.l, j.rows, j.l, j.ldy, 0, 0};
             r.skip = j.skip;
-            rj.push_back(r);
+            if (!fused) rj.push_back(r);
             if (pass >= 1 && j.Wtot) {
                 GemmJob w = pass == 1 ? GemmJob{j.W, j.W2, j.Wtot, j.l, j.l, j.l, j.l, j.l, j.l, 0, 0}
                                       : GemmJob{j.Wtot, j.W, j.W2, j.l, j.l, j.l, j.l, j.l, j.l, 0, 0};
@@ -164,6 +167,15 @@ RRPlan rr_plan(Ctx& ctx, const std::vector<RR>& jobs, int passes, bool chol = fa
             }
             P.jac[pass].push_back(JacobiDesc{j.G, pass != 1 ? W1 : j.W2, j.lam, j.sweeps, j.l, j.l,
                                              j.l, j.skip, j.fail});
+            if (fused) {
+                JacobiDesc& d = P.jac[pass].back();
+                d.Y = j.Y;
+                d.U = j.U;
+                d.rows = j.rows;
+                d.ldy = j.ldy;
+                d.ldu = j.ldu;
+                P.ylds = std::max(P.ylds, cholqr_ylds(j.rows, j.l));
+            }
         }
         P.gram[pass] = gemm_plan(ctx, gj);
         P.rot[pass] = gemm_plan(ctx, rj);
@@ -210,7 +222,8 @@ void rr_issue(Ctx& ctx, RRPlan& P, bool first = false, const ConvDesc* conv = nu
         const bool in_loop = P.passes == 1 && !P.tight;
         if (P.chol)
             launch_cholqr(ctx.stream, P.d_jac[pass], (int)P.jac[pass].size(), P.lmin, P.lmax,
-                          P.span ? 0.0 : cfg.null_rtol * cfg.null_rtol, P.span, conv, conv_rule(cfg));
+                          P.span ? 0.0 : cfg.null_rtol * cfg.null_rtol, P.span, conv, conv_rule(cfg),
+                          P.ylds);
         else if (P.passes == 3 && pass < 2)
             launch_precond(ctx.stream, P.d_jac[pass], (int)P.jac[pass].size(), P.lmin, P.lmax);
         else
