@@ -119,7 +119,7 @@ int tnr_autotune_enable(int on);
  * conv_target (1e-14), block_mult (2), block_extra (2),
  * cholqr_y (1), cholqr_z (1), cholqr_eigh (1) (block iteration steps by
  * pivoted Cholesky QR instead of Rayleigh-Ritz), rv_passes (2), rf_passes (1)
- * (Jacobi passes of the final extraction).  A solve of a larger matrix that
+ * (Cholesky QR and Jacobi passes of the final extraction).  A solve of a larger matrix that
  * reaches max_iters, or one that reaches a sweep cap, unconverged fails its
  * step with TNR_ERR_NOCONV.  Not thread-safe: call it
  * while no other entry point runs. */

@@ -889,7 +889,7 @@ void svd_grouped(Ctx& ctx, const std::vector<SvdIn>& in, std::vector<SvdOut>& ou
         ConvState cs(ctx, P);
         std::vector<FillDesc> fills;
         std::vector<RR> rY, rZ, rV, rF;
-        std::vector<GemmJob> jMV, jMtU, jF, jV;
+        std::vector<GemmJob> jMV, jMtU, jQ, jF, jV;
         std::vector<ConvDesc> conv;
         for (int i = 0; i < P; ++i) {
             const SvdIn& s = in[iter[i]];
@@ -926,12 +926,13 @@ void svd_grouped(Ctx& ctx, const std::vector<SvdIn>& in, std::vector<SvdOut>& ou
             conv.push_back(ConvDesc{cfg.cholqr_z ? x.lam.d() : sv, l, s.kmax, 1, cs.it(i),
                                     cs.prod(i), cs.done(i), std::min(s.m, s.n) <= kWholeMax});
             // the loop's last Rayleigh-Ritz step left Z W in Y2; one pass at the
-            // final threshold (into Z, free until V Wtot) rebuilds V.  With
-            // Cholesky QR on the Z side Y2 is not a Ritz basis: two passes on Z.
+            // final threshold (into Z, free until V Wtot) rebuilds V.  A Cholesky
+            // QR step that ends the loop leaves out its rotation: Z W first, then
+            // a second step on these columns.
             if (cfg.cholqr_z)
-                rV.push_back(RR{x.Z.d(), s.n, l, s.n, x.Y2.d(), x.G.d(), x.W.d(), x.W2.d(),
-                                x.lam.d(), x.sw.as<int>(), nullptr, x.V.d(), s.n, sv, nullptr, fl});
-            else
+                jQ.push_back(GemmJob{x.Z.d(), x.W.d(), cfg.rv_passes > 1 ? x.Y2.d() : x.V.d(), s.n, l, l,
+                                     s.n, l, s.n, 0, 0});
+            if (!cfg.cholqr_z || cfg.rv_passes > 1)
                 rV.push_back(RR{x.Y2.d(), s.n, l, s.n, x.Z.d(), x.G.d(), x.W.d(), x.W2.d(),
                                 x.lam.d(), x.sw.as<int>(), nullptr, x.V.d(), s.n, sv, nullptr, fl});
             // Ritz extraction from Y = M V over the whole basis (the top
@@ -954,19 +955,19 @@ void svd_grouped(Ctx& ctx, const std::vector<SvdIn>& in, std::vector<SvdOut>& ou
         // rebuilt at full accuracy before the final extraction relies on
         // V^T V = I.  Its last rotated Z has columns orthogonal to that
         // threshold, so one pass at the final threshold does what the second
-        // pass of a two-pass step does.
-        const int vpass = cfg.cholqr_z ? cfg.rv_passes : 1;
-        RRPlan pV = rr_plan(ctx, rV, vpass, false, vpass == 1);
+        // pass of a two-pass step does.  After Cholesky QR steps a second one on
+        // the same columns does.
+        RRPlan pV = rr_plan(ctx, rV, 1, cfg.cholqr_z, !cfg.cholqr_z);
         RRPlan pF = rr_plan(ctx, rF, cfg.rf_passes, false, cfg.rf_passes == 1);
-        GemmPlan pjF = gemm_plan(ctx, jF), pjV = gemm_plan(ctx, jV);
+        GemmPlan pQ = gemm_plan(ctx, jQ), pjF = gemm_plan(ctx, jF), pjV = gemm_plan(ctx, jV);
         // all of the solve's descriptors in one upload
         const int64_t nfill = fill_starts(fills);
         DescArena a;
-        for (GemmPlan* g : {&pMV, &pMtU, &pjF, &pjV}) gemm_stage(*g, a);
+        for (GemmPlan* g : {&pMV, &pMtU, &pQ, &pjF, &pjV}) gemm_stage(*g, a);
         for (RRPlan* r : {&pY, &pZ, &pV, &pF}) rr_stage(*r, a);
         const size_t o_conv = a.add(conv), o_fill = a.add(fills);
         a.commit(ctx);
-        for (GemmPlan* g : {&pMV, &pMtU, &pjF, &pjV}) gemm_bind(*g, a);
+        for (GemmPlan* g : {&pMV, &pMtU, &pQ, &pjF, &pjV}) gemm_bind(*g, a);
         for (RRPlan* r : {&pY, &pZ, &pV, &pF}) rr_bind(*r, a);
         const ConvDesc* d_conv = a.at<ConvDesc>(o_conv);
         launch_randfill(ctx.stream, a.at<FillDesc>(o_fill), (int)fills.size(), nfill);
@@ -977,7 +978,8 @@ void svd_grouped(Ctx& ctx, const std::vector<SvdIn>& in, std::vector<SvdOut>& ou
             rr_issue(ctx, pZ, it == 0, cfg.cholqr_z ? d_conv : nullptr);
             if (!cfg.cholqr_z) launch_conv(ctx.stream, d_conv, P, conv_rule(cfg));
         });
-        rr_issue(ctx, pV);
+        gemm_issue(ctx, pQ);
+        if (!rV.empty()) rr_issue(ctx, pV);
         gemm_issue(ctx, pjF);
         rr_issue(ctx, pF);
         gemm_issue(ctx, pjV);
