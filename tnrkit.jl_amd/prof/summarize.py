@@ -19,8 +19,9 @@ import json
 import re
 
 COPY_KIB = 256 * 1024
-# the FP64 GEMM launches: LDS-DMA tiles and the 32-deep register-staged tile
-FP64_GEMM = ("k_gemm_dl", "k_gemm_f64")
+# the FP64 GEMM launches: LDS-DMA tiles, the small launches and the 32-deep
+# register-staged tile
+FP64_GEMM = ("k_gemm_dl", "k_gemm_kw", "k_gemm_f64")
 
 
 def short(name):
