@@ -1361,7 +1361,9 @@ __device__ __forceinline__ void jacobi_rounds(const JacPlaces<M, NS>& P, double*
     load();
     for (int r = 0; r < R; ++r) {
         // the diagonal's arrival means that every LDS access issued before
-        // it is done, the last round's rotations among them
+        // it is done, the last round's rotations among them (a wave's
+        // accesses complete in order); what may be in flight are the reads of
+        // b, entries of S that no other wave touches during the rounds
         asm volatile("s_barrier" ::"v"(d[0]), "v"(d[1]), "v"(d[2]) : "memory");
         // once a round is run, pairs a hundred times below the threshold are
         // rotated too: it costs nothing, and close eigenvalues' vectors feel
@@ -1425,10 +1427,12 @@ struct JacRows {
     template <bool CROSS>
     __device__ __forceinline__ void rounds(const double2* cs, int lane, int R) {
         const bool hi = lane >= 32;
+        // (nothing in flight: a __syncthreads came since this wave's last access)
         asm volatile("s_barrier" ::: "memory");
         for (int r = 0; r < R; ++r) {
-            // (the rotations of the round before have been read)
-            asm volatile("s_barrier" ::: "memory");
+            // The rotations' wave writes round r's buffer again (round r + 2)
+            // behind the next barrier: the reads below are complete by then.
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
             const double2* rot = cs + (r & 1) * H + HP * (lane >> 5);
             double2 k[HP];
 #pragma unroll
@@ -1700,6 +1704,7 @@ __device__ void jacobi_body(const JacobiDesc& D, double* lds, double tol, int ma
             for (int b = 0; b < NB; ++b) ids[b] = nid[b];
         }
     };
+    // (a __syncthreads came since this wave's last LDS access)
     auto idle = [](int R) {
         for (int r = 0; r <= R; ++r) asm volatile("s_barrier" ::: "memory");
     };
@@ -1720,6 +1725,8 @@ __device__ void jacobi_body(const JacobiDesc& D, double* lds, double tol, int ma
             // W^T <- Q^T W^T with the last rotated block round's Q, a few MFMAs
             // per barrier of this one's rounds.  A result is laid out as the
             // next product's B operand, so the strips never leave the registers.
+            // (Reads of Qs may be in flight at these barriers: that buffer is
+            // written next by apply, behind its __syncthreads.)
             const int R = rounds_of(cross);
             int done = 0;
 #pragma unroll
