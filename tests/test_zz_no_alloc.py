@@ -84,6 +84,13 @@ def test_noalloc_jacobi_equals_the_allocating_entry_point(tk):
         assert np.allclose(G[i] @ Wt, Wt * L1[i], atol=1e-11 * np.abs(L1[i]).max())
 
 
+def test_noalloc_jacobi_takes_its_documented_capacity(tk):
+    G = _symmetric(np.random.default_rng(12), 13797, 2)
+    W0, L0, S0 = _host(tk, G)
+    W1, L1, S1 = _noalloc(tk, G)
+    assert np.array_equal(L0, L1) and np.array_equal(W0, W1) and np.array_equal(S0, S1)
+
+
 def test_noalloc_jacobi_refuses_counts_beyond_its_scratch(tk):
     st = tk.lib().tnr_kernel_jacobi_noalloc(13798, 2, 1, 1, 1, None, None)
     assert st == -1 and "scratch" in tk.lib().tnr_last_error().decode()

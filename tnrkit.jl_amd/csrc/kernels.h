@@ -112,7 +112,12 @@ struct JacobiDesc {
                                   // accumulated rotation, close to the
                                   // identity for a nearly diagonal G) instead
                                   // of ordering by |lambda| descending
-    // Cholesky QR of a small Y (cholqr_fused): G is Y^T Y and U = Y W follows
+};
+
+// Pivoted Cholesky QR job: of a Gram matrix (G in, W = P R^{-1} out, lam =
+// R_jj), or of a small Y itself (cholqr_fused), whose G = Y^T Y is formed in
+// LDS and for which U = Y W follows.
+struct CholDesc : JacobiDesc {
     const double* Y = nullptr;
     double* U = nullptr;
     int32_t rows = 0, ldy = 0, ldu = 0;
@@ -262,12 +267,11 @@ void launch_trace_normalize(hipStream_t st, const TraceDesc* d_descs, const Trac
 size_t jacobi_lds_bytes(int n);
 // orthogonal W = Q with (Y Q)^T (Y Q) closer to diagonal than G = Y^T Y
 void launch_precond(hipStream_t st, const JacobiDesc* d_descs, int nd, int nmin, int nmax);
-// pivoted Cholesky QR of Gram matrices (JacobiDesc: G in, W = P R^{-1} out,
-// lam = R_jj); columns below null_rel2 * max diag are dropped, or with span
+// pivoted Cholesky QR; columns below null_rel2 * max diag are dropped, or with span
 // (null_rel2 0) unresolved columns kept as they are.  ylds: the
 // largest cholqr_ylds of the jobs that bring Y.  With d_conv
 // the stopping rule follows, on each problem's R_jj.
-void launch_cholqr(hipStream_t st, const JacobiDesc* d_descs, int nd, int nmin, int nmax,
+void launch_cholqr(hipStream_t st, const CholDesc* d_descs, int nd, int nmin, int nmax,
                    double null_rel2, bool span = false, const ConvDesc* d_conv = nullptr,
                    const ConvRule& rule = ConvRule(), int64_t ylds = 0);
 void launch_jacobi(hipStream_t st, const JacobiDesc* d_descs, int nd, int nmax, double tol,

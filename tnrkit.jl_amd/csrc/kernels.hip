@@ -2060,7 +2060,7 @@ __device__ __forceinline__ void chol_load(const JacobiDesc& D, double* A, int n,
 // A = Y^T Y (zero beyond n) by way of a copy of Y in LDS, summed over the rows
 // in the order of the GEMM kernels (rows < 512: one K chunk).
 template <int N>
-__device__ __forceinline__ void chol_gram(const JacobiDesc& D, double* A, double* Yl, int n) {
+__device__ __forceinline__ void chol_gram(const CholDesc& D, double* A, double* Yl, int n) {
     constexpr int LD = CholLds<N>::LD, NT = 64 * CholLds<N>::WAVES;
     const int t = threadIdx.x, lane = t & 63, l0 = lane & 15, l1 = lane >> 4;
     const int w = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -2111,7 +2111,7 @@ __device__ __forceinline__ void chol_gram(const JacobiDesc& D, double* A, double
 
 // U = Y W = Y P X from the copy of Y.
 template <int N>
-__device__ __forceinline__ void chol_rotate(const JacobiDesc& D, const double* X, const double* Yl, const int* perm,
+__device__ __forceinline__ void chol_rotate(const CholDesc& D, const double* X, const double* Yl, const int* perm,
                                             int rank, int n) {
     constexpr int LD = CholLds<N>::LD;
     const int lane = threadIdx.x & 63, l0 = lane & 15, l1 = lane >> 4;
@@ -2336,14 +2336,14 @@ __device__ __forceinline__ void chol_invert(double* A, double* X, double* piv, d
 }
 
 template <int N, bool SPAN>
-__global__ __launch_bounds__(64 * CholLds<N>::WAVES) void k_cholqr(const JacobiDesc* __restrict__ descs,
+__global__ __launch_bounds__(64 * CholLds<N>::WAVES) void k_cholqr(const CholDesc* __restrict__ descs,
                                                                   int nd, double null_rel2,
                                                                   const ConvDesc* __restrict__ conv,
                                                                   ConvRule rule) {
     using L = CholLds<N>;
     constexpr int LD = L::LD, NT = 64 * L::WAVES;
     extern __shared__ double lds[];
-    const JacobiDesc D = descs[blockIdx.x];
+    const CholDesc D = descs[blockIdx.x];
     // (the other sizes of the group are the other kernel's)
     if (D.n > N || (N > CQ64 && D.n <= CQ64) || (D.skip && *D.skip)) return;
     const int n = D.n, t = threadIdx.x, m = 16 * ((n + 15) / 16);
@@ -3501,7 +3501,7 @@ void launch_jacobi(hipStream_t st, const JacobiDesc* d_descs, int nd, int nmax, 
 // k_cholqr<LMAX> (each kernel skips the other's), so the kernel a problem gets
 // depends on its own size only, never on the rest of its launch group.
 template <int N, bool SPAN>
-static void launch_cholqr_n(hipStream_t st, const JacobiDesc* d_descs, int nd, double null_rel2,
+static void launch_cholqr_n(hipStream_t st, const CholDesc* d_descs, int nd, double null_rel2,
                             const ConvDesc* d_conv, const ConvRule& rule, int64_t ylds) {
     static const hipError_t attr = hipFuncSetAttribute(
         (const void*)k_cholqr<N, SPAN>, hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -3513,7 +3513,7 @@ static void launch_cholqr_n(hipStream_t st, const JacobiDesc* d_descs, int nd, d
     TNR_HIP(hipGetLastError());
 }
 
-void launch_cholqr(hipStream_t st, const JacobiDesc* d_descs, int nd, int nmin, int nmax,
+void launch_cholqr(hipStream_t st, const CholDesc* d_descs, int nd, int nmin, int nmax,
                    double null_rel2, bool span, const ConvDesc* d_conv, const ConvRule& rule, int64_t ylds) {
     if (nd <= 0) return;
     if (nmin <= CQ64) (span ? launch_cholqr_n<CQ64, true> : launch_cholqr_n<CQ64, false>)(

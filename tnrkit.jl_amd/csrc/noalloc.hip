@@ -24,6 +24,8 @@ static __device__ __align__(256) unsigned char scratch[NOALLOC_SCRATCH];
 // descriptor + sweep count of each problem
 constexpr size_t kPerProblem = sizeof(JacobiDesc) + sizeof(int);
 constexpr int kMaxProblems = (int)(NOALLOC_SCRATCH / kPerProblem);
+// the documented capacity (include/tnr_kernels.h): JacobiDesc must not grow
+static_assert(kMaxProblems == 13797, "tnr_kernel_jacobi_noalloc promises 13797 problems");
 
 // The device address of `scratch` on each GPU (the array's name is a host
 // stand-in, not a device address); looked up once per device, with that

@@ -119,9 +119,11 @@ struct RRPlan {
     int64_t ylds = 0;           // LDS for the jobs whose Cholesky QR is one launch
     GemmPlan gram[3], rot[3];
     std::vector<JacobiDesc> jac[3];
+    std::vector<CholDesc> cho;  // (chol: in jac's place)
     std::vector<ColDesc> col;
-    size_t o_jac[3] = {0, 0, 0}, o_col = 0;
+    size_t o_jac[3] = {0, 0, 0}, o_cho = 0, o_col = 0;
     const JacobiDesc* d_jac[3] = {nullptr, nullptr, nullptr};
+    const CholDesc* d_cho = nullptr;
     const ColDesc* d_col = nullptr;
 };
 
@@ -165,15 +167,12 @@ RRPlan rr_plan(Ctx& ctx, const std::vector<RR>& jobs, int passes, bool chol = fa
                 w.skip = j.skip;
                 rj.push_back(w);
             }
-            P.jac[pass].push_back(JacobiDesc{j.G, pass != 1 ? W1 : j.W2, j.lam, j.sweeps, j.l, j.l,
-                                             j.l, j.skip, j.fail});
-            if (fused) {
-                JacobiDesc& d = P.jac[pass].back();
-                d.Y = j.Y;
-                d.U = j.U;
-                d.rows = j.rows;
-                d.ldy = j.ldy;
-                d.ldu = j.ldu;
+            const JacobiDesc d{j.G, pass != 1 ? W1 : j.W2, j.lam, j.sweeps, j.l, j.l,
+                               j.l, j.skip, j.fail};
+            if (!chol) P.jac[pass].push_back(d);
+            else if (!fused) P.cho.push_back(CholDesc{d});
+            else {
+                P.cho.push_back(CholDesc{d, j.Y, j.U, j.rows, j.ldy, j.ldu});
                 P.ylds = std::max(P.ylds, cholqr_ylds(j.rows, j.l));
             }
         }
@@ -200,6 +199,7 @@ void rr_stage(RRPlan& P, DescArena& a) {
         gemm_stage(P.rot[pass], a);
         P.o_jac[pass] = a.add(P.jac[pass]);
     }
+    P.o_cho = a.add(P.cho);
     P.o_col = a.add(P.col);
 }
 
@@ -209,6 +209,7 @@ void rr_bind(RRPlan& P, const DescArena& a) {
         gemm_bind(P.rot[pass], a);
         P.d_jac[pass] = a.at<JacobiDesc>(P.o_jac[pass]);
     }
+    P.d_cho = a.at<CholDesc>(P.o_cho);
     P.d_col = a.at<ColDesc>(P.o_col);
 }
 
@@ -221,7 +222,7 @@ void rr_issue(Ctx& ctx, RRPlan& P, bool first = false, const ConvDesc* conv = nu
         gemm_issue(ctx, P.gram[pass]);
         const bool in_loop = P.passes == 1 && !P.tight;
         if (P.chol)
-            launch_cholqr(ctx.stream, P.d_jac[pass], (int)P.jac[pass].size(), P.lmin, P.lmax,
+            launch_cholqr(ctx.stream, P.d_cho, (int)P.cho.size(), P.lmin, P.lmax,
                           P.span ? 0.0 : cfg.null_rtol * cfg.null_rtol, P.span, conv, conv_rule(cfg),
                           P.ylds);
         else if (P.passes == 3 && pass < 2)
