@@ -174,6 +174,47 @@ def test_failed_run_in_a_batch_leaves_the_others_untouched(tk, solver_caps):
     assert e.value.status == -5 and "run 1" in str(e.value)
 
 
+_SVD_UNDER_ENV = """
+import ctypes as C, sys
+import numpy as np
+sys.path.insert(0, {root!r})
+import __graft_entry__
+lib = __graft_entry__.package().lib()
+m, k = 200, 8                          # block iteration on a 16-wide block
+rng = np.random.default_rng(3)
+A = np.linalg.qr(rng.standard_normal((m, m)))[0] * 0.8 ** np.arange(m) @ rng.standard_normal((m, m))
+M, U, s, V = np.asfortranarray(A), np.zeros((m, k), order="F"), np.zeros(k), np.zeros((m, k), order="F")
+P = C.POINTER(C.c_double)
+st = lib.tnr_kernel_svd(m, m, M.ctypes.data_as(P), k, U.ctypes.data_as(P), s.ctypes.data_as(P),
+                        V.ctypes.data_as(P), None)
+print("status", st, "residual", float(np.abs(A @ V - U * s).max() / s[0]))
+"""
+
+
+@pytest.mark.parametrize("spec,ok", [("rf_passes=2", True), ("rv_passes=1,rf_passes=2", True),
+                                     ("rf_passes=3", False), ("rf_passes=0", False),
+                                     ("rv_passes=3", False), ("rv_passes=0", False),
+                                     ("rv_passes=3,cholqr_z=0", True)])
+def test_pass_counts_from_the_environment(spec, ok):
+    """TNR_SOLVER_CFG is read once a process and not range-checked when it is
+    read: a solve that a pass count in it does not fit is refused, never
+    answered with factors of different passes.  (rv_passes belongs to Cholesky
+    QR on the Z side.)  rv_passes=1 leaves V orthonormal to the Gram matrix's
+    resolution, ~1e-8 of the first value."""
+    import os
+    import subprocess
+    import sys
+    from conftest import ROOT
+    out = subprocess.run([sys.executable, "-c", _SVD_UNDER_ENV.format(root=ROOT)], capture_output=True, text=True,
+                         env=dict(os.environ, TNR_SOLVER_CFG=spec), timeout=60)
+    assert out.returncode == 0, out.stderr
+    _, st, _, res = out.stdout.split()
+    if ok:
+        assert int(st) == 0 and float(res) < (1e-7 if "rv_passes=1" in spec else 1e-12), out.stdout
+    else:
+        assert int(st) != 0, out.stdout
+
+
 def test_nonfinite_tensors_are_refused(tk):
     """NaN / Inf entries: tnr_create and tnr_server_submit return
     TNR_ERR_NONFINITE; a server keeps serving its other requests."""

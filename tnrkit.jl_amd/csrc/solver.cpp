@@ -107,12 +107,13 @@ struct RR {
 
 // `passes` = 1 inside the block iteration (the next iteration corrects
 // what one pass leaves), 2 for the final Ritz extraction and direct solves of
-// the smallest matrices, 3 for the other direct ones: two k_precond passes
-// and one Jacobi pass on what they leave, total rotation in W2, columns in Y2;
-// `tight` = one pass at the final threshold, for columns that are already
+// the smallest matrices; `precond` (the other direct ones) = two k_precond
+// passes and one Jacobi pass on what they leave, total rotation in W2, columns
+// in Y2; `tight` = one pass at the final threshold, for columns that are already
 // orthogonal to the loop's threshold (the second pass of a two-pass step).
 struct RRPlan {
     int passes = 1, lmax = 0, lmin = 0;
+    bool precond = false;       // three passes, the first two by k_precond
     bool chol = false;          // one pass, pivoted Cholesky QR instead of Jacobi
     bool span = false;          // Cholesky QR that keeps every direction (null_rel2 = 0)
     bool tight = false;
@@ -127,13 +128,18 @@ struct RRPlan {
     const ColDesc* d_col = nullptr;
 };
 
-RRPlan rr_plan(Ctx& ctx, const std::vector<RR>& jobs, int passes, bool chol = false,
-               bool tight = false) {
-    TNR_REQUIRE(passes >= 1 && passes <= 3, TNR_ERR_INTERNAL, "one to three passes");
-    TNR_REQUIRE(!chol || passes == 1, TNR_ERR_INTERNAL, "Cholesky QR is a one-pass step");
-    TNR_REQUIRE(!tight || (passes == 1 && !chol), TNR_ERR_INTERNAL, "tight is a one-pass Jacobi step");
+RRPlan rr_plan(Ctx& ctx, const std::vector<RR>& jobs, int jacobi_passes, bool chol = false,
+               bool tight = false, bool precond = false) {
+    // (a pass count out of the environment may be any number)
+    TNR_REQUIRE(jacobi_passes == 1 || jacobi_passes == 2, TNR_ERR_INTERNAL, "one or two passes");
+    TNR_REQUIRE(!chol || jacobi_passes == 1, TNR_ERR_INTERNAL, "Cholesky QR is a one-pass step");
+    TNR_REQUIRE(!tight || (jacobi_passes == 1 && !chol), TNR_ERR_INTERNAL, "tight is a one-pass Jacobi step");
+    TNR_REQUIRE(!precond || (jacobi_passes == 1 && !chol && !tight), TNR_ERR_INTERNAL,
+                "one Jacobi pass follows k_precond");
+    const int passes = precond ? 3 : jacobi_passes;
     RRPlan P;
     P.passes = passes;
+    P.precond = precond;
     P.chol = chol;
     P.tight = tight;
     P.lmin = jobs.empty() ? 0 : jobs[0].l;
@@ -225,7 +231,7 @@ void rr_issue(Ctx& ctx, RRPlan& P, bool first = false, const ConvDesc* conv = nu
             launch_cholqr(ctx.stream, P.d_cho, (int)P.cho.size(), P.lmin, P.lmax,
                           P.span ? 0.0 : cfg.null_rtol * cfg.null_rtol, P.span, conv, conv_rule(cfg),
                           P.ylds);
-        else if (P.passes == 3 && pass < 2)
+        else if (P.precond && pass < 2)
             launch_precond(ctx.stream, P.d_jac[pass], (int)P.jac[pass].size(), P.lmin, P.lmax);
         else
             launch_jacobi(ctx.stream, P.d_jac[pass], (int)P.jac[pass].size(), P.lmax,
@@ -854,7 +860,7 @@ void svd_grouped(Ctx& ctx, const std::vector<SvdIn>& in, std::vector<SvdOut>& ou
         }
         DescArena a;
         const GatherPlan pg = gather_plan(gd, a);
-        RRPlan p2 = rr_plan(ctx, rr, 2), p3 = rr_plan(ctx, rp, 3);
+        RRPlan p2 = rr_plan(ctx, rr, 2), p3 = rr_plan(ctx, rp, 1, false, false, true);
         rr_stage(p2, a);
         rr_stage(p3, a);
         a.commit(ctx);
@@ -958,6 +964,8 @@ void svd_grouped(Ctx& ctx, const std::vector<SvdIn>& in, std::vector<SvdOut>& ou
         // threshold, so one pass at the final threshold does what the second
         // pass of a two-pass step does.  After Cholesky QR steps a second one on
         // the same columns does.
+        TNR_REQUIRE(!cfg.cholqr_z || cfg.rv_passes == 1 || cfg.rv_passes == 2, TNR_ERR_INTERNAL,
+                    "one or two passes");
         RRPlan pV = rr_plan(ctx, rV, 1, cfg.cholqr_z, !cfg.cholqr_z);
         RRPlan pF = rr_plan(ctx, rF, cfg.rf_passes, false, cfg.rf_passes == 1);
         GemmPlan pQ = gemm_plan(ctx, jQ), pjF = gemm_plan(ctx, jF), pjV = gemm_plan(ctx, jV);
