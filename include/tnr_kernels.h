@@ -18,13 +18,15 @@ extern "C" {
 #endif
 
 /* C = alpha op(A) op(B) + beta C, column-major FP64.  mode & 7: 0 = FP64
- * MFMA with the tile shape the engine would choose, 1 = FP32-MFMA hi/lo
+ * MFMA with the kernel and tile shape the engine would choose (small
+ * products: 16x16 or 32x32 tiles whose K chunks one workgroup's waves share,
+ * through LDS-DMA; only the engine's own choice takes these), 1 = FP32-MFMA hi/lo
  * split kernel, 2 / 3 / 4 / 5 = FP64 MFMA with 64x64 / 128x64 / 128x128 /
  * 64x64 (32-deep k-tiles) tiles;
  * mode | 8 never splits K over workgroups, mode | 16 always does (for K of
  * two or more 256-deep chunks); the default decides by launch size;
  * mode | 32 loads the 16-deep tiles through registers instead of LDS-DMA
- * (the same bits).
+ * (the same bits) and keeps small products on such tiles.
  * repeat >= 1 launches the product that many times on device-resident
  * copies; *ms_out (optional) receives the device time of the last launch
  * from HIP events. */

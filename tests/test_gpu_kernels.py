@@ -123,6 +123,29 @@ def test_gemm_lds_dma_matches_register_loads_bitwise(tk, M, N, K, ta, tb, pad):
             assert np.max(np.abs(dma - ref)) <= 1e-14 * (np.sqrt(K) + 1) * 8
 
 
+@pytest.mark.parametrize("M,N,K", [(64, 64, 1024), (300, 64, 600), (512, 96, 1024)])
+def test_register_loads_of_a_small_product(tk, M, N, K):
+    """mode | 32 keeps a product with the engine's own tile shape off LDS-DMA,
+    and so off the small launches' kernels, which add the K chunks themselves:
+    the register-staged tiles split K over workgroups here, with a launch of
+    their own (profile class 2) for the chunk sums.  The bits agree."""
+    rng = np.random.default_rng(M + N + K)
+    A, B, Cm = rng.standard_normal((M, K)), rng.standard_normal((K, N)), rng.standard_normal((M, N))
+    outs, reduces = [], []
+    for mode in (0, 32):
+        assert tk.lib().tnr_profile_enable(1) == 0
+        try:
+            outs.append(gemm(tk, A, B, Cm, 0, 0, 1.1, 0.3, split=mode))
+            n = C.c_int64()
+            args = [C.byref(C.c_double()) for _ in range(5)]
+            assert tk.lib().tnr_profile_read(2, C.byref(n), *args) == 0
+            reduces.append(n.value)
+        finally:
+            tk.lib().tnr_profile_enable(0)
+    assert reduces == [0, 1]
+    assert np.array_equal(*outs)
+
+
 # sizes on both sides of the small launches' rule: 16 x 16 tiles on one wave
 # (one K chunk), 16 x 16 and 32 x 32 tiles with the K chunks over four waves
 # (fewer, as many and more chunks than waves), and the first sizes past them

@@ -593,16 +593,17 @@ static bool gemm_dma_enabled() {
 }
 
 GemmPlan gemm_plan(Ctx& ctx, const std::vector<GemmJob>& jobs, bool split32, int force_shape,
-                   int force_split) {
+                   int force_split, bool allow_dma) {
     GemmPlan P;
     P.split32 = split32;
+    P.dma = allow_dma;
     bool dma_ok = gemm_dma_enabled();
     for (const GemmJob& j : jobs)
         if (j.M > 0 && j.N > 0) dma_ok = dma_ok && gemm_dma_ok(j.ta, j.lda, j.tb, j.ldb);
     if (force_shape >= 0 && !split32) P.shape = force_shape;
     else if (split32) P.shape = GEMM_64x64;
     else {
-        const int small = dma_ok && force_split < 0 ? pick_small(jobs) : -1;
+        const int small = dma_ok && allow_dma && force_split < 0 ? pick_small(jobs) : -1;
         P.shape = small >= 0 ? small
                              : tuned_shape(ctx, jobs, pick_shape(jobs, false), dma_ok, &P.tune_key, &P.trial);
     }
@@ -683,8 +684,7 @@ void gemm_issue(Ctx& ctx, GemmPlan& p) {
 
 void gemm_grouped(Ctx& ctx, const std::vector<GemmJob>& jobs, bool split32, int force_shape,
                   int force_split, bool allow_dma) {
-    GemmPlan p = gemm_plan(ctx, jobs, split32, force_shape, force_split);
-    p.dma = p.dma && allow_dma;
+    GemmPlan p = gemm_plan(ctx, jobs, split32, force_shape, force_split, allow_dma);
     if (p.descs.empty()) return;
     DescArena arena;
     gemm_stage(p, arena);

@@ -146,7 +146,8 @@ struct GemmJob {
     double alpha = 1.0, beta = 0.0;
     const int* skip = nullptr;       // device flag: problem finished
 };
-// allow_dma = false keeps the 16-deep tile shapes on register-staged loads
+// allow_dma = false keeps the 16-deep tile shapes on register-staged loads and
+// takes no kernel that has LDS-DMA loads only (the small launches')
 void gemm_grouped(Ctx& ctx, const std::vector<GemmJob>& jobs, bool split32 = false,
                   int force_shape = -1, int force_split = -1, bool allow_dma = true);
 
@@ -198,7 +199,7 @@ struct GemmPlan {
 // force_shape >= 0 fixes the FP64 tile shape (GemmShape) instead of choosing
 // it; force_split 0 / 1 turns splitting K over workgroups off / on instead
 GemmPlan gemm_plan(Ctx& ctx, const std::vector<GemmJob>& jobs, bool split32 = false,
-                   int force_shape = -1, int force_split = -1);
+                   int force_shape = -1, int force_split = -1, bool allow_dma = true);
 void gemm_stage(GemmPlan& p, DescArena& arena);          // before arena.commit
 void gemm_bind(GemmPlan& p, const DescArena& arena);     // after arena.commit
 void gemm_issue(Ctx& ctx, GemmPlan& p);

@@ -3403,6 +3403,7 @@ void launch_transpose(hipStream_t st, const TransDesc* d_descs, int nd, int64_t 
 void launch_gemm(hipStream_t st, const GemmDesc* d_descs, int nd, int64_t tiles, bool split32,
                  double flops, int shape, bool dma) {
     if (tiles <= 0 || nd <= 0) return;
+    TNR_REQUIRE(split32 || dma || !gemm_shape_kw(shape), TNR_ERR_INTERNAL, "small tiles load through LDS-DMA");
     ProfScope ps(st, split32 ? PK_GEMM_SPLIT32 : PK_GEMM_F64, flops, 0.0);
     unsigned long long* fc = ps.active ? prof_flop_counter(split32) : nullptr;
     if (split32)
