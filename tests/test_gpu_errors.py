@@ -215,6 +215,31 @@ def test_pass_counts_from_the_environment(spec, ok):
         assert int(st) != 0, out.stdout
 
 
+@pytest.mark.parametrize("m,n,k", [(17, 17, 4), (40, 64, 8), (96, 80, 8), (96, 96, 96),   # direct
+                                   (120, 300, 12), (300, 200, 24), (400, 400, 40)])
+def test_nonfinite_matrices_leave_the_next_solve_right(tk, m, n, k):
+    """NaNs of either sign in two columns, or entries whose squares overflow
+    (tensors with such entries are refused before they get here; values may
+    still overflow on the way): every kernel path stays inside its buffers
+    whatever the order its NaNs compare in, and ends."""
+    rng = np.random.default_rng(m + n)
+    A = rng.standard_normal((m, n)) * 0.9 ** np.arange(n)   # (a flat spectrum may reach max_iters)
+
+    def svd(M):
+        M, U, s, V = np.asfortranarray(M), np.zeros((m, k), order="F"), np.zeros(k), np.zeros((n, k), order="F")
+        st = tk.lib().tnr_kernel_svd(m, n, _ptr(M, DP), k, _ptr(U, DP), _ptr(s, DP), _ptr(V, DP), None)
+        return st, s
+
+    bad = A.copy()
+    for first, second in ((1.0, 1.0), (-1.0, -1.0), (1.0, -1.0), (-1.0, 1.0)):
+        bad[m // 2, n - 1] = np.copysign(np.nan, first)
+        bad[m // 3, n // 2] = np.copysign(np.nan, second)
+        assert svd(bad)[0] in (0, -4, -5)
+    assert svd(1e200 * A)[0] in (0, -4, -5)
+    st, s = svd(A)
+    assert st == 0 and np.abs(s / np.linalg.svd(A, compute_uv=False)[:k] - 1).max() < 1e-11
+
+
 def test_nonfinite_tensors_are_refused(tk):
     """NaN / Inf entries: tnr_create and tnr_server_submit return
     TNR_ERR_NONFINITE; a server keeps serving its other requests."""

@@ -2180,7 +2180,9 @@ __device__ __forceinline__ bool chol_panels(double* A, double* X, double* piv, i
 #pragma unroll
                 for (int q = 0; q < ROWS; ++q)
                     key = max(key, (__double2hiint(d[q]) & ~LOW) | (LOW - (lane + 64 * q)));
-                const int p = LOW - (wave_max_i32(key) & LOW);
+                // (NaNs spread to the spare lanes' d, and their signs order them
+                // at will: a row of the matrix all the same)
+                const int p = min(LOW - (wave_max_i32(key) & LOW), n - 1);
                 int hi, lo;
                 if (ROWS > 1 && p >= 64) {
                     hi = __builtin_amdgcn_readlane(__double2hiint(d[ROWS - 1]), p - 64);
@@ -2457,8 +2459,8 @@ __global__ __launch_bounds__(64 * CholLds<N>::WAVES) void k_precond(const Jacobi
     __syncthreads();
     chol_panels<N, true>(B, A, piv, perm, iperm, rank_, n, 0.0);
     chol_invert<N>(B, A, piv, rinv, perm, iperm, *rank_, n);
-    // the rows of R in H's pivot order (the bounds hold for a NaN, whose pivots
-    // are arbitrary, too)
+    // the rows of R in H's pivot order (clamped: perm is not written past a rank
+    // below n)
 #pragma unroll 4
     for (int e = t; e < m * N; e += NT) {
         const int c = e / N, k = e - c * N;
