@@ -221,6 +221,15 @@ def test_jacobi_layout_edges(tk, n):
         assert np.max(np.abs(w.T @ w - np.eye(n))) < 1e-13 * n
 
 
+@pytest.mark.parametrize("n", [7, 16, 24, 32, 64, 96])
+def test_jacobi_without_a_rotation(tk, n):
+    """A diagonal matrix: W is exactly the permutation that orders it."""
+    d = np.random.default_rng(n).standard_normal(n)
+    lam, W, sw = jacobi(tk, np.diag(d)[None])
+    order = np.argsort(-np.abs(d), kind="stable")
+    assert sw == 0 and np.array_equal(lam[0], d[order]) and np.array_equal(W[0], np.eye(n)[:, order])
+
+
 def test_jacobi_graded_gram_relative_accuracy(tk):
     rng = np.random.default_rng(9)
     A = rng.standard_normal((200, 64)) * np.logspace(0, -12, 64)

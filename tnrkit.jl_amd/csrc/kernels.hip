@@ -1827,7 +1827,7 @@ __device__ void jacobi_body(const JacobiDesc& D, double* lds, double tol, int ma
         D.lam[k] = li;
     }
     __syncthreads();
-    if (polish) {
+    if (polish && sweeps > 0) {   // (W = 1 without a rotation)
         // One Newton step towards the nearest orthogonal matrix,
         // X <- (3/2 - X X^T / 2) X for X = W^T: a few hundred rotations leave
         // W^T W off by ~1e-14, which singular vectors of close values feel as
