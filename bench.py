@@ -112,7 +112,7 @@ def roofline_from(prof, precision, traffic, steps=1):
              "peak": PEAK["fp64_mfma"] / 1e12, "unit": "TFLOP/s", "frac": ach / PEAK["fp64_mfma"],
              "launches": d["launches"], "avg_launch_ms": d["ms"] / n,
              "busy_ms_per_step": d["busy_ms"] / steps,
-             "note": "FP64 VALU rotations (no MFMA); MI355X FP64 vector and matrix peaks are "
+             "note": "FP64 VALU rotations, block updates on MFMA; MI355X FP64 vector and matrix peaks are "
                      "both 78.6 TF/s; work = 18n flops per rotation, sweeps read back"}
     else:
         ach = d["bytes"] / (d["busy_ms"] * 1e-3) if d["busy_ms"] else 0.0

@@ -222,7 +222,7 @@ struct GatherDesc {
     int64_t start;
 };
 
-// start = prefix of 4096-element chunks; every job holds < 2^31 elements
+// start = prefix of COPY_CHUNK-element chunks; every job holds < 2^31 elements
 void launch_copy(hipStream_t st, const CopyDesc* d_descs, int nd, int64_t chunks, int64_t elems);
 void launch_transpose(hipStream_t st, const TransDesc* d_descs, int nd, int64_t tiles,
                       int64_t elems);

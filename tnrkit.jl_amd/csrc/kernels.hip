@@ -1366,8 +1366,14 @@ __device__ __forceinline__ void jacobi_rounds(const JacPlaces<M, NS>& P, double*
         // b, entries of S that no other wave touches during the rounds
         asm volatile("s_barrier" ::"v"(d[0]), "v"(d[1]), "v"(d[2]) : "memory");
         // once a round is run, pairs a hundred times below the threshold are
-        // rotated too: it costs nothing, and close eigenvalues' vectors feel
-        // what is left over their gap
+        // rotated too: close eigenvalues' vectors feel what is left over their
+        // gap.  Random and graded spectra take as many sweeps as without the
+        // factor; large clusters take more, as the rotations of (nearly) equal
+        // diagonals keep stirring up roundoff: with half of the eigenvalues
+        // equal, n = 32 / 64 / 96, 11 / 18 / 20 sweeps instead of 8 / 13 / 14
+        // (64 problems 153 / 627 / 1568 us instead of 115 / 450 / 1129; the
+        // kernel before the block Jacobi 313 / 938 / 2440), with pairs of equal
+        // ones 8.8 / 9.9 / 10.5 instead of 7.7 / 8.8 / 9.4.
         const bool on = jacobi_violates(d[0], d[1], d[2], 1e-4 * tol2);
         double c, s, t;
         jacobi_rotation(d[0], d[1], d[2], t, c, s);
@@ -1933,7 +1939,7 @@ __global__ __launch_bounds__(JAC_TMAX) void k_jacobi(const JacobiDesc* __restric
 
 // ------------------------------------------------ stopping rule
 // Stopping rule of the block iteration by one wave, after an iteration whose
-// l values (largest first) are in sv: the contraction of the top-k subspace,
+// l values (largest first, pivots up to k_cholqr's tolerance) are in sv: the contraction of the top-k subspace,
 // (sv_l / sv_k)^2 (or ^1), is accumulated from iteration min_iters on, and the
 // problem is done below the target or at max_iters; one that will be
 // factorised whole anyway stops once even twice its current rate could not
@@ -1990,8 +1996,9 @@ __device__ __forceinline__ void conv_step(const ConvDesc& D, const double* sv, c
 // column) and, by distance from the diagonal, X_IJ = -X_II sum_K R_IK X_KJ on
 // MFMA, the sum's result layout being the next product's operand layout.
 // The pivot search compares the leading 14 (n <= 64) or 13 bits of d's mantissa
-// and settles ties by the lowest index: a pivot within 1e-4 of the largest
-// serves as well, and the result is a function of G.  G is taken as the
+// and settles ties by the lowest index: a pivot within 2^-14 (2^-13 = 1.2e-4) of
+// the largest serves as well, and the result is a function of G.  So the pivots,
+// and lam, descend up to that tolerance only.  G is taken as the
 // product of one GEMM, whose two triangles agree bit for bit.
 // Measured (average launch in whole runs) against the former kernels, which
 // updated all of A and solved for X column by column after every pivot, in one
@@ -3046,8 +3053,8 @@ __global__ __launch_bounds__(EIGT) void k_eig_hqr_g(const EigDesc* __restrict__ 
     eig_hqr_body(D, D.work);
 }
 
-// conv_step for values that another kernel wrote (the eigensolver's Ritz
-// values), one wave per problem.
+// conv_step for values that another kernel wrote (Ritz values, where an
+// option puts Rayleigh-Ritz steps into the loop), one wave per problem.
 __global__ __launch_bounds__(64) void k_conv(const ConvDesc* __restrict__ descs, int nd, ConvRule rule) {
     const ConvDesc D = descs[blockIdx.x];
     if (*D.done) return;

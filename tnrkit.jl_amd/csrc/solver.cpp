@@ -219,8 +219,9 @@ void rr_bind(RRPlan& P, const DescArena& a) {
     P.d_col = a.at<ColDesc>(P.o_col);
 }
 
-// `first`: the block iteration's first step, whose Rayleigh-Ritz step only
-// has to align a random basis roughly (jacobi_tol_first)
+// `first`: the block iteration's first step; a Rayleigh-Ritz step there
+// (cholqr_y, cholqr_z or cholqr_eigh off) only has to align a random basis
+// roughly (jacobi_tol_first)
 // `conv` (Cholesky QR only): the stopping rule, one descriptor per job
 void rr_issue(Ctx& ctx, RRPlan& P, bool first = false, const ConvDesc* conv = nullptr) {
     const SolverCfg& cfg = solver_cfg();
@@ -829,7 +830,8 @@ void svd_grouped(Ctx& ctx, const std::vector<SvdIn>& in, std::vector<SvdOut>& ou
         else wide.push_back((int)p);
     }
     if (!wide.empty()) svd_wide(ctx, in, wide, out);
-    // ---------------- direct problems: Gram/Jacobi twice on the smaller side
+    // ---------------- direct problems, on the smaller side: k_precond twice and
+    // Gram/Jacobi once, or (below kPrecondFrom) Gram/Jacobi twice
     if (!direct.empty()) {
         struct DW { Buf Y, Y2, G, W, W2, Wt, lam, sig, sw; };
         std::vector<DW> w(direct.size());
@@ -932,8 +934,8 @@ void svd_grouped(Ctx& ctx, const std::vector<SvdIn>& in, std::vector<SvdOut>& ou
             // Ritz values of the Z side, or with Cholesky QR the pivots R_jj
             conv.push_back(ConvDesc{cfg.cholqr_z ? x.lam.d() : sv, l, s.kmax, 1, cs.it(i),
                                     cs.prod(i), cs.done(i), std::min(s.m, s.n) <= kWholeMax});
-            // the loop's last Rayleigh-Ritz step left Z W in Y2; one pass at the
-            // final threshold (into Z, free until V Wtot) rebuilds V.  A Cholesky
+            // A last Rayleigh-Ritz step (cholqr_z=0) left Z W in Y2; one pass at
+            // the final threshold (into Z, free until V Wtot) rebuilds V.  A Cholesky
             // QR step that ends the loop leaves out its rotation: Z W first, then
             // a second step on these columns.
             if (cfg.cholqr_z)
@@ -951,19 +953,20 @@ void svd_grouped(Ctx& ctx, const std::vector<SvdIn>& in, std::vector<SvdOut>& ou
                             x.sw.as<int>(), x.Wt.d(), x.U.d(), s.m, x.sigU.d(), nullptr, fl});
             jV.push_back(GemmJob{x.V.d(), x.Wt.d(), x.Z.d(), s.n, l, l, s.n, l, s.n, 0, 0});
         }
-        // the random start block is not orthonormalised: the first
-        // Rayleigh-Ritz step on Y = M V builds an orthonormal basis of its span
+        // the random start block is not orthonormalised: the first step on
+        // Y = M V builds an orthonormal basis of its span
         GemmPlan pMV = gemm_plan(ctx, jMV), pMtU = gemm_plan(ctx, jMtU);
-        // Y side: an orthonormal basis of span(M V) is all the next product
-        // needs (pivoted Cholesky QR); Z side: Rayleigh-Ritz, whose values
-        // drive the stopping rule
+        // Both sides: an orthonormal basis of the product's span is all the next
+        // product needs (pivoted Cholesky QR); the Z side's pivots drive the
+        // stopping rule.  cholqr_y=0, cholqr_z=0: a Rayleigh-Ritz step there
+        // (the Z side's Ritz values then drive it, through k_conv).
         RRPlan pY = rr_plan(ctx, rY, 1, cfg.cholqr_y), pZ = rr_plan(ctx, rZ, 1, cfg.cholqr_z);
-        // the loop orthonormalises only to its looser Jacobi threshold: V is
-        // rebuilt at full accuracy before the final extraction relies on
-        // V^T V = I.  Its last rotated Z has columns orthogonal to that
-        // threshold, so one pass at the final threshold does what the second
-        // pass of a two-pass step does.  After Cholesky QR steps a second one on
-        // the same columns does.
+        // V is rebuilt at full accuracy before the final extraction relies on
+        // V^T V = I: one Cholesky QR step leaves it orthonormal to the Gram
+        // matrix's resolution, a second one on the same columns to roundoff.
+        // After Rayleigh-Ritz steps, whose last rotated Z has columns orthogonal
+        // to the loop's Jacobi threshold, one pass at the final threshold does
+        // what the second pass of a two-pass step does.
         TNR_REQUIRE(!cfg.cholqr_z || cfg.rv_passes == 1 || cfg.rv_passes == 2, TNR_ERR_INTERNAL,
                     "one or two passes");
         RRPlan pV = rr_plan(ctx, rV, 1, cfg.cholqr_z, !cfg.cholqr_z);

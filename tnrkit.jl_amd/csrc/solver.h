@@ -67,8 +67,10 @@ void eigh_grouped(Ctx& ctx, const std::vector<EighIn>& in, std::vector<EighOut>&
 struct SolverCfg {
     double jacobi_tol = 1e-15;   // relative off-diagonal threshold (final Ritz extraction, direct)
     int jacobi_sweeps = 40;
-    // Rayleigh-Ritz inside the block iteration.  Measured on BTRG chi = 32
-    // beta scans: looser thresholds or sweep caps here make the iteration
+    // Rayleigh-Ritz inside the block iteration: the loop takes such steps, with
+    // these thresholds and k_conv, only where cholqr_y, cholqr_z or cholqr_eigh
+    // is 0.  Measured with them on BTRG chi = 32 beta
+    // scans: looser thresholds or sweep caps here make the iteration
     // and the final extraction take longer than they save, so the loop
     // keeps a tight threshold; V is still rebuilt at full accuracy (1e-15)
     // once the loop ends.
